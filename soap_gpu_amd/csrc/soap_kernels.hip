@@ -2615,7 +2615,11 @@ hipError_t launch_mask_wsum(int n_lines, int n_v, int64_t n_t, const int32_t *m_
 // spec_norm and the CCF of the unnormalised spectra in one launch: the blocks come
 // in groups of one CCF block followed by `ratio` norm blocks (ratio = n_norm /
 // n_ccf), the remaining norm blocks after the groups, so that every CU holds both
-// kinds and the norm's streaming runs beside the CCF's gathers.  blockDim.x is the
+// kinds and the norm's streaming runs beside the CCF's gathers.  Block b runs on XCD
+// b % 8: where the group length shares a factor with 8, a CCF block at a fixed place
+// in its group would meet only some of the XCDs (one of them at a length of 32, as
+// 3,800 lines of a 100-phase series give: 7.9 ms per launch against 0.90 ms), so the
+// place moves with the group and eight CCF blocks in a row meet all eight.  blockDim.x is the
 // CCF's thread count (velocities rounded up to a wave); a norm block covers
 // kNormPer * blockDim.x pixels of one spectrum.
 __device__ __forceinline__ void norm_ccf_body(const NormCcfArgs &a, long b, double *ccf_lds) {
@@ -2624,10 +2628,12 @@ __device__ __forceinline__ void norm_ccf_body(const NormCcfArgs &a, long b, doub
   long ci = -1, ni;
   if (b < mixed) {
     long g = b / grp, r = b - g * grp;
-    if (r == 0)
+    const long rot = min(grp & -grp, 8L);  // gcd(grp, 8)
+    const long slot = (g / (8 / rot)) % rot;
+    if (r == slot)
       ci = g;
     else
-      ni = g * a.ratio + r - 1;
+      ni = g * a.ratio + r - (r > slot);
   } else {
     ni = (long)a.n_ccf * a.ratio + (b - mixed);
   }
