@@ -2477,7 +2477,7 @@ int batch_build(soap_batch *b) {
   std::vector<FitJob> ft(ni);
   std::vector<int64_t> w[BS_COUNT];
   for (auto &v : w) v.assign(ni, 0);
-  size_t lds_taps = 0, lds_fir = 0, lds_conv = 0, lds_ccf = 0;
+  size_t lds_taps = 0, lds_fir = 0, lds_conv = 0, lds_ccf = 0, lds_fit = 0;
   int ccf_threads = 64, red_threads = 64;
   for (size_t i = 0; i < ni; i++) {
     soap_ctx *c = b->inst[i];
@@ -2583,6 +2583,7 @@ int batch_build(soap_batch *b) {
                    (const int32_t *)c->m_start.p, (const uint32_t *)c->m_alive.p, (const double2 *)c->m_val.p,
                    c->d_w_sorted, (const int2 *)c->fp.p, c->ccf_cap, (double *)c->ccf_part.p};
     lds_ccf = std::max(lds_ccf, ccf_lds_bytes(c->ccf_cap));
+    lds_fit = std::max(lds_fit, fit_lds_bytes(c->n_v));
     w[BS_CCF][i] = (int64_t)nc * ((n_spec + ccf_spec_chunk() - 1) / ccf_spec_chunk());
     ccf_threads = std::max(ccf_threads, (c->n_v + 63) / 64 * 64);
     int rt = 64;
@@ -2615,7 +2616,7 @@ int batch_build(soap_batch *b) {
       (rc = batch_upload(b, BS_NORM, nm, w[BS_NORM], 256, 0)) ||
       (rc = batch_upload(b, BS_CCF, cc, w[BS_CCF], ccf_threads, lds_ccf)) ||
       (rc = batch_upload(b, BS_CCF_REDUCE, cr, w[BS_CCF_REDUCE], red_threads, 0)) ||
-      (rc = batch_upload(b, BS_FIT, ft, w[BS_FIT], 64, 0)))
+      (rc = batch_upload(b, BS_FIT, ft, w[BS_FIT], 64, lds_fit)))
     return rc;
   b->sig.resize(ni);
   for (size_t i = 0; i < ni; i++) b->sig[i] = batch_signature(b->inst[i]);

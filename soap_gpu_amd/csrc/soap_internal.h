@@ -142,6 +142,84 @@ __device__ __forceinline__ double fx_value(unsigned long long hi, unsigned long 
 // contributions of magnitude <= w_max; the hi word's total stays below 2^62.
 inline bool fx_capacity_ok(double n_contrib, double w_max) { return n_contrib * w_max < 1073741824.0; }
 
+// Sums over a 64-lane wave of 16 values per lane, each total in every lane.  Four DPP
+// exchanges within the rows of 16 lanes halve the values a lane holds while they double
+// the lanes summed (8 + 4 + 2 + 1 adds), so lane r of a row ends with value r of its
+// row; two swaps across the rows finish it and the totals are read from lanes 0..15.
+// 17 adds against 96 shuffles and adds of 16 butterflies; the order is fixed.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x) {
+  const long long v = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double lane_f64(double x, int lane) {
+  const long long v = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)v, lane), hi = __builtin_amdgcn_readlane((int)(v >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int N, int CTRL>
+__device__ __forceinline__ void wave_fold(double (&v)[16], bool up) {
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    const double send = up ? v[q] : v[q + N], keep = up ? v[q + N] : v[q];
+    v[q] = keep + dpp_f64<CTRL>(send);
+  }
+}
+__device__ __forceinline__ void wave_sums16(double (&v)[16]) {
+  const int lane = threadIdx.x & 63;
+  wave_fold<8, 0x140>(v, lane & 8);  // row mirror: lane i <-> 15 - i
+  wave_fold<4, 0x141>(v, lane & 4);  // half-row mirror: i <-> 7 - i
+  wave_fold<2, 0x4e>(v, lane & 2);   // quad permutation 2 3 0 1
+  wave_fold<1, 0xb1>(v, lane & 1);   // quad permutation 1 0 3 2
+  double x = v[0];
+  x += __shfl_xor(x, 16);
+  x += __shfl_xor(x, 32);
+#pragma unroll
+  for (int q = 0; q < 16; q++) v[q] = lane_f64(x, q);
+}
+
+// First index of the largest value over a wave: better(a, b) of the serial scan
+// "if (a > best)" in index order, so ties keep the smaller index and NaNs never win.
+__device__ __forceinline__ void wave_argmax(double &best, int &at) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const double b = __shfl_xor(best, off);
+    const int i = __shfl_xor(at, off);
+    if (b > best || (b == best && i < at)) {
+      best = b;
+      at = i;
+    }
+  }
+}
+
+// The bisector's walk of BIS_FIT2.cpp:244-250 from index im of a normalised CCF nc[n] in
+// LDS: b steps down while nc[b] > dep (not below 1), r up while nc[r + 1] > dep (not
+// above n - 2).  Eight values are read ahead of their tests on each side, so a step does
+// not wait for an LDS read of its own.
+__device__ __forceinline__ void bisector_walk(const double *nc, int n, int im, double dep, int &b, int &r) {
+  constexpr int kAhead = 8;
+  b = im;
+  r = im;
+  bool gb = true, gr = true;
+  while (gb || gr) {
+    double xb[kAhead], xr[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) {
+      xb[u] = nc[max(b - u, 0)];
+      xr[u] = nc[min(r + 1 + u, n - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) {
+      gb = gb && xb[u] > dep && b > 1;
+      gr = gr && xr[u] > dep && r < n - 2;
+      b -= gb;
+      r += gr;
+    }
+  }
+}
+
 // Cell classification of one phase: loop over the phase's visible regions in
 // order, later ones overwriting earlier ones (SOAP_integration.cu:724-785,
 // spot_scan :346-387).  Returns -1 (quiet), 0 (spot) or 1 (facula).
@@ -390,6 +468,7 @@ hipError_t launch_ccf_reduce(const double *part, int nc, int n_spec, int n_v, co
                              const double *wsum, double *ccf, hipStream_t s);
 // err: per-point errors [n_ccf][n_v] or NULL (unit errors); status (optional): per
 // CCF 0 (converged), 27 (no progress), 11 (iteration limit)
+size_t fit_lds_bytes(int n_v);
 hipError_t launch_fit(const double *v, int n_v, const double *y, const double *err, int n_ccf, double *par,
                       double *model, double *depth, double *bis, int32_t *iters, hipStream_t s,
                       int32_t *status = nullptr);

@@ -2698,61 +2698,50 @@ hipError_t launch_ccf_sum(const double *part, int nc, int n_spec, int n_v, doubl
 // ------------------------------------------------------------------ a9: fit
 constexpr int kMaxV = 1024;
 
-__device__ __forceinline__ double wave_sum(double x) {
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-  return x;
-}
-
 struct GaussEval {
   double sum_f2;
   double A[10];  // upper triangle of J^T J: 00 01 02 03 11 12 13 22 23 33
   double g[4];
-  double colsq[4];
 };
 
-// gauss_f / gauss_df of BIS_FIT2.cpp:31-81, lane-strided over points: residual
-// (fit - y) / err and Jacobian rows divided by err (BIS_FIT2.cpp:49,74-77); err
-// NULL = unit errors (the driver's CCF_error.txt of ones, run_all_SOAP.py:317).
-// with_jac = false evaluates only sum f^2.
-__device__ void gauss_eval(const double *px, const double *y, const double *err, int n, const double *x,
-                           bool with_jac, GaussEval &r) {
-  double c = x[0], k = x[1], x0 = x[2], fwhm = x[3];
-  double sigma = fwhm / 2 / sqrt(2 * log(2.0));
-  double f2 = 0, A[10] = {0}, g[4] = {0};
-  for (int i = threadIdx.x; i < n; i += 64) {
-    double e = exp(-(px[i] - x0) * (px[i] - x0) / 2 / sigma / sigma);
-    double fi = err ? ((c + k * e) - y[i]) / err[i] : (c + k * e) - y[i];
-    f2 += fi * fi;
-    if (with_jac) {
-      double J[4];
-      if (err) {
-        double ei = err[i];
-        J[0] = 1 / ei;
-        J[1] = e / ei;
-        J[2] = k / ei * e * (px[i] - x0) / sigma / sigma;
-        J[3] = k / ei * e * (px[i] - x0) * (px[i] - x0) / sigma / sigma / sigma / 2 / sqrt(2 * log(2.0));
-      } else {
-        J[0] = 1.0;
-        J[1] = e;
-        J[2] = k * e * (px[i] - x0) / sigma / sigma;
-        J[3] = k * e * (px[i] - x0) * (px[i] - x0) / sigma / sigma / sigma / 2 / sqrt(2 * log(2.0));
-      }
+// gauss_f / gauss_df of BIS_FIT2.cpp:31-81 at x = (c, k, x0, fwhm), lane-strided over
+// points: residual (fit - y) / err and Jacobian rows divided by err (BIS_FIT2.cpp:49,74-77);
+// rerr = 1 / err, NULL = unit errors (the driver's CCF_error.txt of ones,
+// run_all_SOAP.py:317).  Three points of a lane are in flight together (their exp chains
+// overlap); points past n add zeros.
+__device__ __forceinline__ void gauss_eval(const double *px, const double *y, const double *rerr, int n,
+                                           const double (&x)[4], GaussEval &r) {
+  const double c = x[0], k = x[1], x0 = x[2], fwhm = x[3];
+  const double inv_s = 2 * sqrt(2 * log(2.0)) / fwhm, inv_s2 = inv_s * inv_s;
+  const double j2 = k * inv_s2, j3 = j2 / fwhm;  // 1 / (2 sqrt(2 ln 2) sigma^3) = 1 / (sigma^2 fwhm)
+  double v[16];
+#pragma unroll
+  for (int q = 0; q < 16; q++) v[q] = 0.0;
+  for (int i0 = threadIdx.x; i0 - (int)threadIdx.x < n; i0 += 192) {
+#pragma unroll
+    for (int u = 0; u < 3; u++) {
+      const int i = min(i0 + 64 * u, n - 1);
+      const bool in = i0 + 64 * u < n;
+      const double d = px[i] - x0, ex = exp(-0.5 * inv_s2 * d * d);
+      const double e = in ? ex : 0.0, w = rerr ? rerr[i] : 1.0;
+      const double f = in ? ((c + k * e) - y[i]) * w : 0.0;
+      const double J[4] = {in ? w : 0.0, e * w, j2 * e * d * w, j3 * e * d * d * w};
       int q = 0;
-      for (int a = 0; a < 4; a++) {
-        g[a] += J[a] * fi;
-        for (int b = a; b < 4; b++) A[q++] += J[a] * J[b];
-      }
+#pragma unroll
+      for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int b = a; b < 4; b++, q++) v[q] = fma(J[a], J[b], v[q]);
+#pragma unroll
+      for (int a = 0; a < 4; a++) v[10 + a] = fma(J[a], f, v[10 + a]);
+      v[14] = fma(f, f, v[14]);
     }
   }
-  r.sum_f2 = wave_sum(f2);
-  if (with_jac) {
-    for (int q = 0; q < 10; q++) r.A[q] = wave_sum(A[q]);
-    for (int a = 0; a < 4; a++) r.g[a] = wave_sum(g[a]);
-    r.colsq[0] = r.A[0];
-    r.colsq[1] = r.A[4];
-    r.colsq[2] = r.A[7];
-    r.colsq[3] = r.A[9];
-  }
+  wave_sums16(v);
+#pragma unroll
+  for (int q = 0; q < 10; q++) r.A[q] = v[q];
+#pragma unroll
+  for (int a = 0; a < 4; a++) r.g[a] = v[10 + a];
+  r.sum_f2 = v[14];
 }
 
 __device__ __forceinline__ double symA(const double *A, int a, int b) {
@@ -2765,30 +2754,38 @@ __device__ __forceinline__ double symA(const double *A, int a, int b) {
   return A[idx[a][b]];
 }
 
-__device__ int solve4(const double *A, const double *D, double mu, const double *g, double *dx) {
-  double L[4][4] = {{0}};
+// (A + mu diag(D2)) dx = -g by Cholesky; returns 0 on success
+__device__ __forceinline__ int solve4(const double *A, const double *D2, double mu, const double *g, double *dx) {
+  double L[4][4], inv[4];
+#pragma unroll
   for (int i = 0; i < 4; i++) {
+#pragma unroll
     for (int j = 0; j <= i; j++) {
-      double s = symA(A, i, j) + (i == j ? mu * D[i] * D[i] : 0.0);
+      double s = symA(A, i, j) + (i == j ? mu * D2[i] : 0.0);
+#pragma unroll
       for (int k = 0; k < j; k++) s -= L[i][k] * L[j][k];
       if (i == j) {
         if (!(s > 0)) return -1;
-        L[i][i] = sqrt(s);
+        inv[i] = 1.0 / sqrt(s);
       } else {
-        L[i][j] = s / L[j][j];
+        L[i][j] = s * inv[j];
       }
     }
   }
   double z[4];
+#pragma unroll
   for (int i = 0; i < 4; i++) {
     double s = -g[i];
+#pragma unroll
     for (int k = 0; k < i; k++) s -= L[i][k] * z[k];
-    z[i] = s / L[i][i];
+    z[i] = s * inv[i];
   }
+#pragma unroll
   for (int i = 3; i >= 0; i--) {
     double s = z[i];
+#pragma unroll
     for (int k = i + 1; k < 4; k++) s -= L[k][i] * dx[k];
-    dx[i] = s / L[i][i];
+    dx[i] = s * inv[i];
   }
   return 0;
 }
@@ -2796,54 +2793,61 @@ __device__ int solve4(const double *A, const double *D, double mu, const double 
 // BIS_FIT2 (BIS_FIT2.cpp:97-320) for one CCF per 64-lane block: the same
 // Levenberg-Marquardt restatement of GSL's trust-region solver as the oracle
 // (More scaling, Nielsen damping, xtol = gtol = 1e-8), then the bisector.
-// E_: per-point errors [n_ccf][n] (CCF_error.txt), NULL = unit errors; held in
-// s_p0 during the fit (s_p0 is bisector scratch afterwards).
+// E_: per-point errors [n_ccf][n] (CCF_error.txt), NULL = unit errors; their
+// reciprocals are held in s_p0 during the fit (s_p0 is bisector scratch afterwards).
 // status_ (optional): 0 when the xtol or gtol test ended the fit, 27 when no step
 // reduced the residual (GSL_ENOPROG: a flat or degenerate CCF), 11 after 10000
 // iterations (GSL_EMAXITER).
+// One wave per CCF, so a fit is a chain of dependent steps and its latency is the time:
+// the 15 sums of an evaluation share one folding reduction (wave_sums16), divisions by
+// sigma and the Cholesky diagonal are reciprocals, the two scans for a maximum and the
+// span's means are wave reductions, and the walk reads ahead.  LDS is sized by n, so
+// that a batch's fits fill the CU.
+// lds: fit_lds_bytes(n).
 __device__ __forceinline__ void fit_body(const double *v_, int n, const double *Y_, const double *E_, double *par_,
                                          double *model_, double *depth_out_, double *bis_out_, int32_t *iters_,
-                                         int bx_, int32_t *status_ = nullptr) {
+                                         int bx_, double *lds, int32_t *status_ = nullptr) {
   const GLOBAL double *v = gl(v_), *Y = gl(Y_);
   GLOBAL double *par = gw(par_), *model = gw(model_), *depth_out = gw(depth_out_), *bis_out = gw(bis_out_);
   GLOBAL int32_t *iters = gw(iters_);
-  __shared__ double s_px[kMaxV], s_y[kMaxV], s_nc[kMaxV], s_p0[kMaxV], s_p1[kMaxV], s_p2[kMaxV];
-  __shared__ double s_bis[91];
-  __shared__ double s_init[4];
-  int cidx = bx_;
+  double *s_px = lds, *s_y = lds + n, *s_nc = lds + 2 * n, *s_p0 = lds + 3 * n, *s_p1 = lds + 4 * n, *s_p2 = lds + 5 * n;
+  const int cidx = bx_, lane = threadIdx.x;
   const GLOBAL double *y = Y + (long)cidx * n;
-  for (int i = threadIdx.x; i < n; i += 64) {
-    s_px[i] = v[i] - v[0];
+  const double v00 = v[0];
+  for (int i = lane; i < n; i += 64) {
+    s_px[i] = v[i] - v00;
     s_y[i] = y[i];
   }
-  const double *s_err = nullptr;
+  const double *s_rerr = nullptr;
   if (E_) {
     const GLOBAL double *er = gl(E_) + (long)cidx * n;
-    for (int i = threadIdx.x; i < n; i += 64) s_p0[i] = er[i];
-    s_err = s_p0;
+    for (int i = lane; i < n; i += 64) s_p0[i] = 1.0 / er[i];
+    s_rerr = s_p0;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double c = (s_y[0] + s_y[n - 1]) / 2;
-    double fwhm = (s_px[n - 1] - s_px[0]) / 5.;
-    double k = 0., x0 = s_px[n / 2];
-    for (int i = 0; i < n; i++)
-      if (fabs(s_y[i] - c) > fabs(k)) {
-        k = s_y[i] - c;
-        x0 = s_px[i];
+  // start: the ends' mean, the first point farthest from it, a fifth of the range
+  double x[4] = {(s_y[0] + s_y[n - 1]) / 2, 0.0, s_px[n / 2], (s_px[n - 1] - s_px[0]) / 5.};
+  {
+    double best = 0.0;
+    int at = n;
+    for (int i = lane; i < n; i += 64) {
+      const double a = fabs(s_y[i] - x[0]);
+      if (a > best) {
+        best = a;
+        at = i;
       }
-    s_init[0] = c;
-    s_init[1] = k;
-    s_init[2] = x0;
-    s_init[3] = fwhm;
+    }
+    wave_argmax(best, at);
+    if (at < n) {
+      x[1] = s_y[at] - x[0];
+      x[2] = s_px[at];
+    }
   }
-  __syncthreads();
-  double x[4] = {s_init[0], s_init[1], s_init[2], s_init[3]};
   const double xtol = 1.0e-8, gtol = 1.0e-8;
   GaussEval ev;
-  gauss_eval(s_px, s_y, s_err, n, x, true, ev);
-  double D[4];
-  for (int a = 0; a < 4; a++) D[a] = sqrt(ev.colsq[a]) > 0 ? sqrt(ev.colsq[a]) : 1.0;
+  gauss_eval(s_px, s_y, s_rerr, n, x, ev);
+  double D2[4];  // squared column scales
+  for (int a = 0; a < 4; a++) D2[a] = symA(ev.A, a, a) > 0 ? symA(ev.A, a, a) : 1.0;
   double mu = 1.0e-3, nu = 2.0;
   int iter = 0, fit_status = 11;
   GaussEval et;
@@ -2852,7 +2856,7 @@ __device__ __forceinline__ void fit_body(const double *v_, int n, const double *
     int bad = 0;
     bool accepted = false;
     while (!accepted) {
-      if (solve4(ev.A, D, mu, ev.g, dx) != 0) {
+      if (solve4(ev.A, D2, mu, ev.g, dx) != 0) {
         mu *= nu;
         nu *= 2;
         if (++bad > 15) break;
@@ -2861,12 +2865,12 @@ __device__ __forceinline__ void fit_body(const double *v_, int n, const double *
       for (int a = 0; a < 4; a++) xt[a] = x[a] + dx[a];
       // the trial point with its Jacobian sums: an accepted trial's evaluation is
       // the next iteration's (the same sums at the same point)
-      gauss_eval(s_px, s_y, s_err, n, xt, true, et);
+      gauss_eval(s_px, s_y, s_rerr, n, xt, et);
       double pred = 0;
       for (int a = 0; a < 4; a++) {
         double Adx = 0;
         for (int b = 0; b < 4; b++) Adx += symA(ev.A, a, b) * dx[b];
-        pred += dx[a] * Adx + 2 * mu * D[a] * D[a] * dx[a] * dx[a];
+        pred += dx[a] * Adx + 2 * mu * D2[a] * dx[a] * dx[a];
       }
       double rho = pred > 0 ? (ev.sum_f2 - et.sum_f2) / pred : -1.0;
       if (rho > 0) {
@@ -2888,7 +2892,7 @@ __device__ __forceinline__ void fit_body(const double *v_, int n, const double *
     for (int a = 0; a < 4; a++) x[a] = xt[a];
     ev = et;
     for (int a = 0; a < 4; a++)
-      if (sqrt(ev.colsq[a]) > D[a]) D[a] = sqrt(ev.colsq[a]);
+      if (symA(ev.A, a, a) > D2[a]) D2[a] = symA(ev.A, a, a);
     bool small = true;
     for (int a = 0; a < 4; a++)
       if (!(fabs(dx[a]) < xtol * xtol + xtol * fabs(x[a]))) small = false;
@@ -2912,73 +2916,68 @@ __device__ __forceinline__ void fit_body(const double *v_, int n, const double *
   double c = x[0], k = x[1], x0 = x[2], fwhm = x[3];
   double sigma_m = fwhm / 2 / sqrt(2 * log(2.0));
   if (model)
-    for (int i = threadIdx.x; i < n; i += 64)
+    for (int i = lane; i < n; i += 64)
       model[(long)cidx * n + i] = c + k * exp(-(s_px[i] - x0) * (s_px[i] - x0) / 2 / sigma_m / sigma_m);
   // bisector, BIS_FIT2.cpp:214-268
   double sigma = fwhm / 2. / sqrt(2. * log(2.));
-  double v0 = x0 + v[0];
-  for (int i = threadIdx.x; i < n; i += 64) s_nc[i] = -c / k * (1. - s_y[i] / c);
-  __syncthreads();  // also: every lane is done with s_err (s_p0) before s_p0 is rewritten
-  for (int i = threadIdx.x; i < n - 1; i += 64) {
-    double vr = (v[i] + v[i + 1]) / 2.;
+  double v0 = x0 + v00;
+  for (int i = lane; i < n; i += 64) s_nc[i] = -c / k * (1. - s_y[i] / c);
+  __syncthreads();  // also: every lane is done with s_rerr (s_p0) before s_p0 is rewritten
+  for (int i = lane; i < n - 1; i += 64) {
+    const double va = v[i], vb = v[i + 1], na = s_nc[i], nb = s_nc[i + 1];
+    double vr = (va + vb) / 2.;
     double s2 = sigma * sigma;
     double dd = (vr - v0) * (vr - v0);
-    double dccf = -(vr - v0) / s2 * exp(-dd / 2. / s2);
-    double d2ccf = (dd / s2 - 1) / s2 * exp(-dd / 2. / s2);
+    double ex = exp(-dd / 2. / s2);
+    double dccf = -(vr - v0) / s2 * ex;
+    double d2ccf = (dd / s2 - 1) / s2 * ex;
     double d2rv = -d2ccf / (dccf * dccf * dccf);
     double p2 = d2rv / 2.;
-    double p1 = (v[i + 1] - v[i] - p2 * (s_nc[i + 1] * s_nc[i + 1] - s_nc[i] * s_nc[i])) / (s_nc[i + 1] - s_nc[i]);
+    double p1 = (vb - va - p2 * (nb * nb - na * na)) / (nb - na);
     s_p2[i] = p2;
     s_p1[i] = p1;
-    s_p0[i] = v[i] - p1 * s_nc[i] - p2 * (s_nc[i] * s_nc[i]);
+    s_p0[i] = va - p1 * na - p2 * (na * na);
   }
-  if (threadIdx.x == 0) {
+  if (lane == 0) {
     s_p0[n - 1] = 0;
     s_p1[n - 1] = 0;
     s_p2[n - 1] = 0;
   }
-  __syncthreads();
-  __shared__ int s_imax;
-  if (threadIdx.x == 0) {
-    int im = 0;
-    for (int i = 0; i < n; i++)
-      if (s_nc[i] > s_nc[im]) im = i;
-    s_imax = im;
+  int ind_max = 0;
+  {
+    double best = s_nc[0];
+    if (best == best) {  // a NaN first value keeps index 0, as the scan's comparisons do
+      for (int i = lane; i < n; i += 64)
+        if (s_nc[i] > best) {
+          best = s_nc[i];
+          ind_max = i;
+        }
+      wave_argmax(best, ind_max);
+    }
   }
   __syncthreads();
-  int ind_max = s_imax;
-  for (int i = threadIdx.x; i < 91; i += 64) {
+  double top = 0., bot = 0.;  // depths in [0.1, 0.4] and [0.6, 0.9]: 31 levels each
+  for (int i = lane; i < 91; i += 64) {
     double dep = (double)(i + 5) / 100;
-    int i_b = ind_max, i_r = ind_max;
-    while ((s_nc[i_b] > dep) && (i_b > 1)) i_b--;
-    while ((s_nc[i_r + 1] > dep) && (i_r < (n - 2))) i_r++;
+    int i_b, i_r;
+    bisector_walk(s_nc, n, ind_max, dep, i_b, i_r);
     double b = (s_p0[i_b] + s_p0[i_r]) + (s_p1[i_b] + s_p1[i_r]) * dep + (s_p2[i_b] + s_p2[i_r]) * (dep * dep);
     b /= 2.;
-    s_bis[i] = b;
+    if (dep >= 0.1 && dep <= 0.4) top += b;
+    if (dep >= 0.6 && dep <= 0.9) bot += b;
     if (bis_out) bis_out[(long)cidx * 91 + i] = b;
     if (depth_out) depth_out[(long)cidx * 91 + i] = 1.0 - fabs(k) * dep;
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int n1 = 0, n2 = 0;
-    double top = 0., bot = 0.;
-    for (int i = 0; i < 91; i++) {
-      double dep = (double)(i + 5) / 100;
-      if ((dep >= 0.1) && (dep <= 0.4)) {
-        n1++;
-        top += s_bis[i];
-      }
-      if ((dep >= 0.6) && (dep <= 0.9)) {
-        n2++;
-        bot += s_bis[i];
-      }
-    }
-    top /= n1;
-    bot /= n2;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    top += __shfl_xor(top, off);
+    bot += __shfl_xor(bot, off);
+  }
+  if (lane == 0) {
     GLOBAL double *pp = par + (long)cidx * 5;
     pp[0] = c;
     pp[1] = fabs(k);
-    pp[2] = top - bot;
+    pp[2] = top / 31 - bot / 31;
     pp[3] = v0;
     pp[4] = fwhm;
     if (iters) iters[cidx] = iter;
@@ -2986,17 +2985,20 @@ __device__ __forceinline__ void fit_body(const double *v_, int n, const double *
   }
 }
 
+size_t fit_lds_bytes(int n_v) { return (size_t)6 * n_v * sizeof(double); }
+
 __global__ __launch_bounds__(64) void k_fit(const double *v, int n, const double *Y, const double *E, double *par,
                                             double *model, double *depth_out, double *bis_out, int32_t *iters,
                                             int32_t *status) {
-  fit_body(v, n, Y, E, par, model, depth_out, bis_out, iters, blockIdx.x, status);
+  extern __shared__ double fit_lds[];
+  fit_body(v, n, Y, E, par, model, depth_out, bis_out, iters, blockIdx.x, fit_lds, status);
 }
 
 hipError_t launch_fit(const double *v, int n_v, const double *y, const double *err, int n_ccf, double *par,
                       double *model, double *depth, double *bis, int32_t *iters, hipStream_t s, int32_t *status) {
   if (n_ccf == 0) return hipSuccess;
   if (n_v > kMaxV || n_v < 3) return hipErrorInvalidValue;
-  k_fit<<<n_ccf, 64, 0, s>>>(v, n_v, y, err, par, model, depth, bis, iters, status);
+  k_fit<<<n_ccf, 64, fit_lds_bytes(n_v), s>>>(v, n_v, y, err, par, model, depth, bis, iters, status);
   return hipGetLastError();
 }
 
@@ -3150,8 +3152,9 @@ __global__ __launch_bounds__(1024) void kb_ccf_reduce(SOAP_BATCH_ARGS(CcfRedJob)
 
 template <bool P>
 __global__ __launch_bounds__(64) void kb_fit(SOAP_BATCH_ARGS(FitJob)) {
+  extern __shared__ double fit_lds[];
   batch_loop<P>(jobs, prefix, n_inst, total, [&](const FitJob &j, int local) {
-    fit_body(j.v, j.n_v, j.y, nullptr, j.par, j.model, j.depth, j.bis, j.iters, local);
+    fit_body(j.v, j.n_v, j.y, nullptr, j.par, j.model, j.depth, j.bis, j.iters, local, fit_lds);
   });
 }
 
