@@ -170,29 +170,35 @@ __global__ __launch_bounds__(kDT) void k_diff_taps(DiffArgs a, int cells_per_blo
   }
 }
 
-// fixed point -> taps [p][k][d][ns] and the nonzero range per (p, k)
-__global__ void k_diff_taps_finalize(DiffArgs a) {
-  int p = blockIdx.x;
-  const int ns = a.ns;
-  for (int k = threadIdx.x; k < a.n_mu; k += blockDim.x) {
-    int lo = a.nd, hi = -1;
-    for (int d = 0; d < a.nd; d++) {
-      const unsigned long long *e = a.acc + (((long)p * a.n_mu + k) * a.nd + d) * ns * 2;
-      double *o = a.taps + (((long)p * a.n_mu + k) * a.nd + d) * ns;
-      bool nz = false;
-      for (int q = 0; q < ns; q++) {
-        double v = fx_value(e[q * 2], e[q * 2 + 1]);
-        o[q] = v;
-        nz |= v != 0.0;
-      }
-      if (nz) {
-        lo = d < lo ? d : lo;
-        hi = d;
-      }
-    }
-    a.krange[((long)p * a.n_mu + k) * 2] = lo;
-    a.krange[((long)p * a.n_mu + k) * 2 + 1] = hi;
+// fixed point -> taps [p][k][d][ns] and the nonzero range per (p, k).  One thread per
+// (bin, offset) of a phase; the ranges are formed in LDS (one thread per bin walked its
+// offsets in turn before: 15-86 us against 3-6 us).
+__global__ __launch_bounds__(kDT) void k_diff_taps_finalize(DiffArgs a) {
+  extern __shared__ int s_rg[];  // [n_mu][2]: lo, hi
+  const int p = blockIdx.x, ns = a.ns, nd = a.nd, n_mu = a.n_mu;
+  for (int k = threadIdx.x; k < n_mu; k += blockDim.x) {
+    s_rg[2 * k] = nd;
+    s_rg[2 * k + 1] = -1;
   }
+  __syncthreads();
+  const long base = (long)p * n_mu * nd;
+  for (int e = threadIdx.x; e < n_mu * nd; e += blockDim.x) {
+    const int k = e / nd, d = e - k * nd;
+    const unsigned long long *in = a.acc + (base + e) * ns * 2;
+    double *o = a.taps + (base + e) * ns;
+    bool nz = false;
+    for (int q = 0; q < ns; q++) {
+      const double v = fx_value(in[q * 2], in[q * 2 + 1]);
+      o[q] = v;
+      nz |= v != 0.0;
+    }
+    if (nz) {
+      atomicMin(s_rg + 2 * k, d);
+      atomicMax(s_rg + 2 * k + 1, d);
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < 2 * n_mu; e += blockDim.x) a.krange[(long)p * n_mu * 2 + e] = s_rg[e];
 }
 
 // I_p[j] = sum_k sum_d HQ[d] Q_k[j - dmin - d] + HS[d] S_k[j - dmin - d] (+ HF[d] Fa_k[j - dmin - d]);
@@ -275,92 +281,144 @@ __global__ __launch_bounds__(kDT) void k_diff_conv(DiffArgs a, ConvArgs c, const
 
 // ------------------------------------------------------------ Gaussian fit: polish and adjoint
 // gradient (4) and Hessian (10, upper) of 0.5 sum r^2 (BIS_FIT2 model, exact second
-// derivatives), summed over the wave's lanes; every lane receives the totals
-__device__ void gauss_gh(const double *x, const double *y, int n, const double th[4], double g[4], double H[4][4],
-                         double *r2out) {
-  double s = th[3] / (2 * sqrt(2 * log(2.0)));
-  double acc[15];
+// derivatives), summed over the wave's lanes; every lane receives the totals.  Three
+// points of a lane are in flight together; points past n add zeros.
+__device__ __forceinline__ void gauss_gh(const double *x, const double *y, int n, const double (&th)[4], double (&g)[4],
+                                         double (&H)[4][4], double *r2out) {
+  const double rs = 2 * sqrt(2 * log(2.0)) / th[3], rf = 1.0 / th[3];
+  double v[16];
 #pragma unroll
-  for (int i = 0; i < 15; i++) acc[i] = 0.0;
-  for (int i = threadIdx.x & 63; i < n; i += 64) {
-    double u = (x[i] - th[2]) / s, e = exp(-u * u / 2);
-    double r = th[0] + th[1] * e - y[i];
-    double j4[4] = {1.0, e, th[1] * e * u / s, th[1] * e * u * u / th[3]};
-    double h12 = e * u / s, h13 = e * u * u / th[3];
-    double h22 = th[1] * e * (u * u - 1) / (s * s), h23 = th[1] * e * u * (u * u - 2) / (s * th[3]);
-    double h33 = th[1] * e * u * u * (u * u - 3) / (th[3] * th[3]);
-    int q = 0;
-    for (int a = 0; a < 4; a++) acc[q++] += j4[a] * r;
-    double hh[4][4] = {{0, 0, 0, 0}, {0, 0, h12, h13}, {0, h12, h22, h23}, {0, h13, h23, h33}};
-    for (int a = 0; a < 4; a++)
-      for (int b = a; b < 4; b++) acc[q++] += j4[a] * j4[b] + r * hh[a][b];
-    acc[14] += r * r;
+  for (int q = 0; q < 16; q++) v[q] = 0.0;
+  const int lane = threadIdx.x & 63;
+  for (int i0 = lane; i0 - lane < n; i0 += 192) {
+#pragma unroll
+    for (int w = 0; w < 3; w++) {
+      const bool in = i0 + 64 * w < n;
+      const int i = in ? i0 + 64 * w : n - 1;
+      const double u = (x[i] - th[2]) * rs, ex = exp(-0.5 * u * u);
+      const double e = in ? ex : 0.0, r = in ? th[0] + th[1] * e - y[i] : 0.0;
+      const double eu = e * u, ku = th[1] * eu;
+      const double j4[4] = {in ? 1.0 : 0.0, e, ku * rs, ku * u * rf};
+      const double hh[4][4] = {{0, 0, 0, 0},
+                               {0, 0, eu * rs, eu * u * rf},
+                               {0, 0, th[1] * e * (u * u - 1) * rs * rs, ku * (u * u - 2) * rs * rf},
+                               {0, 0, 0, ku * u * (u * u - 3) * rf * rf}};
+      int q = 4;
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        v[a] = fma(j4[a], r, v[a]);
+#pragma unroll
+        for (int b = a; b < 4; b++, q++) v[q] += j4[a] * j4[b] + r * hh[a][b];
+      }
+      v[14] = fma(r, r, v[14]);
+    }
   }
+  wave_sums16(v);
+  int q = 4;
 #pragma unroll
-  for (int i = 0; i < 15; i++)
-    for (int off = 32; off > 0; off >>= 1) acc[i] += __shfl_xor(acc[i], off);
-  int q = 0;
-  for (int a = 0; a < 4; a++) g[a] = acc[q++];
-  for (int a = 0; a < 4; a++)
-    for (int b = a; b < 4; b++) H[a][b] = H[b][a] = acc[q++];
-  *r2out = acc[14];
+  for (int a = 0; a < 4; a++) {
+    g[a] = v[a];
+#pragma unroll
+    for (int b = a; b < 4; b++) H[a][b] = H[b][a] = v[q++];
+  }
+  *r2out = v[14];
 }
 
-__device__ int solve4(const double A_in[4][4], const double *b, double *x) {
+// Gaussian elimination with row pivoting.  Each column's largest entry is brought up by
+// exchanges with constant indices (selects), so that the system stays in registers.
+__device__ __forceinline__ int solve4(const double (&A_in)[4][4], const double (&b)[4], double (&x)[4]) {
   double A[4][5];
+#pragma unroll
   for (int i = 0; i < 4; i++) {
+#pragma unroll
     for (int j = 0; j < 4; j++) A[i][j] = A_in[i][j];
     A[i][4] = b[i];
   }
+  double inv[4];
+#pragma unroll
   for (int col = 0; col < 4; col++) {
-    int piv = col;
-    for (int r = col + 1; r < 4; r++)
-      if (fabs(A[r][col]) > fabs(A[piv][col])) piv = r;
-    if (A[piv][col] == 0.0) return -1;
-    if (piv != col)
-      for (int j = 0; j < 5; j++) {
-        double t = A[col][j];
-        A[col][j] = A[piv][j];
-        A[piv][j] = t;
-      }
+#pragma unroll
     for (int r = col + 1; r < 4; r++) {
-      double f = A[r][col] / A[col][col];
-      for (int j = col; j < 5; j++) A[r][j] -= f * A[col][j];
+      const bool up = fabs(A[r][col]) > fabs(A[col][col]);
+#pragma unroll
+      for (int j = col; j < 5; j++) {
+        const double t = A[col][j];
+        A[col][j] = up ? A[r][j] : t;
+        A[r][j] = up ? t : A[r][j];
+      }
+    }
+    if (A[col][col] == 0.0) return -1;
+    inv[col] = 1.0 / A[col][col];
+#pragma unroll
+    for (int r = col + 1; r < 4; r++) {
+      const double f = A[r][col] * inv[col];
+#pragma unroll
+      for (int j = col + 1; j < 5; j++) A[r][j] -= f * A[col][j];
     }
   }
+#pragma unroll
   for (int i = 3; i >= 0; i--) {
     double s = A[i][4];
+#pragma unroll
     for (int j = i + 1; j < 4; j++) s -= A[i][j] * x[j];
-    x[i] = s / A[i][i];
+    x[i] = s * inv[i];
   }
   return 0;
 }
 
 // one wave per CCF: theta from the fit parameters (signed amplitude), then
-// damped Newton steps on the exact Hessian to the least-squares optimum
-__global__ void k_fit_polish(const double *v, int n_v, const double *ccf, const double *par, double *theta) {
-  int sp = blockIdx.x;
-  const double *y = ccf + (long)sp * n_v;
+// damped Newton steps on the exact Hessian to the least-squares optimum.
+// A full Newton step below kPolishStep of the amplitude and the width is the end of the search: it
+// changes the residual by less than its rounding ((1e-7)^2 of it), so comparing
+// residuals there decides nothing and used to try up to thirty damped steps (461 us for
+// the 50 CCFs of the full adjoint, a chain of about 150 evaluations).  The two undamped
+// steps that follow take 1e-7 to rounding.
+constexpr double kPolishStep = 1e-7;
+__global__ __launch_bounds__(64) void k_fit_polish(const double *v, int n_v, const double *ccf, const double *par,
+                                                   double *theta) {
+  extern __shared__ double s_fit[];  // velocities, CCF
+  const int sp = blockIdx.x, lane = threadIdx.x;
+  double *s_v = s_fit, *s_y = s_fit + n_v;
   const double *pp = par + (long)sp * 5;
-  int inear = 0;
-  for (int i = 1; i < n_v; i++)
-    if (fabs(v[i] - pp[3]) < fabs(v[inear] - pp[3])) inear = i;
-  double th[4] = {pp[0], y[inear] < pp[0] ? -pp[1] : pp[1], pp[3], pp[4]};
+  const double c0 = pp[0], k0 = pp[1], x0 = pp[3], f0 = pp[4];
+  double best = -HUGE_VAL;
+  int inear = n_v;
+  for (int i = lane; i < n_v; i += 64) {
+    const double x = v[i], d = -fabs(x - x0);
+    s_v[i] = x;
+    s_y[i] = ccf[(long)sp * n_v + i];
+    if (d > best) {
+      best = d;
+      inear = i;
+    }
+  }
+  wave_argmax(best, inear);
+  if (inear >= n_v) inear = 0;  // NaN centre
+  __syncthreads();
+  double th[4] = {c0, s_y[inear] < c0 ? -k0 : k0, x0, f0};
   double g[4], H[4][4], r2;
-  gauss_gh(v, y, n_v, th, g, H, &r2);
+  gauss_gh(s_v, s_y, n_v, th, g, H, &r2);
   for (int it = 0; it < 60; it++) {
-    double mu = 0.0, dx[4] = {0, 0, 0, 0}, tn[4] = {th[0], th[1], th[2], th[3]}, r2n = r2;
-    bool ok = false;
+    double mu = 0.0, dx[4] = {0, 0, 0, 0}, tn[4], gn[4], Hn[4][4], r2n = r2;
+    bool ok = false, small = false;
     for (int tries = 0; tries < 30; tries++) {
       double Hd[4][4], mg[4];
+#pragma unroll
       for (int a = 0; a < 4; a++) {
         mg[a] = -g[a];
+#pragma unroll
         for (int b = 0; b < 4; b++) Hd[a][b] = H[a][b] + (a == b ? mu * (fabs(H[a][a]) + 1e-300) : 0.0);
       }
       if (solve4(Hd, mg, dx) == 0) {
+#pragma unroll
         for (int a = 0; a < 4; a++) tn[a] = th[a] + dx[a];
-        double gn[4], Hn[4][4];
-        gauss_gh(v, y, n_v, tn, gn, Hn, &r2n);
+        const double sk = kPolishStep * fabs(th[1]), sf = kPolishStep * fabs(th[3]);
+        const bool tiny = mu == 0.0 && fabs(dx[0]) <= sk && fabs(dx[1]) <= sk && fabs(dx[2]) <= sf && fabs(dx[3]) <= sf;
+        if (tiny) {
+          ok = small = true;
+          break;
+        }
+        gauss_gh(s_v, s_y, n_v, tn, gn, Hn, &r2n);
         if (r2n <= r2 * (1 + 1e-15)) {
           ok = true;
           break;
@@ -369,22 +427,35 @@ __global__ void k_fit_polish(const double *v, int n_v, const double *ccf, const 
       mu = mu == 0.0 ? 1e-6 : mu * 10;
     }
     if (!ok) break;
-    bool small = true;
-    for (int a = 0; a < 4; a++)
-      if (fabs(dx[a]) > 1e-12 * fabs(th[a]) + 1e-300) small = false;
+    if (!small) {
+      small = true;
+#pragma unroll
+      for (int a = 0; a < 4; a++)
+        if (fabs(dx[a]) > 1e-12 * fabs(th[a]) + 1e-300) small = false;
+      r2 = r2n;
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        g[a] = gn[a];
+#pragma unroll
+        for (int b = 0; b < 4; b++) H[a][b] = Hn[a][b];
+      }
+    }
+#pragma unroll
     for (int a = 0; a < 4; a++) th[a] = tn[a];
-    gauss_gh(v, y, n_v, th, g, H, &r2);
     if (small) break;
   }
   // two undamped Newton steps on the gradient fix the optimum to rounding
   for (int it = 0; it < 2; it++) {
     double mg[4], dx[4];
-    gauss_gh(v, y, n_v, th, g, H, &r2);
+    gauss_gh(s_v, s_y, n_v, th, g, H, &r2);
+#pragma unroll
     for (int a = 0; a < 4; a++) mg[a] = -g[a];
     if (solve4(H, mg, dx) != 0) break;
+#pragma unroll
     for (int a = 0; a < 4; a++) th[a] += dx[a];
   }
-  if (threadIdx.x == 0)
+  if (lane == 0)
+#pragma unroll
     for (int a = 0; a < 4; a++) theta[(long)sp * 4 + a] = th[a];
 }
 
@@ -447,10 +518,10 @@ __device__ void bis_p2(double vr, double v0, double s2, double *p2, double *dp2_
 constexpr int kBisLevels = 91;
 __global__ __launch_bounds__(64) void k_diff_bis(const double *v, int n_v, const double *ccf, const double *theta,
                                                  double *bisd) {
-  __shared__ double s_nc[kMaxVDiff], s_p0[kMaxVDiff], s_p1[kMaxVDiff], s_p2[kMaxVDiff];
-  __shared__ double s_bis[kBisLevels], s_dA[kBisLevels][2], s_dB[kBisLevels][2], s_th[kBisLevels][4];
+  extern __shared__ double s_bis[];  // norm, p0, p1, p2
+  double *s_nc = s_bis, *s_p0 = s_bis + n_v, *s_p1 = s_bis + 2 * n_v, *s_p2 = s_bis + 3 * n_v;
+  __shared__ double s_dA[kBisLevels][2], s_dB[kBisLevels][2];
   __shared__ int s_side[kBisLevels][2];
-  __shared__ int s_imax;
   const int sp = blockIdx.x;
   const double *y = ccf + (long)sp * n_v;
   double *out = bisd + (long)sp * (n_v + kBisHead);
@@ -467,24 +538,31 @@ __global__ __launch_bounds__(64) void k_diff_bis(const double *v, int n_v, const
     s_p1[i] = p1;
     s_p0[i] = v[i] - p1 * s_nc[i] - p2 * (s_nc[i] * s_nc[i]);
   }
-  if (threadIdx.x == 0) {
-    int im = 0;
-    for (int i = 0; i < n_v; i++)
-      if (s_nc[i] > s_nc[im]) im = i;
-    s_imax = im;
+  if (threadIdx.x == 0) s_p0[n_v - 1] = s_p1[n_v - 1] = s_p2[n_v - 1] = 0.0;
+  int ind_max = 0;
+  {
+    double best = s_nc[0];
+    if (best == best) {  // a NaN first value keeps index 0, as the scan's comparisons do
+      for (int i = threadIdx.x; i < n_v; i += 64)
+        if (s_nc[i] > best) {
+          best = s_nc[i];
+          ind_max = i;
+        }
+      wave_argmax(best, ind_max);
+    }
   }
   __syncthreads();
-  const int ind_max = s_imax;
+  double top = 0., bot = 0., th4[4] = {0, 0, 0, 0};
   for (int i = threadIdx.x; i < kBisLevels; i += 64) {
     double dep = (double)(i + 5) / 100;
-    int i_b = ind_max, i_r = ind_max;
-    while ((s_nc[i_b] > dep) && (i_b > 1)) i_b--;
-    while ((s_nc[i_r + 1] > dep) && (i_r < (n_v - 2))) i_r++;
+    int i_b, i_r;
+    bisector_walk(s_nc, n_v, ind_max, dep, i_b, i_r);
     double b = (s_p0[i_b] + s_p0[i_r]) + (s_p1[i_b] + s_p1[i_r]) * dep + (s_p2[i_b] + s_p2[i_r]) * (dep * dep);
-    s_bis[i] = b / 2.;
+    b /= 2.;
+    if (dep >= 0.1 && dep <= 0.4) top += b;
+    if (dep >= 0.6 && dep <= 0.9) bot += b;
     // weight of this level in the span, halved for the mean of the two sides
     double w = ((dep >= 0.1) && (dep <= 0.4)) ? 0.5 / 31 : ((dep >= 0.6) && (dep <= 0.9)) ? -0.5 / 31 : 0.0;
-    double th4[4] = {0, 0, 0, 0};
     for (int side = 0; side < 2; side++) {
       int sx = side ? i_r : i_b;
       s_side[i][side] = sx;
@@ -505,37 +583,45 @@ __global__ __launch_bounds__(64) void k_diff_bis(const double *v, int n_v, const
       th4[2] += dP * dp2_v0;
       th4[3] += dP * dp2_s2 * 2 * s2 / fwhm;
     }
-    for (int q4 = 0; q4 < 4; q4++) s_th[i][q4] = th4[q4];
   }
   __syncthreads();
+  // dspan/dy_j: the levels' sides in order, kBisU reads ahead of their adds
+  constexpr int kBisU = 7;
+  static_assert(kBisLevels % kBisU == 0, "levels per pass");
   for (int j = threadIdx.x; j < n_v; j += 64) {
     double g = 0.0;
-    for (int i = 0; i < kBisLevels; i++)
-      for (int side = 0; side < 2; side++) {
-        int sx = s_side[i][side];
-        if (sx == j) g += s_dA[i][side];
-        if (sx + 1 == j) g += s_dB[i][side];
-      }
+    for (int i = 0; i < kBisLevels; i += kBisU) {
+      int sx[kBisU][2];
+      double dA[kBisU][2], dB[kBisU][2];
+#pragma unroll
+      for (int u = 0; u < kBisU; u++)
+#pragma unroll
+        for (int side = 0; side < 2; side++) {
+          sx[u][side] = s_side[i + u][side];
+          dA[u][side] = s_dA[i + u][side];
+          dB[u][side] = s_dB[i + u][side];
+        }
+#pragma unroll
+      for (int u = 0; u < kBisU; u++)
+#pragma unroll
+        for (int side = 0; side < 2; side++) {
+          g += sx[u][side] == j ? dA[u][side] : 0.0;
+          g += sx[u][side] + 1 == j ? dB[u][side] : 0.0;
+        }
+    }
     out[kBisHead + j] = g;
   }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    top += __shfl_xor(top, off);
+    bot += __shfl_xor(bot, off);
+#pragma unroll
+    for (int q4 = 0; q4 < 4; q4++) th4[q4] += __shfl_xor(th4[q4], off);
+  }
   if (threadIdx.x == 0) {
-    int n1 = 0, n2 = 0;
-    double top = 0., bot = 0.;
-    double th4[4] = {0, 0, 0, 0};
-    for (int i = 0; i < kBisLevels; i++) {
-      double dep = (double)(i + 5) / 100;
-      if ((dep >= 0.1) && (dep <= 0.4)) {
-        n1++;
-        top += s_bis[i];
-      }
-      if ((dep >= 0.6) && (dep <= 0.9)) {
-        n2++;
-        bot += s_bis[i];
-      }
-      for (int q4 = 0; q4 < 4; q4++) th4[q4] += s_th[i][q4];
-    }
-    out[0] = top / n1 - bot / n2;
+    out[0] = top / 31 - bot / 31;  // 31 levels in each range
     out[1] = 0.0;
+#pragma unroll
     for (int q4 = 0; q4 < 4; q4++) out[2 + q4] = th4[q4];
   }
 }
@@ -544,7 +630,7 @@ hipError_t launch_diff_bis(const double *v, int n_v, const double *ccf, const do
                            hipStream_t s) {
   if (n_ccf == 0) return hipSuccess;
   if (n_v < 3 || n_v > kMaxVDiff) return hipErrorInvalidValue;
-  k_diff_bis<<<n_ccf, 64, 0, s>>>(v, n_v, ccf, theta, bisd);
+  k_diff_bis<<<n_ccf, 64, (size_t)4 * n_v * sizeof(double), s>>>(v, n_v, ccf, theta, bisd);
   return hipGetLastError();
 }
 
@@ -907,7 +993,8 @@ hipError_t launch_diff_forward_spectra(const DiffArgs &a, const ConvArgs &c, con
   else
     k_diff_taps<2><<<gt, kDT, use_lds ? nacc * 8 : 0, s>>>(a, cpb, use_lds);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  k_diff_taps_finalize<<<a.n_phase, 64, 0, s>>>(a);
+  if ((size_t)a.n_mu * 8 > 65536) return hipErrorInvalidValue;
+  k_diff_taps_finalize<<<a.n_phase, kDT, (size_t)a.n_mu * 8, s>>>(a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   size_t lds_fir = (size_t)a.ns * (kDT + a.nd - 1) * sizeof(double);
   if (lds_fir > 65536) return hipErrorInvalidValue;
@@ -942,8 +1029,19 @@ __global__ __launch_bounds__(kDT) void k_diff_loss(int n_phase, int res_blocks, 
                                                    double *dth) {
   extern __shared__ double term[];  // [n_phase]
   for (int p = threadIdx.x; p < n_phase; p += blockDim.x) {
+    // the residual partials in order, kResU loads ahead of their adds
+    constexpr int kResU = 16;
+    const double *rp = res_part + (long)p * res_blocks;
     double r2 = 0;
-    for (int b = 0; b < res_blocks; b++) r2 += res_part[(long)p * res_blocks + b];
+    int b = 0;
+    for (; b + kResU <= res_blocks; b += kResU) {
+      double x[kResU];
+#pragma unroll
+      for (int u = 0; u < kResU; u++) x[u] = rp[b + u];
+#pragma unroll
+      for (int u = 0; u < kResU; u++) r2 += x[u];
+    }
+    for (; b < res_blocks; b++) r2 += rp[b];
     double drv = theta[p * 4 + 2] - rv_t[p], dfw = theta[p * 4 + 3] - fw_t[p];
     double t = w_spec * r2 + w_rv * drv * drv + w_fw * dfw * dfw;
     double d4[4] = {0.0, 0.0, 2 * w_rv * drv, 2 * w_fw * dfw};
@@ -1022,7 +1120,8 @@ int diff_cell_blocks(int64_t ncell) { return (int)((ncell + kDT - 1) / kDT); }
 hipError_t launch_fit_polish(const double *v, int n_v, const double *ccf, const double *par, int n_ccf, double *theta,
                              hipStream_t s) {
   if (n_ccf == 0) return hipSuccess;
-  k_fit_polish<<<n_ccf, 64, 0, s>>>(v, n_v, ccf, par, theta);
+  if (n_v < 1 || n_v > kMaxVDiff) return hipErrorInvalidValue;
+  k_fit_polish<<<n_ccf, 64, (size_t)2 * n_v * sizeof(double), s>>>(v, n_v, ccf, par, theta);
   return hipGetLastError();
 }
 
