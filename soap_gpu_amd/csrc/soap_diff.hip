@@ -25,8 +25,19 @@ namespace soap {
 
 constexpr int kDT = 256;
 
-// ------------------------------------------------------------ per cell
-__global__ void k_diff_cells(DiffArgs a) {
+// ------------------------------------------------------------ the disk
+// Under rigid rotation every cell of a disk row has the same shift (m, t), and a row
+// crosses each mu bin in one or two runs, so a phase's taps, scalar gradients and map
+// gradients need the cells only through sums over runs ("pieces"): with a = 1 - mu and
+// b = 1 + LB(mu), the limb L = 1 - u1 a - u2 a^2 is a combination of 1, a, a^2, and
+//   sum_c L phi = M0 - u1 M1 - u2 M2,  M_q = sum_c a^q phi,
+// likewise for psi and b psi.  The kernels below form those sums once per (piece,
+// phase), lanes over phases and cells in turn (no reduction across lanes and no
+// atomics: every sum has a fixed order), and everything after works on pieces: 12,500 of
+// them instead of 283,000 cells at grid 600 with 10 bins.
+
+// per-cell tables of the plan
+__global__ void k_diff_cells(DiffArgs a, const double *mu_bounds, int32_t *ck, double2 *cell) {
 #pragma clang fp contract(off)
   long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   long ncell = (long)a.grid * a.grid;
@@ -34,171 +45,235 @@ __global__ void k_diff_cells(DiffArgs a) {
   int iy = (int)(idx / a.grid), iz = (int)(idx % a.grid);
   double y = -1. + iy * (2. / a.grid), z = -1. + iz * (2. / a.grid);
   if (!(y * y + z * z <= 1.)) {
-    a.ck[idx] = -1;
+    ck[idx] = -1;
+    cell[idx] = make_double2(0.0, 0.0);
     return;
   }
   double mu = sqrt(1. - (y * y + z * z));
   int k = a.n_mu - 1;
   for (int b = 0; b < a.n_mu - 1; b++)
-    if (mu > a.mu_bounds[b]) {
+    if (mu > mu_bounds[b]) {
       k = b;
       break;
     }
-  const double u1 = a.prm ? a.prm[1] : a.u1, u2 = a.prm ? a.prm[2] : a.u2, vsini = a.prm ? a.prm[0] : a.vsini;
-  double L = 1. - u1 * (1 - mu) - u2 * (1 - mu) * (1 - mu);
-  double delta = vsini * y;
-  double beta = delta * 1000. / kC;
-  double g = sqrt((1 + beta) / (1 - beta));
-  double fbeta = -1 * (1 - g);
-  double sh = log1p(fbeta) / a.h;
-  double mc = ceil(sh);
-  double t = expm1((mc - sh) * a.h) / a.expm1_h;
-  a.ck[idx] = k;
-  a.cm[idx] = (int32_t)mc;
-  a.ct[idx] = t;
-  a.cL[idx] = L;
-  a.cmu[idx] = mu;
-  // dt/d(delta) = -exp((m-s)h)/expm1(h) / (g^2 (1-beta)^2) * 1000/c (m piecewise constant)
-  a.cdt[idx] = -exp((mc - sh) * a.h) / a.expm1_h / (g * g * (1 - beta) * (1 - beta)) * (1000. / kC) * y;
+  ck[idx] = k;
+  // facula intensity factor 1 + LB(mu) (SOAP_initialize.cu:367, SOAP_integration.cu:317-323)
+  cell[idx] = make_double2(1. - mu, 1. + (a.lb[0] + a.lb[1] * mu + a.lb[2] * mu * mu + a.lb[3] * mu * mu * mu));
 }
 
-// bilinear sample of map p at the cell; i0, j0, fy, fz of the sample
-__device__ __forceinline__ double map_sample(const double *mp, int M, double y, double z, int &i0, int &j0,
-                                             double &fy, double &fz) {
-#pragma clang fp contract(off)
-  double gy = (y + 1) * 0.5 * (M - 1), gz = (z + 1) * 0.5 * (M - 1);
-  i0 = (int)floor(gy);
-  j0 = (int)floor(gz);
-  i0 = i0 > M - 2 ? M - 2 : (i0 < 0 ? 0 : i0);
-  j0 = j0 > M - 2 ? M - 2 : (j0 < 0 ? 0 : j0);
-  fy = gy - i0;
-  fz = gz - j0;
-  return (1 - fy) * (1 - fz) * mp[i0 * M + j0] + fy * (1 - fz) * mp[(i0 + 1) * M + j0] +
-         (1 - fy) * fz * mp[i0 * M + j0 + 1] + fy * fz * mp[(i0 + 1) * M + j0 + 1];
-}
-
-__device__ __forceinline__ void cell_yz(long idx, int grid, double &y, double &z) {
-#pragma clang fp contract(off)
-  int iy = (int)(idx / grid), iz = (int)(idx % grid);
-  y = -1. + iy * (2. / grid);
-  z = -1. + iz * (2. / grid);
-}
-
-// facula intensity factor 1 + LB(mu) (SOAP_initialize.cu:367, SOAP_integration.cu:317-323)
-__device__ __forceinline__ double lb_factor(const DiffArgs &a, double mu) {
-#pragma clang fp contract(off)
-  return 1. + (a.lb[0] + a.lb[1] * mu + a.lb[2] * mu * mu + a.lb[3] * mu * mu * mu);
-}
-
-// taps of every phase (blockIdx.y): fixed-point sums in LDS when they fit, then global.
-// All cells of one disk row share the shift (m, t), and neighbouring cells of a row
-// share the mu bin, so each wave first sums its lanes' weights over runs of equal
-// (row, bin) (a segmented shuffle scan, lanes = consecutive cells); the last lane of
-// each run adds the run's four tap terms.  This removes the many-way atomic
-// contention of one atomic per cell on the same few tap addresses.
-template <int NS>
-__global__ __launch_bounds__(kDT) void k_diff_taps(DiffArgs a, int cells_per_block, int use_lds) {
-  const double kappa = a.prm ? a.prm[3] : a.kappa;
-  const double kappa_f = a.prm ? a.prm[4] : a.kappa_f;
-  extern __shared__ unsigned long long lacc[];  // [n_mu][nd][NS sets][2]
-  int p = blockIdx.y;
-  long ncell = (long)a.grid * a.grid;
-  long c0 = (long)blockIdx.x * cells_per_block, c1 = min(ncell, c0 + cells_per_block);
-  long nacc = (long)a.n_mu * a.nd * NS * 2;
-  unsigned long long *gacc = a.acc + (long)p * nacc;
-  if (use_lds) {
-    for (long e = threadIdx.x; e < nacc; e += blockDim.x) lacc[e] = 0ull;
-    __syncthreads();
+__global__ void k_diff_psum(DiffArgs a, double2 *psum) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n_piece) return;
+  const DiffPiece pc = a.piece[i];
+  double s1 = 0.0, s2 = 0.0;
+  for (int c = 0; c < pc.len; c++) {
+    const double ca = a.cell[(long)pc.iy * a.grid + pc.iz0 + c].x;
+    s1 += ca;
+    s2 = fma(ca, ca, s2);
   }
-  unsigned long long *dst = use_lds ? lacc : gacc;
-  const double *mp = a.maps + (long)p * a.map_res * a.map_res;
-  const double *fp = NS == 3 ? a.fmaps + (long)p * a.map_res * a.map_res : nullptr;
+  psum[i] = make_double2(s1, s2);
+}
+
+// Shift of every disk row, and what follows from it: the rows of each tap index and the
+// lags of each bin (over all rows between the bin's first and last, one wave per bin).
+// One block (a grid has at most 8192 rows).
+constexpr int kDiffRowT = 1024;
+__global__ __launch_bounds__(kDiffRowT) void k_diff_rows(DiffArgs a) {
+  extern __shared__ int s_rows[];  // [nd][2] first / last row, then [G] tap indices
+  int *s_d = s_rows, *s_m = s_rows + 2 * a.nd;
+  for (int e = threadIdx.x; e < a.nd; e += blockDim.x) {
+    s_d[2 * e] = a.grid;
+    s_d[2 * e + 1] = -1;
+  }
+  __syncthreads();
+  const double vsini = a.prm ? a.prm[0] : a.vsini;
+  for (int iy = threadIdx.x; iy < a.grid; iy += blockDim.x) {
+#pragma clang fp contract(off)
+    const double y = -1. + iy * (2. / a.grid);
+    const double delta = vsini * y;
+    const double beta = delta * 1000. / kC;
+    const double g = sqrt((1 + beta) / (1 - beta));
+    const double fbeta = -1 * (1 - g);
+    const double sh = log1p(fbeta) / a.h;
+    const double mc = ceil(sh);
+    a.row_m[iy] = (int32_t)mc;
+    // dt/d(delta) = -exp((m-s)h)/expm1(h) / (g^2 (1-beta)^2) * 1000/c (m piecewise constant)
+    a.row_t[iy] = make_double2(expm1((mc - sh) * a.h) / a.expm1_h,
+                               -exp((mc - sh) * a.h) / a.expm1_h / (g * g * (1 - beta) * (1 - beta)) * (1000. / kC) * y);
+    const int d0 = (int32_t)mc - a.dmin;  // tap index of offset m; m-1 at d0-1
+    const bool in = d0 >= 1 && d0 < a.nd;  // the host bounds every shift
+    s_m[iy] = in ? d0 : -1;
+    if (in) {
+      atomicMin(s_d + 2 * d0, iy);
+      atomicMax(s_d + 2 * d0 + 1, iy);
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < 2 * a.nd; e += blockDim.x) a.drow[e] = s_d[e];
   const int lane = threadIdx.x & 63;
-  // every lane of a wave runs every iteration (the shuffles need the whole wave)
-  for (long base = c0; base < c1; base += blockDim.x) {
-    long idx = base + threadIdx.x;
-    int key = -1, k = -1, d0 = 0;
-    double w[NS], t = 0.0;
-#pragma unroll
-    for (int q = 0; q < NS; q++) w[q] = 0.0;
-    if (idx < c1) k = a.ck[idx];
-    if (k >= 0) {
-      d0 = a.cm[idx] - a.dmin;  // tap index of offset m; m-1 at d0-1
-      if (d0 >= 1 && d0 < a.nd) {  // the host bounds every shift
-        double y, z, fy, fz;
-        int i0, j0;
-        cell_yz(idx, a.grid, y, z);
-        double phi = map_sample(mp, a.map_res, y, z, i0, j0, fy, fz);
-        double psi = NS == 3 ? map_sample(fp, a.map_res, y, z, i0, j0, fy, fz) : 0.0;
-        double L = a.cL[idx];
-        t = a.ct[idx];
-        w[0] = L * (1 - phi - psi);
-        w[1] = kappa * L * phi;
-        if (NS == 3) w[NS - 1] = kappa_f * lb_factor(a, a.cmu[idx]) * L * psi;
-        key = (int)(idx / a.grid) * 1024 + k;  // (row, bin): rows share (m, t); k < 1024
-      }
+  for (int k = threadIdx.x >> 6; k < a.n_mu; k += kDiffRowT / 64) {
+    int lo = a.nd, hi = -1;
+    for (int iy = a.brow[2 * k] + lane; iy <= a.brow[2 * k + 1]; iy += 64) {
+      const int d0 = s_m[iy];
+      if (d0 < 0) continue;
+      lo = min(lo, d0 - 1);
+      hi = max(hi, d0);
     }
-    const int kprev = __shfl_up(key, 1), knext = __shfl_down(key, 1);
-    bool f = lane == 0 || kprev != key;  // run head
-    const bool tail = lane == 63 || knext != key;
-    for (int off = 1; off < 64; off <<= 1) {  // inclusive segmented scan of the weights
-      double x[NS];
 #pragma unroll
-      for (int q = 0; q < NS; q++) x[q] = __shfl_up(w[q], off);
-      int fo = __shfl_up((int)f, off);
-      if (lane >= off && !f) {
-#pragma unroll
-        for (int q = 0; q < NS; q++) w[q] += x[q];
-        f = fo != 0;
-      }
+    for (int off = 32; off > 0; off >>= 1) {
+      lo = min(lo, __shfl_xor(lo, off));
+      hi = max(hi, __shfl_xor(hi, off));
     }
-    if (tail && key >= 0) {
-      unsigned long long *row = dst + (long)k * a.nd * NS * 2;
-#pragma unroll
-      for (int q = 0; q < NS; q++) {
-        fx_add(row + ((long)d0 * NS + q) * 2, w[q] * (1.0 - t));
-        fx_add(row + ((long)(d0 - 1) * NS + q) * 2, w[q] * t);
-      }
-    }
-  }
-  if (use_lds) {
-    __syncthreads();
-    for (long e = threadIdx.x; e < nacc; e += blockDim.x) {
-      unsigned long long v = lacc[e];
-      if (v) atomicAdd(gacc + e, v);
+    if (lane == 0) {
+      a.blag[2 * k] = lo;
+      a.blag[2 * k + 1] = hi;
     }
   }
 }
 
-// fixed point -> taps [p][k][d][ns] and the nonzero range per (p, k).  One thread per
-// (bin, offset) of a phase; the ranges are formed in LDS (one thread per bin walked its
-// offsets in turn before: 15-86 us against 3-6 us).
-__global__ __launch_bounds__(kDT) void k_diff_taps_finalize(DiffArgs a) {
-  extern __shared__ int s_rg[];  // [n_mu][2]: lo, hi
-  const int p = blockIdx.x, ns = a.ns, nd = a.nd, n_mu = a.n_mu;
-  for (int k = threadIdx.x; k < n_mu; k += blockDim.x) {
-    s_rg[2 * k] = nd;
-    s_rg[2 * k + 1] = -1;
-  }
-  __syncthreads();
-  const long base = (long)p * n_mu * nd;
-  for (int e = threadIdx.x; e < n_mu * nd; e += blockDim.x) {
-    const int k = e / nd, d = e - k * nd;
-    const unsigned long long *in = a.acc + (base + e) * ns * 2;
-    double *o = a.taps + (base + e) * ns;
-    bool nz = false;
-    for (int q = 0; q < ns; q++) {
-      const double v = fx_value(in[q * 2], in[q * 2 + 1]);
-      o[q] = v;
-      nz |= v != 0.0;
+// LDS written by some lanes of a wave and read by others: the LDS serves a wave's
+// accesses in order, so only the compiler has to be held
+__device__ __forceinline__ void wave_lds_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Moments of one piece for up to 64 phases: one wave per (piece, 64 phases).  The wave
+// samples its cells' filling factors bilinearly (two phases x 32 cells per step, loads
+// of neighbouring cells from neighbouring nodes) into LDS and then sums them with lanes
+// over phases, the cell's own factors read from the lane that holds them.  Blocks are in
+// contiguous runs per XCD: neighbouring pieces read the same map rows.  Outputs: mom rows
+// 0-2 sum a^q phi, 3-5 sum a^q psi, 6-8 sum a^q b psi, and the sets' tap weights
+// sum L (1 - phi - psi), kappa sum L phi, kappa_f sum L b psi.
+constexpr int kMomW = 4;       // waves (pieces) per block
+constexpr int kMomU = 4;       // sampling steps in flight
+constexpr int kMomStride = kDiffPiece + 1;
+template <int NS>
+__global__ __launch_bounds__(64 * kMomW) void k_diff_moments(DiffArgs a, int blocks_per_xcd) {
+  extern __shared__ double s_mom[];  // per wave [phases][kMomStride]
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int blk = (blockIdx.x & 7) * blocks_per_xcd + (blockIdx.x >> 3);
+  const int ip = __builtin_amdgcn_readfirstlane(blk * kMomW + w);
+  const int p0 = blockIdx.y * 64, np = min(64, a.n_phase - p0), P = a.n_phase;
+  if (ip >= a.n_piece) return;  // no barriers below
+  double *sp = s_mom + (size_t)w * min(64, P) * kMomStride;
+  const CONSTANT int32_t *pi = gc((const int32_t *)(a.piece + ip));
+  const DiffPiece pc = {pi[0], pi[1], pi[2], pi[3]};
+  const int M = a.map_res;
+  const long MM = (long)M * M;
+  // this lane's cell and its stencil (the same for every phase)
+  const int c = lane & 31, ph = lane >> 5;
+  const int cc = min(c, pc.len - 1);
+  const double2 me = a.cell[(long)pc.iy * a.grid + pc.iz0 + cc];
+  const int j0 = a.map_j[pc.iz0 + cc], i0 = gc(a.map_j)[pc.iy];
+  const double fz = a.map_f[pc.iz0 + cc], fy = gc(a.map_f)[pc.iy];
+  const double w00 = (1 - fy) * (1 - fz), w10 = fy * (1 - fz), w01 = (1 - fy) * fz, w11 = fy * fz;
+  const long off = (long)i0 * M + j0;
+  double m[9];
+#pragma unroll
+  for (int q = 0; q < 9; q++) m[q] = 0.0;
+#pragma unroll
+  for (int set = 0; set < NS - 1; set++) {
+    const double *mp = (set ? a.fmaps : a.maps) + (long)p0 * MM + off;
+    for (int s = 0; s < np; s += 2 * kMomU) {
+      double x[kMomU][4];
+#pragma unroll
+      for (int u = 0; u < kMomU; u++) {
+        const double *q = mp + (long)min(s + 2 * u + ph, np - 1) * MM;
+        x[u][0] = q[0];
+        x[u][1] = q[M];
+        x[u][2] = q[1];
+        x[u][3] = q[M + 1];
+      }
+#pragma unroll
+      for (int u = 0; u < kMomU; u++) {
+        const int p = s + 2 * u + ph;
+        if (p < np) sp[p * kMomStride + c] = w00 * x[u][0] + w10 * x[u][1] + w01 * x[u][2] + w11 * x[u][3];
+      }
     }
-    if (nz) {
-      atomicMin(s_rg + 2 * k, d);
-      atomicMax(s_rg + 2 * k + 1, d);
+    wave_lds_order();
+    const double *mine = sp + min(lane, np - 1) * kMomStride;
+#pragma unroll 4
+    for (int i = 0; i < pc.len; i++) {
+      const double f = mine[i], ca = lane_f64(me.x, i);
+      const double fa = f * ca;
+      m[3 * set] += f;
+      m[3 * set + 1] += fa;
+      m[3 * set + 2] = fma(fa, ca, m[3 * set + 2]);
+      if (set) {
+        const double g = f * lane_f64(me.y, i), ga = g * ca;
+        m[6] += g;
+        m[7] += ga;
+        m[8] = fma(ga, ca, m[8]);
+      }
+    }
+    wave_lds_order();
+  }
+  if (lane >= np) return;
+  constexpr int NM = diff_moments(NS);
+  double *o = a.mom + (long)ip * NM * P + p0 + lane;
+#pragma unroll
+  for (int q = 0; q < NM; q++) o[(long)q * P] = m[q];
+  const double u1 = a.prm ? a.prm[1] : a.u1, u2 = a.prm ? a.prm[2] : a.u2;
+  const double kappa = a.prm ? a.prm[3] : a.kappa, kappa_f = a.prm ? a.prm[4] : a.kappa_f;
+  const double s1 = gc((const double *)(a.psum + ip))[0], s2 = gc((const double *)(a.psum + ip))[1];
+  double *wt = a.wts + (long)ip * NS * P + p0 + lane;
+  const double Lphi = m[0] - u1 * m[1] - u2 * m[2];
+  wt[0] = ((double)pc.len - m[0] - m[3]) - u1 * (s1 - m[1] - m[4]) - u2 * (s2 - m[2] - m[5]);
+  wt[P] = kappa * Lphi;
+  if (NS == 3) wt[2L * P] = kappa_f * (m[6] - u1 * m[7] - u2 * m[8]);
+}
+
+// taps[p][k][d][q] = sum over the pieces of bin k whose row has tap index d of w (1 - t),
+// and of those with index d + 1 of w t.  Block = (d, k), lanes over phases, the piece
+// range split over kTapW waves whose sums are added in wave order; the lanes first load
+// the factors of 64 pieces, which are then read from them one by one, so the weight
+// loads do not wait on a chain of look-ups.
+constexpr int kTapW = 8;
+template <int NS>
+__global__ __launch_bounds__(64 * kTapW) void k_diff_taps(DiffArgs a) {
+  __shared__ double s_t[kTapW][NS][64];
+  const int d = blockIdx.x, k = blockIdx.y, P = a.n_phase;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int p = blockIdx.z * 64 + lane, pl = min(p, P - 1);
+  const CONSTANT int32_t *ps = gc(a.pstart) + (long)k * (a.grid + 1);
+  double acc[NS];
+#pragma unroll
+  for (int q = 0; q < NS; q++) acc[q] = 0.0;
+  for (int side = 0; side < 2; side++) {
+    const int dd = d + side;
+    if (dd < 1 || dd >= a.nd) continue;
+    const int r0 = gc(a.drow)[2 * dd], r1 = gc(a.drow)[2 * dd + 1];
+    if (r0 > r1) continue;
+    const int i0 = ps[r0], cnt = ps[r1 + 1] - i0;
+    const int q0 = i0 + (int)((long)cnt * w / kTapW), q1 = i0 + (int)((long)cnt * (w + 1) / kTapW);
+    for (int b = q0; b < q1; b += 64) {
+      const int iy = a.piece[min(b + lane, q1 - 1)].iy;
+      const double t = a.row_t[iy].x;
+      const double f = a.row_m[iy] - a.dmin == dd ? (side ? t : 1.0 - t) : 0.0;
+      const double *wt = a.wts + (long)b * NS * P + pl;
+      const int m = min(64, q1 - b);
+#pragma unroll 8
+      for (int i = 0; i < m; i++) {
+        const double fi = lane_f64(f, i);
+#pragma unroll
+        for (int q = 0; q < NS; q++) acc[q] = fma(wt[((long)i * NS + q) * P], fi, acc[q]);
+      }
     }
   }
+#pragma unroll
+  for (int q = 0; q < NS; q++) s_t[w][q][lane] = acc[q];
   __syncthreads();
-  for (int e = threadIdx.x; e < 2 * n_mu; e += blockDim.x) a.krange[(long)p * n_mu * 2 + e] = s_rg[e];
+  if (w == 0 && p < P) {
+    double *o = a.taps + (((long)p * a.n_mu + k) * a.nd + d) * NS;
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+      double x = s_t[0][q][lane];
+#pragma unroll
+      for (int i = 1; i < kTapW; i++) x += s_t[i][q][lane];
+      o[q] = x;
+    }
+  }
 }
 
 // I_p[j] = sum_k sum_d HQ[d] Q_k[j - dmin - d] + HS[d] S_k[j - dmin - d] (+ HF[d] Fa_k[j - dmin - d]);
@@ -212,7 +287,7 @@ __global__ __launch_bounds__(kDT) void k_diff_fir(DiffArgs a) {
   long src0 = j0 - a.dmin - nd + 1;
   double acc = 0.0;
   for (int k = 0; k < a.n_mu; k++) {
-    int lo = a.krange[((long)p * a.n_mu + k) * 2], hi = a.krange[((long)p * a.n_mu + k) * 2 + 1];
+    int lo = a.blag[2 * k], hi = a.blag[2 * k + 1];
     if (lo > hi) continue;  // uniform
     __syncthreads();
     for (int e = threadIdx.x; e < row_len; e += blockDim.x) {
@@ -712,7 +787,7 @@ __global__ __launch_bounds__(kDT) void k_diff_convT(DiffArgs a, ConvArgs c, cons
   }
 }
 
-// lag correlations C[p][k][d][set] = sum_j G_I[p][j] X_k[j - dmin - d], in two
+// lag correlations C[k][d][set][p] = sum_j G_I[p][j] X_k[j - dmin - d], in two
 // passes.  Pass 1: block = (chunk of kCorrT pixels, bin k, group of kCorrPG
 // phases); the bin's two seed-row segments are staged once for the group.  Each
 // thread owns kCorrPer consecutive pixels (G_I of the phase in registers) and,
@@ -724,22 +799,6 @@ constexpr int kCorrPer = 9;  // odd: a thread stride of kCorrPer doubles is free
 constexpr int kCorrT = kDT * kCorrPer;
 constexpr int kCorrL = 8;
 constexpr int kCorrPG = 10;
-// Lags the cells can use: a cell's shift index d0 (k_diff_cells: m = ceil(log1p(fb)/h),
-// fb monotone in delta = vsini y, |y| <= 1) lies in [m(-vsini), m(vsini)] - dmin, and the
-// per-cell derivatives read lags d0 and d0 - 1; two lags of margin on each side.
-// Lags outside need no correlation (the tap range fixed by a bound on vsini can be
-// much wider than the current vsini needs).
-__device__ __forceinline__ void diff_lag_range(const DiffArgs &a, int &lo, int &hi) {
-  const double vs = a.prm ? a.prm[0] : a.vsini;
-  auto m = [&](double v) {
-    double beta = v * 1000. / kC;
-    double fb = -1 * (1 - sqrt((1 + beta) / (1 - beta)));
-    return (int)ceil(log1p(fb) / a.h);
-  };
-  lo = max(0, m(-vs) - a.dmin - 3);
-  hi = min(a.nd - 1, m(vs) - a.dmin + 2);
-}
-
 // One pass covers nsp <= 2 seed cubes (x0, x1), written to sets soff, soff + 1 of
 // the ns-set tables; the facula set, when present, is a second pass (three staged
 // rows would not fit the LDS budget).
@@ -767,8 +826,7 @@ __global__ __launch_bounds__(kDT) void k_diff_corr(DiffArgs a, const double *GI,
       g[u] = j < a.n ? GI[(long)p * a.n + j] : 0.0;
     }
     double *out = Cpart + (((long)p * a.n_mu + k) * nchunk + chunk) * nd * ns;
-    int dlo, dhi;
-    diff_lag_range(a, dlo, dhi);  // uniform
+    const int dlo = a.blag[2 * k], dhi = a.blag[2 * k + 1];  // the lags this bin's cells use
     for (int set = 0; set < nsp; set++) {
       const double *row = (set ? rs : rq) + threadIdx.x * kCorrPer;
       for (int d0 = dlo; d0 <= dhi; d0 += kCorrL) {
@@ -808,134 +866,167 @@ __global__ void k_diff_corr_reduce(DiffArgs a, int n_pk, int nd, int nchunk, con
   long e = (long)blockIdx.x * blockDim.x + threadIdx.x;  // (p, k) x (d, set)
   if (e >= (long)n_pk * nd * ns) return;
   long pk = e / (nd * ns), r = e % (nd * ns);
-  int dlo, dhi;
-  diff_lag_range(a, dlo, dhi);
-  const int d = (int)(r / ns);
+  const int d = (int)(r / ns), p = (int)(pk / a.n_mu), k = (int)(pk % a.n_mu);
   double x = 0.0;
-  if (d >= dlo && d <= dhi)  // k_diff_corr computes only these lags
+  if (d >= a.blag[2 * k] && d <= a.blag[2 * k + 1])  // k_diff_corr computes only these lags
     for (int c = 0; c < nchunk; c++) x += Cpart[(pk * nchunk + c) * nd * ns + r];
-  C[e] = x;
+  C[((long)k * nd * ns + r) * a.n_phase + p] = x;
 }
 
 int diff_corr_chunks(int64_t n) { return (int)((n + kCorrT - 1) / kCorrT); }
 
-// per-cell derivatives from the correlations, phases summed per cell; scalar
-// partials per block: [gvsini, gu1, gu2, gkappa, gkappa_f]
-__global__ __launch_bounds__(kDT) void k_diff_cellgrad(DiffArgs a, const double *C, double *part) {
-  const double kappa = a.prm ? a.prm[3] : a.kappa;
-  const double kappa_f = a.prm ? a.prm[4] : a.kappa_f;
-  const int ns = a.ns;
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long ncell = (long)a.grid * a.grid;
-  double sv = 0, su1 = 0, su2 = 0, sk = 0, sf = 0;
-  if (idx < ncell && a.ck[idx] >= 0) {
-    int k = a.ck[idx];
-    int d0 = a.cm[idx] - a.dmin;
-    if (d0 >= 1 && d0 < a.nd) {
-      double y, z;
-      cell_yz(idx, a.grid, y, z);
-      double L = a.cL[idx], t = a.ct[idx], mu = a.cmu[idx];
-      const double lbf = ns == 3 ? lb_factor(a, mu) : 0.0;
-      double gL = 0, gt = 0;
-      int M = a.map_res;
-      for (int p = 0; p < a.n_phase; p++) {
-        const double *Cp = C + (((long)p * a.n_mu + k) * a.nd) * ns;
-        double cq0 = Cp[d0 * ns], cq1 = Cp[(d0 - 1) * ns], cs0 = Cp[d0 * ns + 1], cs1 = Cp[(d0 - 1) * ns + 1];
-        double aq = (1 - t) * cq0 + t * cq1, as = (1 - t) * cs0 + t * cs1;
-        double bq = cq1 - cq0, bs = cs1 - cs0;
-        int i0, j0;
-        double fy, fz;
-        double phi = map_sample(a.maps + (long)p * M * M, M, y, z, i0, j0, fy, fz);
-        if (ns == 3) {
-          double cf0 = Cp[d0 * ns + 2], cf1 = Cp[(d0 - 1) * ns + 2];
-          double af = (1 - t) * cf0 + t * cf1, bf = cf1 - cf0;
-          double psi = map_sample(a.fmaps + (long)p * M * M, M, y, z, i0, j0, fy, fz);
-          double ef = kappa_f * lbf * psi;
-          gL += (1 - phi - psi) * aq + kappa * phi * as + ef * af;
-          gt += L * ((1 - phi - psi) * bq + kappa * phi * bs + ef * bf);
-          sf += L * lbf * psi * af;
-        } else {
-          gL += (1 - phi) * aq + kappa * phi * as;
-          gt += L * ((1 - phi) * bq + kappa * phi * bs);
+// a_X = (1 - t) C[d0] + t C[d0 - 1] of the bin and phase (C [k][d][set][P])
+__device__ __forceinline__ double corr_at(const double *Cd, int ns, int P, int set, double t, double &diff) {
+  const double c0 = Cd[(long)set * P], c1 = Cd[(long)(set - ns) * P];
+  diff = c1 - c0;
+  return (1 - t) * c0 + t * c1;
+}
+
+// scalar gradients from the correlations and the moments: one wave per piece, lanes over
+// phases; partials per block: [gvsini, gu1, gu2, gkappa, gkappa_f]
+__global__ __launch_bounds__(256) void k_diff_piecegrad(DiffArgs a, const double *C, double *part) {
+  __shared__ double s_p[4][kDiffScalars];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, P = a.n_phase, ns = a.ns;
+  const int ip = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + w);
+  double v[16];
+#pragma unroll
+  for (int q = 0; q < 16; q++) v[q] = 0.0;
+  if (ip < a.n_piece) {
+    const CONSTANT int32_t *pc = gc((const int32_t *)(a.piece + ip));
+    const int iy = pc[0], len = pc[2], k = pc[3];
+    const double kappa = a.prm ? a.prm[3] : a.kappa, kappa_f = a.prm ? a.prm[4] : a.kappa_f;
+    const double u1 = a.prm ? a.prm[1] : a.u1, u2 = a.prm ? a.prm[2] : a.u2;
+    const double t = gc((const double *)(a.row_t + iy))[0], dt = gc((const double *)(a.row_t + iy))[1];
+    const int d0 = gc(a.row_m)[iy] - a.dmin, nm = diff_moments(ns);
+    const double s[3] = {(double)len, gc((const double *)(a.psum + ip))[0], gc((const double *)(a.psum + ip))[1]};
+    if (d0 >= 1 && d0 < a.nd)
+      for (int p = lane; p < P; p += 64) {
+        const double *Cd = C + ((long)k * a.nd + d0) * ns * P + p;
+        const double *mo = a.mom + (long)ip * nm * P + p;
+        double bq, bs, bf = 0.0;
+        const double aq = corr_at(Cd, ns, P, 0, t, bq), as = corr_at(Cd, ns, P, 1, t, bs);
+        const double af = ns == 3 ? corr_at(Cd, ns, P, 2, t, bf) : 0.0;
+        double quiet[3], spot[3], fac[3];  // sums of a^q (1 - phi - psi), a^q phi, a^q b psi
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+          spot[q] = mo[(long)q * P];
+          quiet[q] = s[q] - spot[q] - (ns == 3 ? mo[(long)(q + 3) * P] : 0.0);
+          fac[q] = ns == 3 ? mo[(long)(q + 6) * P] : 0.0;
         }
-        sk += L * phi * as;
+        auto limb = [&](const double (&x)[3]) { return x[0] - u1 * x[1] - u2 * x[2]; };
+        v[0] += dt * (limb(quiet) * bq + kappa * limb(spot) * bs + kappa_f * limb(fac) * bf);
+        v[1] -= quiet[1] * aq + kappa * spot[1] * as + kappa_f * fac[1] * af;
+        v[2] -= quiet[2] * aq + kappa * spot[2] * as + kappa_f * fac[2] * af;
+        v[3] += limb(spot) * as;
+        v[4] += limb(fac) * af;
       }
-      su1 = -gL * (1 - mu);
-      su2 = -gL * (1 - mu) * (1 - mu);
-      sv = gt * a.cdt[idx];  // dt/d(delta) * d(delta)/d(vsini)
-    }
   }
-  __shared__ double s_p[kDiffScalars][kDT / 64];
-  double v5[kDiffScalars] = {sv, su1, su2, sk, sf};
-  for (int q = 0; q < kDiffScalars; q++) {
-    double x = v5[q];
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-    if ((threadIdx.x & 63) == 0) s_p[q][threadIdx.x >> 6] = x;
-  }
+  wave_sums16(v);
+  if (lane == 0)
+#pragma unroll
+    for (int q = 0; q < kDiffScalars; q++) s_p[w][q] = v[q];
   __syncthreads();
   if (threadIdx.x < kDiffScalars) {
-    double s = 0;
-    for (int w = 0; w < kDT / 64; w++) s += s_p[threadIdx.x][w];
-    part[(long)blockIdx.x * kDiffScalars + threadIdx.x] = s;
+    double x = 0;
+    for (int i = 0; i < 4; i++) x += s_p[i][threadIdx.x];
+    part[(long)blockIdx.x * kDiffScalars + threadIdx.x] = x;
   }
 }
 
-// map-pixel gradients as a gather (no atomics): node (i, j) of phase p sums, over
-// the cells whose bilinear stencil in map_sample holds it, weight x L (kappa a_S -
-// a_Q) for the spot map and weight x L (kappa_f (1 + LB) a_F - a_Q) for the facula
-// map, with a_Q, a_S, a_F the cell's interpolated correlations.  A cell at map
-// coordinate gy = iy (M - 1) / G touches nodes floor(gy) and floor(gy) + 1, so
-// node i looks at the rows with floor(gy) in {i - 1, i} (a superset is scanned
-// and filtered with the same arithmetic as map_sample).
-__global__ __launch_bounds__(kDT) void k_diff_mapgrad(DiffArgs a, const double *C, double *gmaps, double *gfmaps) {
-#pragma clang fp contract(off)
-  const double kappa = a.prm ? a.prm[3] : a.kappa;
-  const double kappa_f = a.prm ? a.prm[4] : a.kappa_f;
-  const int ns = a.ns;
-  const int M = a.map_res, G = a.grid;
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;  // map column
-  const int i = blockIdx.y;                              // map row
-  const int p = blockIdx.z;
-  if (j >= M) return;
-  const double sc = (double)G / (M - 1), dg = 2. / G;
+// map-pixel gradients: node (i, j) of phase p sums, over the cells whose bilinear stencil
+// holds it, weight x L (kappa a_S - a_Q) for the spot map and weight x L (kappa_f (1 + LB)
+// a_F - a_Q) for the facula map.  One wave per (node row, 16 nodes, 64 phases), lanes over
+// phases: the wave walks the cells of the disk rows that touch its node row, the
+// correlation factors change only with the bin, and a cell costs a few multiply-adds on
+// uniform weights; a node's two running sums go to LDS when the walk passes it, and the
+// 16-node rows of all phases are written from there.
+constexpr int kMgN = 16;
+constexpr int kMgStride = kMgN + 1;
+template <int NS>
+__global__ __launch_bounds__(256) void k_diff_mapgrad(DiffArgs a, const double *C, double *gmaps, double *gfmaps) {
+  extern __shared__ double s_mg[];  // per wave [NS - 1][phases][kMgStride]
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int M = a.map_res, G = a.grid, P = a.n_phase;
+  const int jb = (blockIdx.x * 4 + w) * kMgN, i = blockIdx.y;
+  const int p0 = blockIdx.z * 64, np = min(64, P - p0), ps = min(64, P);
+  if (jb >= M) return;  // no barriers below
+  double *tile = s_mg + (size_t)w * (NS - 1) * ps * kMgStride;
+  for (int e = lane; e < (NS - 1) * ps * kMgStride; e += 64) tile[e] = 0.0;
+  wave_lds_order();
+  const double kappa = a.prm ? a.prm[3] : a.kappa, kappa_f = a.prm ? a.prm[4] : a.kappa_f;
+  const double u1 = a.prm ? a.prm[1] : a.u1, u2 = a.prm ? a.prm[2] : a.u2;
+  const int pl = min(lane, np - 1);
+  double *mine = tile + pl * kMgStride;
+  auto put = [&](int j, double s, double f) {
+    if (j < jb || j >= jb + kMgN || lane >= np) return;
+    __hip_atomic_fetch_add(mine + (j - jb), s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    if (NS == 3)
+      __hip_atomic_fetch_add(mine + ps * kMgStride + (j - jb), f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  };
+  // cells whose stencil can reach the nodes: a superset, filtered by the plan's own nodes
+  const double sc = (double)G / (M - 1);
   const int y_lo = max(0, (int)floor((i - 1) * sc) - 1), y_hi = min(G - 1, (int)ceil((i + 1) * sc) + 1);
-  const int z_lo = max(0, (int)floor((j - 1) * sc) - 1), z_hi = min(G - 1, (int)ceil((j + 1) * sc) + 1);
-  double acc = 0.0, accf = 0.0;
+  const int z_lo = max(0, (int)floor((jb - 1) * sc) - 1), z_hi = min(G - 1, (int)ceil((jb + kMgN) * sc) + 1);
   for (int iy = y_lo; iy <= y_hi; iy++) {
-    // the row half of map_sample: gy, its clamped floor and fraction
-    double y = -1. + iy * dg;
-    double gy = (y + 1) * 0.5 * (M - 1);
-    int i0 = (int)floor(gy);
-    i0 = i0 > M - 2 ? M - 2 : (i0 < 0 ? 0 : i0);
+    const int i0 = gc(a.map_j)[iy];
     if (i0 != i && i0 + 1 != i) continue;
-    double fy = gy - i0;
-    double wy = i0 == i ? 1 - fy : fy;
-    for (int iz = z_lo; iz <= z_hi; iz++) {
-      double z = -1. + iz * dg;
-      double gz = (z + 1) * 0.5 * (M - 1);
-      int j0 = (int)floor(gz);
-      j0 = j0 > M - 2 ? M - 2 : (j0 < 0 ? 0 : j0);
-      if (j0 != j && j0 + 1 != j) continue;
-      long idx = (long)iy * G + iz;
-      int k = a.ck[idx];
-      if (k < 0) continue;
-      int d0 = a.cm[idx] - a.dmin;
-      if (d0 < 1 || d0 >= a.nd) continue;
-      double fz = gz - j0;
-      double wz = j0 == j ? 1 - fz : fz;
-      const double *Cp = C + (((long)p * a.n_mu + k) * a.nd) * ns;
-      double t = a.ct[idx];
-      double aq = (1 - t) * Cp[d0 * ns] + t * Cp[(d0 - 1) * ns];
-      double as = (1 - t) * Cp[d0 * ns + 1] + t * Cp[(d0 - 1) * ns + 1];
-      acc += wy * wz * (a.cL[idx] * (kappa * as - aq));
-      if (ns == 3) {
-        double af = (1 - t) * Cp[d0 * ns + 2] + t * Cp[(d0 - 1) * ns + 2];
-        accf += wy * wz * (a.cL[idx] * (kappa_f * lb_factor(a, a.cmu[idx]) * af - aq));
+    const int d0 = gc(a.row_m)[iy] - a.dmin;
+    if (d0 < 1 || d0 >= a.nd) continue;
+    const double fy = gc(a.map_f)[iy], wy = i0 == i ? 1 - fy : fy, t = gc((const double *)(a.row_t + iy))[0];
+    int kcur = -1, cur = -2;
+    double e1 = 0.0, eq = 0.0, ef = 0.0, s0 = 0.0, s1 = 0.0, f0 = 0.0, f1 = 0.0;
+    for (int zb = z_lo; zb <= z_hi; zb += 64) {
+      // 64 cells of the row, one per lane: bin, first node, weights on its two nodes
+      const int iz = min(zb + lane, G - 1), jz = a.map_j[iz];
+      const long idx = (long)iy * G + iz;
+      const bool in = zb + lane <= z_hi && jz + 1 >= jb && jz < jb + kMgN;
+      const int kz = in ? a.ck[idx] : -1;
+      const double2 ce = a.cell[idx];
+      const double fz = a.map_f[iz], L = 1. - u1 * ce.x - u2 * ce.x * ce.x, wz0 = L * (1 - fz), wz1 = L * fz;
+      unsigned long long todo = __ballot(kz >= 0);
+      while (todo) {
+        const int l = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const int k = __builtin_amdgcn_readlane(kz, l), j0 = __builtin_amdgcn_readlane(jz, l);
+        if (k != kcur) {
+          kcur = k;
+          const double *Cd = C + ((long)k * a.nd + d0) * NS * P + p0 + pl;
+          double unused;
+          eq = wy * corr_at(Cd, NS, P, 0, t, unused);
+          e1 = wy * kappa * corr_at(Cd, NS, P, 1, t, unused) - eq;
+          if (NS == 3) ef = wy * kappa_f * corr_at(Cd, NS, P, NS - 1, t, unused);
+        }
+        if (j0 != cur) {
+          put(cur, s0, f0);
+          const bool next = j0 == cur + 1;
+          if (!next) put(cur + 1, s1, f1);
+          s0 = next ? s1 : 0.0;
+          f0 = next ? f1 : 0.0;
+          s1 = f1 = 0.0;
+          cur = j0;
+        }
+        const double w0 = lane_f64(wz0, l), w1 = lane_f64(wz1, l);
+        s0 = fma(w0, e1, s0);
+        s1 = fma(w1, e1, s1);
+        if (NS == 3) {
+          const double x = fma(lane_f64(ce.y, l), ef, -eq);
+          f0 = fma(w0, x, f0);
+          f1 = fma(w1, x, f1);
+        }
       }
     }
+    put(cur, s0, f0);
+    put(cur + 1, s1, f1);
   }
-  gmaps[((long)p * M + i) * M + j] = acc;
-  if (ns == 3) gfmaps[((long)p * M + i) * M + j] = accf;
+  wave_lds_order();
+  const int nj = min(kMgN, M - jb);
+  for (int e = lane; e < np * kMgN; e += 64) {
+    const int p = e / kMgN, j = e % kMgN;
+    if (j >= nj) continue;
+    const long o = ((long)(p0 + p) * M + i) * M + jb + j;
+    gmaps[o] = tile[p * kMgStride + j];
+    if (NS == 3) gfmaps[o] = tile[(ps + p) * kMgStride + j];
+  }
 }
 
 // seed gradients gX_k[i] = sum_p sum_d HX_pk[d] G_I,p[i + dmin + d]; block = (tile, bin)
@@ -950,7 +1041,7 @@ __global__ __launch_bounds__(kDT) void k_diff_seedgrad(DiffArgs a, const double 
 #pragma unroll
   for (int q = 0; q < NS; q++) ax[q] = 0.0;
   for (int p = 0; p < a.n_phase; p++) {
-    int lo = a.krange[((long)p * a.n_mu + k) * 2], hi = a.krange[((long)p * a.n_mu + k) * 2 + 1];
+    int lo = a.blag[2 * k], hi = a.blag[2 * k + 1];
     if (lo > hi) continue;  // uniform
     __syncthreads();
     for (int e = threadIdx.x; e < len; e += blockDim.x) {
@@ -976,25 +1067,25 @@ __global__ __launch_bounds__(kDT) void k_diff_seedgrad(DiffArgs a, const double 
 // ------------------------------------------------------------ launchers
 hipError_t launch_diff_forward_spectra(const DiffArgs &a, const ConvArgs &c, const double *target, int trim,
                                        double *res_part, int *res_blocks, hipStream_t s) {
-  long ncell = (long)a.grid * a.grid;
-  k_diff_cells<<<(unsigned)((ncell + kDT - 1) / kDT), kDT, 0, s>>>(a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  hipError_t e;
   if (a.ns != 2 && a.ns != 3) return hipErrorInvalidValue;
   if (a.ns == 3 && (!a.f || !a.fmaps)) return hipErrorInvalidValue;
-  long nacc = (long)a.n_mu * a.nd * a.ns * 2;
-  e = launch_fill_u64(a.acc, (size_t)a.n_phase * nacc, s);
-  if (e != hipSuccess) return e;
-  int use_lds = nacc * 8 <= 49152;
-  int cpb = 4096;
-  dim3 gt((unsigned)((ncell + cpb - 1) / cpb), a.n_phase);
-  if (a.ns == 3)
-    k_diff_taps<3><<<gt, kDT, use_lds ? nacc * 8 : 0, s>>>(a, cpb, use_lds);
-  else
-    k_diff_taps<2><<<gt, kDT, use_lds ? nacc * 8 : 0, s>>>(a, cpb, use_lds);
+  k_diff_rows<<<1, kDiffRowT, (size_t)(2 * a.nd + a.grid) * sizeof(int), s>>>(a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((size_t)a.n_mu * 8 > 65536) return hipErrorInvalidValue;
-  k_diff_taps_finalize<<<a.n_phase, kDT, (size_t)a.n_mu * 8, s>>>(a);
+  const unsigned pg = (a.n_phase + 63) / 64;
+  const int pw = a.n_phase < 64 ? a.n_phase : 64;
+  const unsigned mbx = (a.n_piece + 8 * kMomW - 1) / (8 * kMomW);  // blocks per XCD
+  dim3 gm(8 * mbx, pg), gt(a.nd, a.n_mu, pg);
+  const size_t lds_mom = (size_t)kMomW * pw * kMomStride * sizeof(double);  // at most 68 KB
+  if (a.ns == 3) {
+    k_diff_moments<3><<<gm, 64 * kMomW, lds_mom, s>>>(a, (int)mbx);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    k_diff_taps<3><<<gt, 64 * kTapW, 0, s>>>(a);
+  } else {
+    k_diff_moments<2><<<gm, 64 * kMomW, lds_mom, s>>>(a, (int)mbx);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    k_diff_taps<2><<<gt, 64 * kTapW, 0, s>>>(a);
+  }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   size_t lds_fir = (size_t)a.ns * (kDT + a.nd - 1) * sizeof(double);
   if (lds_fir > 65536) return hipErrorInvalidValue;
@@ -1115,7 +1206,18 @@ hipError_t launch_diff_grad(int n_blocks, const double *cell_part, double *g, hi
   k_diff_grad<<<1, kDT, 0, s>>>(n_blocks, cell_part, g);
   return hipGetLastError();
 }
-int diff_cell_blocks(int64_t ncell) { return (int)((ncell + kDT - 1) / kDT); }
+int diff_piece_blocks(int n_piece) { return (n_piece + 3) / 4; }
+
+hipError_t launch_diff_psum(const DiffArgs &a, double2 *psum, hipStream_t s) {
+  k_diff_psum<<<(a.n_piece + kDT - 1) / kDT, kDT, 0, s>>>(a, psum);
+  return hipGetLastError();
+}
+
+hipError_t launch_diff_cells(const DiffArgs &a, const double *mu_bounds, int32_t *ck, double2 *cell, hipStream_t s) {
+  const long ncell = (long)a.grid * a.grid;
+  k_diff_cells<<<(unsigned)((ncell + kDT - 1) / kDT), kDT, 0, s>>>(a, mu_bounds, ck, cell);
+  return hipGetLastError();
+}
 
 hipError_t launch_fit_polish(const double *v, int n_v, const double *ccf, const double *par, int n_ccf, double *theta,
                              hipStream_t s) {
@@ -1163,11 +1265,15 @@ hipError_t launch_diff_backward(const DiffArgs &a, const ConvArgs &c, const doub
   long nc = (long)a.n_phase * a.n_mu * a.nd * a.ns;
   k_diff_corr_reduce<<<(unsigned)((nc + kDT - 1) / kDT), kDT, 0, s>>>(a, a.n_phase * a.n_mu, a.nd, nchunk, Cpart, C);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  long ncell = (long)a.grid * a.grid;
-  k_diff_cellgrad<<<(unsigned)((ncell + kDT - 1) / kDT), kDT, 0, s>>>(a, C, cell_part);
+  k_diff_piecegrad<<<diff_piece_blocks(a.n_piece), 256, 0, s>>>(a, C, cell_part);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  dim3 gmg((unsigned)((a.map_res + kDT - 1) / kDT), a.map_res, a.n_phase);
-  k_diff_mapgrad<<<gmg, kDT, 0, s>>>(a, C, gmaps, gfmaps);
+  const int pw = a.n_phase < 64 ? a.n_phase : 64;
+  dim3 gmg((a.map_res + 4 * kMgN - 1) / (4 * kMgN), a.map_res, (a.n_phase + 63) / 64);
+  const size_t lds_mg = (size_t)4 * (a.ns - 1) * pw * kMgStride * sizeof(double);  // at most 70 KB
+  if (a.ns == 3)
+    k_diff_mapgrad<3><<<gmg, 256, lds_mg, s>>>(a, C, gmaps, gfmaps);
+  else
+    k_diff_mapgrad<2><<<gmg, 256, lds_mg, s>>>(a, C, gmaps, gfmaps);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   size_t lds_seed = (size_t)(kDT + a.nd - 1) * sizeof(double);
   dim3 gsd((unsigned)((a.n + kDT - 1) / kDT), a.n_mu);

@@ -101,7 +101,12 @@ struct soap_ctx {
     double lb[4] = {0, 0, 0, 0};  // facula intensity polynomial, constant term first
     int ns = 2;                   // tap sets of the last forward: 2, or 3 with the facula population
     const double *q = nullptr, *s = nullptr, *f = nullptr, *maps = nullptr, *fmaps = nullptr, *target = nullptr;
-    DevBuf ck, cm, ct, cL, cmu, cdt, acc, taps, krange, I, F, res_part, ccf, par, model, depth, bis, iters, th,
+    // the disk's plan and what it was built for (diff_plan)
+    DevBuf ck, cell, map_j, map_f, piece, psum, pstart, brow;
+    int n_piece = 0, plan_G = 0, plan_M = 0;
+    std::vector<double> plan_mu;
+    double plan_lb[4] = {0, 0, 0, 0};
+    DevBuf row_m, row_t, drow, blag, mom, wts, taps, I, F, res_part, ccf, par, model, depth, bis, iters, th,
         dth, gy, GF, GI, C, Cpart, cell_part;
     DevBuf bisd;  // [P][n_v + kBisHead]: span, loss coefficient, dspan/dtheta, dspan/dy
     DevBuf tg;    // per-call targets [3][P] (RV, FWHM, BIS span), the loss [1], the scalar gradients [5]
@@ -2063,6 +2068,100 @@ int soap_fit_ccf_host_noalloc(soap_ctx *c, const double *v, int32_t n_v, const d
   return SOAP_OK;
 }
 
+// The disk's plan: per-cell tables, the map stencil of every grid row or column, and the
+// pieces (runs of cells of one bin along a row) sorted by bin and row.  It depends on the
+// grid, the bins, the map size and LB only; built by diff_setup, and again by the next
+// forward, bind or step when the bins were set anew.
+static bool diff_plan_current(const soap_ctx *c) {
+  const auto &d = c->diff;
+  return d.n_piece > 0 && d.plan_G == d.G && d.plan_M == d.M && d.plan_mu == c->mu_bounds &&
+         std::equal(d.lb, d.lb + 4, d.plan_lb);
+}
+
+static int diff_plan(soap_ctx *c) {
+  auto &d = c->diff;
+  if (diff_plan_current(c)) return SOAP_OK;
+  const int G = d.G, M = d.M, n_mu = c->n_mu;
+  const size_t g2 = (size_t)G * G;
+  int rc;
+  d.n_piece = 0;
+  if ((rc = ensure(c, d.ck, g2 * 4)) || (rc = ensure(c, d.cell, g2 * 16)) || (rc = ensure(c, d.map_j, (size_t)G * 4)) ||
+      (rc = ensure(c, d.map_f, (size_t)G * 8)) || (rc = ensure(c, d.row_m, (size_t)G * 4)) ||
+      (rc = ensure(c, d.row_t, (size_t)G * 16)) || (rc = ensure(c, d.pstart, (size_t)n_mu * (G + 1) * 4)) ||
+      (rc = ensure(c, d.brow, (size_t)n_mu * 2 * 4)))
+    return rc;
+  DiffArgs a{};
+  a.grid = G;
+  a.n_mu = n_mu;
+  for (int q = 0; q < 4; q++) a.lb[q] = d.lb[q];
+  HIPCHK(c, launch_diff_cells(a, c->d_mub, (int32_t *)d.ck.p, (double2 *)d.cell.p, c->stream));
+  std::vector<int32_t> ck(g2), map_j(G), pstart((size_t)n_mu * (G + 1));
+  std::vector<double> map_f(G);
+  HIPCHK(c, hipMemcpyAsync(ck.data(), d.ck.p, g2 * 4, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  for (int i = 0; i < G; i++) {
+    const double y = -1. + i * (2. / G), g = (y + 1) * 0.5 * (M - 1);
+    const int j = std::min(std::max((int)floor(g), 0), M - 2);
+    map_j[i] = j;
+    map_f[i] = g - j;
+  }
+  std::vector<std::vector<DiffPiece>> by(n_mu);
+  for (int iy = 0; iy < G; iy++) {
+    for (int k = 0; k < n_mu; k++) pstart[(size_t)k * (G + 1) + iy] = (int32_t)by[k].size();
+    const int32_t *row = ck.data() + (size_t)iy * G;
+    for (int iz = 0; iz < G;) {
+      const int k = row[iz];
+      int e = iz + 1;
+      while (e < G && row[e] == k && (k < 0 || e - iz < kDiffPiece)) e++;
+      if (k >= 0) by[k].push_back({iy, iz, e - iz, k});
+      iz = e;
+    }
+  }
+  std::vector<DiffPiece> pieces;
+  std::vector<int32_t> brow;
+  for (int k = 0; k < n_mu; k++) {
+    brow.push_back(by[k].empty() ? 1 : by[k].front().iy);
+    brow.push_back(by[k].empty() ? 0 : by[k].back().iy);
+    const int32_t base = (int32_t)pieces.size();
+    for (int iy = 0; iy < G; iy++) pstart[(size_t)k * (G + 1) + iy] += base;
+    pieces.insert(pieces.end(), by[k].begin(), by[k].end());
+    pstart[(size_t)k * (G + 1) + G] = (int32_t)pieces.size();
+  }
+  if (pieces.empty()) return fail(c, SOAP_ERR_ARG, "diff: no cell of a %d grid on the disk", G);
+  if ((rc = ensure(c, d.piece, pieces.size() * sizeof(DiffPiece))) || (rc = ensure(c, d.psum, pieces.size() * 16)) ||
+      (rc = ensure(c, d.cell_part, (size_t)diff_piece_blocks((int)pieces.size()) * kDiffScalars * 8)))
+    return rc;
+  HIPCHK(c, hipMemcpyAsync(d.piece.p, pieces.data(), pieces.size() * sizeof(DiffPiece), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(d.pstart.p, pstart.data(), pstart.size() * 4, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(d.brow.p, brow.data(), brow.size() * 4, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(d.map_j.p, map_j.data(), (size_t)G * 4, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(d.map_f.p, map_f.data(), (size_t)G * 8, hipMemcpyHostToDevice, c->stream));
+  a.cell = (const double2 *)d.cell.p;
+  a.piece = (const DiffPiece *)d.piece.p;
+  a.n_piece = (int)pieces.size();
+  HIPCHK(c, launch_diff_psum(a, (double2 *)d.psum.p, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  d.plan_G = G;
+  d.plan_M = M;
+  d.plan_mu = c->mu_bounds;
+  for (int q = 0; q < 4; q++) d.plan_lb[q] = d.lb[q];
+  d.n_piece = (int)pieces.size();
+  return SOAP_OK;
+}
+
+// buffers of an evaluation with nd tap offsets and ns sets
+static int diff_buffers(soap_ctx *c, int nd, int ns) {
+  auto &d = c->diff;
+  const size_t per = (size_t)d.P * c->n_mu * nd * ns;
+  int rc;
+  if ((rc = ensure(c, d.drow, (size_t)nd * 2 * 4)) || (rc = ensure(c, d.blag, (size_t)c->n_mu * 2 * 4)) ||
+      (rc = ensure(c, d.mom, (size_t)d.n_piece * diff_moments(ns) * d.P * 8)) ||
+      (rc = ensure(c, d.wts, (size_t)d.n_piece * ns * d.P * 8)) || (rc = ensure(c, d.taps, per * 8)) ||
+      (rc = ensure(c, d.C, per * 8)) || (rc = ensure(c, d.Cpart, per * diff_corr_chunks(c->n) * 8)))
+    return rc;
+  return SOAP_OK;
+}
+
 // ------------------------------------------------------------------ a11: differentiable path
 int soap_diff_setup(soap_ctx *c, int32_t grid, int32_t n_phase, int32_t map_res, double sigma_ms, const double *lb) {
   if (!c || grid < 2 || grid > 8192 || n_phase < 1 || map_res < 2 || map_res > 8192 || !(sigma_ms > 0))
@@ -2074,11 +2173,8 @@ int soap_diff_setup(soap_ctx *c, int32_t grid, int32_t n_phase, int32_t map_res,
   if (c->n_mu > 1024) return fail(c, SOAP_ERR_LIMIT, "diff_setup: %d mu bins (at most 1024)", c->n_mu);
   HIPCHK(c, hipSetDevice(c->device));
   auto &d = c->diff;
-  size_t g2 = (size_t)grid * grid;
   int rc;
-  if ((rc = ensure(c, d.ck, g2 * 4)) || (rc = ensure(c, d.cm, g2 * 4)) || (rc = ensure(c, d.ct, g2 * 8)) ||
-      (rc = ensure(c, d.cL, g2 * 8)) || (rc = ensure(c, d.cmu, g2 * 8)) || (rc = ensure(c, d.cdt, g2 * 8)) ||
-      (rc = ensure(c, d.I, (size_t)n_phase * c->n * 8)) || (rc = ensure(c, d.F, (size_t)n_phase * c->n * 8)) ||
+  if ((rc = ensure(c, d.I, (size_t)n_phase * c->n * 8)) || (rc = ensure(c, d.F, (size_t)n_phase * c->n * 8)) ||
       (rc = ensure(c, d.GF, (size_t)n_phase * c->n * 8)) || (rc = ensure(c, d.GI, (size_t)n_phase * c->n * 8)) ||
       (rc = ensure(c, d.res_part, (size_t)n_phase * diff_conv_blocks(c->n) * 8)) ||
       (rc = ensure(c, d.ccf, (size_t)n_phase * c->n_v * 8)) || (rc = ensure(c, d.par, (size_t)n_phase * 5 * 8)) ||
@@ -2088,7 +2184,6 @@ int soap_diff_setup(soap_ctx *c, int32_t grid, int32_t n_phase, int32_t map_res,
       (rc = ensure(c, d.gy, (size_t)n_phase * c->n_v * 8)) ||
       (rc = ensure(c, d.bisd, (size_t)n_phase * (c->n_v + kBisHead) * 8)) ||
       (rc = ensure(c, d.tg, ((size_t)n_phase * 3 + 1 + kDiffScalars) * 8)) ||
-      (rc = ensure(c, d.cell_part, (size_t)diff_cell_blocks((int64_t)g2) * kDiffScalars * 8)) ||
       (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines) * n_phase * c->n_v * 8)))
     return rc;
   int wid = conv_window(c->wave, sigma_ms);
@@ -2099,6 +2194,7 @@ int soap_diff_setup(soap_ctx *c, int32_t grid, int32_t n_phase, int32_t map_res,
   d.M = map_res;
   d.sigma = sigma_ms;
   for (int q = 0; q < 4; q++) d.lb[q] = lb ? lb[q] : 0.0;
+  if ((rc = diff_plan(c))) return rc;
   d.ready = true;
   d.have_fwd = false;
   return SOAP_OK;
@@ -2133,18 +2229,24 @@ static DiffArgs diff_args(soap_ctx *c) {
   a.kappa_f = d.prm.contrast_fac;
   a.ns = d.ns;
   for (int q = 0; q < 4; q++) a.lb[q] = d.lb[q];
-  a.mu_bounds = c->d_mub;
-  a.ck = (int32_t *)d.ck.p;
-  a.cm = (int32_t *)d.cm.p;
-  a.ct = (double *)d.ct.p;
-  a.cL = (double *)d.cL.p;
-  a.cmu = (double *)d.cmu.p;
-  a.cdt = (double *)d.cdt.p;
+  a.ck = (const int32_t *)d.ck.p;
+  a.cell = (const double2 *)d.cell.p;
+  a.map_j = (const int32_t *)d.map_j.p;
+  a.map_f = (const double *)d.map_f.p;
+  a.piece = (const DiffPiece *)d.piece.p;
+  a.psum = (const double2 *)d.psum.p;
+  a.pstart = (const int32_t *)d.pstart.p;
+  a.brow = (const int32_t *)d.brow.p;
+  a.n_piece = d.n_piece;
+  a.row_m = (int32_t *)d.row_m.p;
+  a.row_t = (double2 *)d.row_t.p;
+  a.drow = (int32_t *)d.drow.p;
+  a.blag = (int32_t *)d.blag.p;
+  a.mom = (double *)d.mom.p;
+  a.wts = (double *)d.wts.p;
   a.maps = d.maps;
   a.fmaps = d.fmaps;
-  a.acc = (unsigned long long *)d.acc.p;
   a.taps = (double *)d.taps.p;
-  a.krange = (int32_t *)d.krange.p;
   a.q = d.q;
   a.s = d.s;
   a.f = d.f;
@@ -2197,12 +2299,7 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
   if (d.nd > 2048) return fail(c, SOAP_ERR_LIMIT, "diff_forward: shift range of %d pixels", d.nd);
   const int ns = d_f ? 3 : 2;
   int rc;
-  if ((rc = ensure(c, d.acc, (size_t)d.P * c->n_mu * d.nd * ns * 2 * 8)) ||
-      (rc = ensure(c, d.taps, (size_t)d.P * c->n_mu * d.nd * ns * 8)) ||
-      (rc = ensure(c, d.krange, (size_t)d.P * c->n_mu * 2 * 4)) ||
-      (rc = ensure(c, d.C, (size_t)d.P * c->n_mu * d.nd * ns * 8)) ||
-      (rc = ensure(c, d.Cpart, (size_t)d.P * c->n_mu * diff_corr_chunks(c->n) * d.nd * ns * 8)))
-    return rc;
+  if ((rc = diff_plan(c)) || (rc = diff_buffers(c, d.nd, ns))) return rc;
   if (!c->mask_built && (rc = build_mask(c))) return rc;
   d.prm = *prm;
   d.ns = ns;
@@ -2285,7 +2382,7 @@ int soap_diff_backward(soap_ctx *c, double *grad5, double *d_gq, double *d_gs, d
   // the scalar gradients: the same device reduction as the graph path; the sums
   // land in the tail of the loss slot buffer
   double *g5 = (double *)d.tg.p + 3 * d.P + 1;
-  HIPCHK(c, launch_diff_grad(diff_cell_blocks((int64_t)d.G * d.G), (const double *)d.cell_part.p, g5, c->stream));
+  HIPCHK(c, launch_diff_grad(diff_piece_blocks(d.n_piece), (const double *)d.cell_part.p, g5, c->stream));
   HIPCHK(c, hipMemcpyAsync(grad5, g5, kDiffScalars * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return SOAP_OK;
@@ -2911,10 +3008,10 @@ namespace {
 std::vector<uintptr_t> dbatch_signature(const soap_ctx *c) {
   auto &d = c->diff;
   auto u = [](const void *p) { return (uintptr_t)p; };
-  return {u(d.acc.p),  u(d.taps.p),  u(d.krange.p), u(d.C.p),     u(d.Cpart.p),  u(d.res_part.p), u(d.ccf.p),
+  return {u(d.mom.p),  u(d.wts.p),   u(d.drow.p),   u(d.blag.p),  u(d.row_m.p),  u(d.row_t.p),    u(d.taps.p),  u(d.C.p),     u(d.Cpart.p),  u(d.res_part.p), u(d.ccf.p),
           u(d.par.p),  u(d.model.p), u(d.depth.p),  u(d.bis.p),   u(d.iters.p),  u(d.th.p),       u(d.dth.p),
           u(d.gy.p),   u(d.GF.p),    u(d.GI.p),     u(d.cell_part.p), u(d.I.p),  u(d.F.p),        u(d.ck.p),
-          u(d.cm.p),   u(d.ct.p),    u(d.cL.p),     u(d.cmu.p),   u(d.cdt.p),    u(d.mt_ptr.p),   u(d.mt_w.p),
+          u(d.cell.p), u(d.map_j.p), u(d.map_f.p),  u(d.piece.p), u(d.psum.p), u(d.brow.p), u(d.pstart.p), (uintptr_t)d.n_piece, u(d.mt_ptr.p), u(d.mt_w.p),
           u(d.mt_col.p), u(d.mt_val.p), u(c->ccf_part.p), u(c->m_start.p), u(c->m_alive.p), u(c->m_val.p),
           u(c->d_w_sorted), u(c->ctap.p), u(d.bisd.p), u(d.maps), u(d.q), u(d.s), u(d.target), u(d.f), u(d.fmaps),
           (uintptr_t)d.ns, (uintptr_t)d.nd,
@@ -3027,7 +3124,7 @@ hipError_t dbatch_enqueue_one(soap_diffbatch::Item &it, hipStream_t st, bool adj
                                (const double *)d.mt_val.p, (double *)d.GF.p, (double *)d.GI.p, (double *)d.Cpart.p,
                                (double *)d.C.p, it.gmaps, it.gfmaps, (double *)d.cell_part.p, it.gq, it.gs, it.gf,
                                bisd, st);
-    if (e == hipSuccess) e = launch_diff_grad(diff_cell_blocks((int64_t)d.G * d.G), (const double *)d.cell_part.p,
+    if (e == hipSuccess) e = launch_diff_grad(diff_piece_blocks(d.n_piece), (const double *)d.cell_part.p,
                                               it.g5, st);
     return e;
   }
@@ -3112,11 +3209,7 @@ int soap_diff_batch_bind(soap_diffbatch *b, int32_t i, double vsini_max, const d
   int nd = mshift(vsini_max) - dmin + 3;
   if (nd > 2048) return dfail(b, SOAP_ERR_LIMIT, "diff_batch_bind: shift range of %d pixels", nd);
   int rc;
-  if ((rc = ensure(c, d.acc, (size_t)d.P * c->n_mu * nd * ns * 2 * 8)) ||
-      (rc = ensure(c, d.taps, (size_t)d.P * c->n_mu * nd * ns * 8)) ||
-      (rc = ensure(c, d.krange, (size_t)d.P * c->n_mu * 2 * 4)) ||
-      (rc = ensure(c, d.C, (size_t)d.P * c->n_mu * nd * ns * 8)) ||
-      (rc = ensure(c, d.Cpart, (size_t)d.P * c->n_mu * diff_corr_chunks(c->n) * nd * ns * 8)) ||
+  if ((rc = diff_plan(c)) || (rc = diff_buffers(c, nd, ns)) ||
       (!c->mask_built && (rc = build_mask(c))) || (rc = diff_mask_transpose(c)))
     return dfail(b, rc, "diff_batch_bind: instance %d: %s", i, c->err.c_str());
   d.dmin = dmin;
@@ -3166,6 +3259,13 @@ int soap_diff_batch_step(soap_diffbatch *b, int32_t use_graph, int32_t with_adjo
     // the buffers were sized for the bound tap range; a per-call forward in between changes it
     if (it.bound && dbatch_signature(it.c) != it.sig)
       return dfail(b, SOAP_ERR_STATE, "diff_batch_step: an instance was changed after binding");
+    if (it.bound && !diff_plan_current(it.c)) {  // other bins of the same number: the plan is laid out anew
+      int rc = diff_plan(it.c);
+      if (!rc) rc = diff_buffers(it.c, it.nd, it.c->diff.ns);
+      if (rc) return dfail(b, rc, "diff_batch_step: %s", it.c->err.c_str());
+      it.sig = dbatch_signature(it.c);
+      dbatch_drop_graph(b);
+    }
   }
   const bool adj = with_adjoint != 0;
   if (!use_graph) return dbatch_enqueue(b, adj);

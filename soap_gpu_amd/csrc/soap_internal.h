@@ -286,6 +286,15 @@ struct LinSolar {
 };
 
 // Differentiable path (soap_diff.hip)
+// A run of at most kDiffPiece neighbouring cells (along a disk row) of one mu bin.
+// Rigid rotation gives a row one shift, so everything a cell needs beside its own limb
+// and filling factors is shared by the run.
+struct DiffPiece {
+  int32_t iy, iz0, len, k;
+};
+constexpr int kDiffPiece = 32;
+constexpr int diff_moments(int ns) { return ns == 3 ? 9 : 3; }
+
 struct DiffArgs {
   int64_t n;
   int32_t grid, n_mu, n_phase, map_res, dmin, nd;
@@ -293,11 +302,24 @@ struct DiffArgs {
   double h, expm1_h, vsini, u1, u2, kappa, kappa_f;
   double lb[4];                  // facula intensity 1 + LB(mu), LB = lb0 + lb1 mu + lb2 mu^2 + lb3 mu^3
   const double *prm;             // device (vsini, u1, u2, kappa, kappa_f) if not null (graph replays), else the fields above
-  const double *mu_bounds;       // n_mu - 1
-  int32_t *ck, *cm;              // per cell [G*G]: bin (-1 off disk), shift m
-  double *ct, *cL, *cmu, *cdt;   // weight t, limb, mu, dt/d(vsini)
+  // the disk's plan (grid, bins, map size and LB only: built once, see DiffPiece)
+  const int32_t *ck;             // per cell [G*G]: bin (-1 off disk)
+  const double2 *cell;           // per cell: 1 - mu, facula intensity factor 1 + LB(mu)
+  const int32_t *map_j;          // per grid row or column: first map node of its bilinear stencil
+  const double *map_f;           // and the weight of the second
+  const DiffPiece *piece;        // [n_piece], by bin, then row
+  const double2 *psum;           // [n_piece]: sums over the piece of a and a^2, a = 1 - mu
+  const int32_t *pstart;         // [n_mu][G + 1]: first piece of a bin at or after a row
+  const int32_t *brow;           // [n_mu][2]: first and last row that holds cells of a bin (first > last: none)
+  int32_t n_piece;
+  // per evaluation
+  int32_t *row_m;                // [G]: shift m of a disk row (delta = vsini y: one shift per row)
+  double2 *row_t;                // [G]: weight t, dt/d(vsini)
+  int32_t *drow;                 // [nd][2]: first and last row whose shift has tap index d
+  int32_t *blag;                 // [n_mu][2]: lags a bin's cells use (lo > hi: none)
+  double *mom;                   // [n_piece][diff_moments(ns)][P]: sums of phi, psi times 1, a, a^2 (see k_diff_moments)
+  double *wts;                   // [n_piece][ns][P]: the tap weights of the sets
   const double *maps, *fmaps;    // spot / facula filling factors [P][M][M] (fmaps null when ns == 2)
-  unsigned long long *acc;       // [P][n_mu][nd][ns][hi, lo]
   double *taps;                  // [P][n_mu][nd][ns]
   int32_t *krange;               // [P][n_mu][2]
   const double *q, *s, *f;       // quiet / spot / facula seed rows [n_mu][n] (f null when ns == 2)
@@ -512,7 +534,10 @@ hipError_t launch_mask_build_linear(const double *line_l, const double *line_w, 
 hipError_t launch_diff_forward_spectra(const DiffArgs &a, const ConvArgs &c, const double *target, int trim,
                                        double *res_part, int *res_blocks, hipStream_t s);
 int diff_conv_blocks(int64_t n);
-int diff_cell_blocks(int64_t ncell);
+int diff_piece_blocks(int n_piece);
+// the plan's per-cell tables (ck, cell) of a.grid, a.mu_bounds, a.lb
+hipError_t launch_diff_cells(const DiffArgs &a, const double *mu_bounds, int32_t *ck, double2 *cell, hipStream_t s);
+hipError_t launch_diff_psum(const DiffArgs &a, double2 *psum, hipStream_t s);
 hipError_t launch_fit_polish(const double *v, int n_v, const double *ccf, const double *par, int n_ccf, double *theta,
                              hipStream_t s);
 // mt_*: the mask in pixel-major form, sliced by 64 rows (row t = trimmed pixel
