@@ -19,6 +19,8 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <algorithm>
+
 #include "soap_internal.h"
 
 namespace soap {
@@ -224,7 +226,7 @@ __global__ __launch_bounds__(64 * kMomW) void k_diff_moments(DiffArgs a, int blo
   if (NS == 3) wt[2L * P] = kappa_f * (m[6] - u1 * m[7] - u2 * m[8]);
 }
 
-// taps[p][k][d][q] = sum over the pieces of bin k whose row has tap index d of w (1 - t),
+// taps (phase, bin k, offset d, set q) = sum over the pieces of bin k whose row has tap index d of w (1 - t),
 // and of those with index d + 1 of w t.  Block = (d, k), lanes over phases, the piece
 // range split over kTapW waves whose sums are added in wave order; the lanes first load
 // the factors of 64 pieces, which are then read from them one by one, so the weight
@@ -265,48 +267,162 @@ __global__ __launch_bounds__(64 * kTapW) void k_diff_taps(DiffArgs a) {
   for (int q = 0; q < NS; q++) s_t[w][q][lane] = acc[q];
   __syncthreads();
   if (w == 0 && p < P) {
-    double *o = a.taps + (((long)p * a.n_mu + k) * a.nd + d) * NS;
+    const int gp = p / a.grp_p, ngr = (a.n_mu * NS + a.grp_r - 1) / a.grp_r;
+    double *op = a.taps_p + ((((long)gp * a.n_mu + k) * a.nd + d) * NS) * 16 + p % a.grp_p;
 #pragma unroll
     for (int q = 0; q < NS; q++) {
       double x = s_t[0][q][lane];
 #pragma unroll
       for (int i = 1; i < kTapW; i++) x += s_t[i][q][lane];
-      o[q] = x;
+      op[q * 16] = x;
+      const int row = k * NS + q;
+      a.taps_r[(((long)p * ngr + row / a.grp_r) * a.nd + d) * 16 + row % a.grp_r] = x;
     }
   }
 }
 
+// ------------------------------------------------------------ contractions
+// The forward FIR, the seed gradients and the lag correlations are dense products in
+// FP64.  The matrix unit's 16x16x4 form sustains 32-47 TFLOP/s here and would pad 50
+// phases to 64, the vector unit 62-66, so they run as outer products on the vector unit:
+// R accumulators per lane and pixel, the R coefficients of a step in one register (lane
+// r of each row of 16 lanes holds coefficient r) and broadcast by the multiply-add itself
+// (DPP row_newbcast), so that a step costs one coefficient read and one pixel read for R
+// multiply-adds.  One coefficient per LDS word and multiply-add before: 311 (FIR), 311
+// (seed gradients) and 324 us (correlations, 492 before their lags were cut to the
+// bins') on the full adjoint, 15 TFLOP/s.
+#define SOAP_FMB(I) "v_fmac_f64_dpp %" #I ", %[t], %[x] row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\t"
+#define SOAP_FMB4 SOAP_FMB(0) SOAP_FMB(1) SOAP_FMB(2) SOAP_FMB(3)
+#define SOAP_FMB8 SOAP_FMB4 SOAP_FMB(4) SOAP_FMB(5) SOAP_FMB(6) SOAP_FMB(7)
+#define SOAP_FMB10 SOAP_FMB8 SOAP_FMB(8) SOAP_FMB(9)
+#define SOAP_FMB12 SOAP_FMB10 SOAP_FMB(10) SOAP_FMB(11)
+#define SOAP_FMB16 SOAP_FMB12 SOAP_FMB(12) SOAP_FMB(13) SOAP_FMB(14) SOAP_FMB(15)
+#define SOAP_O4(F) "+v"(F[0]), "+v"(F[1]), "+v"(F[2]), "+v"(F[3])
+#define SOAP_O8(F) SOAP_O4(F), "+v"(F[4]), "+v"(F[5]), "+v"(F[6]), "+v"(F[7])
+#define SOAP_O10(F) SOAP_O8(F), "+v"(F[8]), "+v"(F[9])
+#define SOAP_O12(F) SOAP_O10(F), "+v"(F[10]), "+v"(F[11])
+#define SOAP_O16(F) SOAP_O12(F), "+v"(F[12]), "+v"(F[13]), "+v"(F[14]), "+v"(F[15])
+// F[r] += t(lane r of this lane's row) x, one rounding each.  Two wait states lie between
+// a vector write of t and its broadcast read.
+template <int R>
+__device__ __forceinline__ void row_fma(double (&F)[R], double t, double x) {
+  static_assert(R == 4 || R == 8 || R == 10 || R == 12 || R == 16, "group sizes");
+  if constexpr (R == 4)
+    asm("s_nop 1\n\t" SOAP_FMB4 : SOAP_O4(F) : [t] "v"(t), [x] "v"(x));
+  else if constexpr (R == 8)
+    asm("s_nop 1\n\t" SOAP_FMB8 : SOAP_O8(F) : [t] "v"(t), [x] "v"(x));
+  else if constexpr (R == 10)
+    asm("s_nop 1\n\t" SOAP_FMB10 : SOAP_O10(F) : [t] "v"(t), [x] "v"(x));
+  else if constexpr (R == 12)
+    asm("s_nop 1\n\t" SOAP_FMB12 : SOAP_O12(F) : [t] "v"(t), [x] "v"(x));
+  else
+    asm("s_nop 1\n\t" SOAP_FMB16 : SOAP_O16(F) : [t] "v"(t), [x] "v"(x));
+}
+
 // I_p[j] = sum_k sum_d HQ[d] Q_k[j - dmin - d] + HS[d] S_k[j - dmin - d] (+ HF[d] Fa_k[j - dmin - d]);
-// block = (tile, p)
-template <int NS>
+// block = (tile of kDT * XB pixels, group of R phases).  Per bin the NS rows and the
+// taps of up to kFirD offsets are staged, the next bin's loads in flight during this
+// bin's sums where a block is small (XB = 1: few blocks, nothing else hides them; with
+// XB = 2 the registers cost more waves than they save, 104 -> 116 us); the reads of an
+// offset are issued before the multiply-adds of the one before it (left to the compiler
+// each read waits right before its use).
+constexpr int kFirD = 32;
+template <int NS, int R, int XB>
 __global__ __launch_bounds__(kDT) void k_diff_fir(DiffArgs a) {
-  extern __shared__ double rows[];  // [NS][row_len]
-  int p = blockIdx.y;
-  long j0 = (long)blockIdx.x * kDT;
-  int nd = a.nd, row_len = kDT + nd - 1;
-  long src0 = j0 - a.dmin - nd + 1;
-  double acc = 0.0;
-  for (int k = 0; k < a.n_mu; k++) {
-    int lo = a.blag[2 * k], hi = a.blag[2 * k + 1];
-    if (lo > hi) continue;  // uniform
-    __syncthreads();
-    for (int e = threadIdx.x; e < row_len; e += blockDim.x) {
-      long i = src0 + e;
-      bool in = i >= 0 && i < a.n;
-      rows[e] = in ? a.q[(long)k * a.n + i] : 0.0;
-      rows[row_len + e] = in ? a.s[(long)k * a.n + i] : 0.0;
-      if (NS == 3) rows[2 * row_len + e] = in ? a.f[(long)k * a.n + i] : 0.0;
-    }
-    __syncthreads();
-    const double *T = a.taps + ((long)p * a.n_mu + k) * nd * NS;
-    for (int di = lo; di <= hi; di++) {
-      int e = threadIdx.x + nd - 1 - di;
+  extern __shared__ double s_fir[];  // [NS][row_len], then [kFirD][NS][16]
+  constexpr int kRow = XB + 1, kTap = kFirD * NS * 16 / kDT;  // values per thread of a bin's staging
+  constexpr bool kAhead = XB == 1;
+  const int g = blockIdx.y, lane16 = threadIdx.x & 15, tid = threadIdx.x;
+  const long j0 = (long)blockIdx.x * (kDT * XB), n = a.n;
+  const int nd = a.nd, n_mu = a.n_mu, row_len = kDT * XB + nd - 1;
+  const long src0 = j0 - a.dmin - nd + 1;
+  double *s_t = s_fir + NS * row_len;
+  double F[XB][R];
 #pragma unroll
-      for (int q = 0; q < NS; q++) acc = fma(T[di * NS + q], rows[q * row_len + e], acc);
+  for (int b = 0; b < XB; b++)
+#pragma unroll
+    for (int r = 0; r < R; r++) F[b][r] = 0.0;
+  auto row_at = [&](int k, int q, int e) {  // element e of the staged row, 0 outside the spectrum
+    const long i = src0 + e;
+    const bool in = i >= 0 && i < n;
+    const double *X = q == 0 ? a.q : q == 1 ? a.s : a.f;
+    const double v = X[(long)k * n + (in ? i : 0)];
+    return in ? v : 0.0;
+  };
+  auto taps_at = [&](int k, int d) { return a.taps_p + ((((long)g * n_mu + k) * nd + d) * NS) * 16; };
+  double rv[NS][kRow], tv[kTap];
+  auto fetch = [&](int k) {
+    const int lo = a.blag[2 * k], hi = a.blag[2 * k + 1];
+    if (lo > hi) return;  // uniform
+#pragma unroll
+    for (int q = 0; q < NS; q++)
+#pragma unroll
+      for (int u = 0; u < kRow; u++) rv[q][u] = row_at(k, q, min(tid + u * kDT, row_len - 1));
+    const double *T = taps_at(k, lo);
+    const int nt = min(kFirD, hi + 1 - lo) * NS * 16;
+#pragma unroll
+    for (int u = 0; u < kTap; u++) tv[u] = T[min(tid + u * kDT, nt - 1)];
+  };
+  if (kAhead) fetch(0);
+  for (int k = 0; k < n_mu; k++) {
+    const int lo = a.blag[2 * k], hi = a.blag[2 * k + 1];
+    if (!kAhead) fetch(k);
+    for (int dc = lo; dc <= hi; dc += kFirD) {
+      const int nc = min(kFirD, hi + 1 - dc);
+      __syncthreads();
+      if (dc == lo) {
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+#pragma unroll
+          for (int u = 0; u < kRow; u++)
+            if (tid + u * kDT < row_len) s_fir[q * row_len + tid + u * kDT] = rv[q][u];
+          for (int e = tid + kRow * kDT; e < row_len; e += kDT) s_fir[q * row_len + e] = row_at(k, q, e);  // nd > kDT
+        }
+#pragma unroll
+        for (int u = 0; u < kTap; u++)
+          if (tid + u * kDT < nc * NS * 16) s_t[tid + u * kDT] = tv[u];
+      } else {
+        const double *T = taps_at(k, dc);
+        for (int e = tid; e < nc * NS * 16; e += kDT) s_t[e] = T[e];
+      }
+      __syncthreads();
+      if (kAhead && dc == lo && k + 1 < n_mu) fetch(k + 1);
+      const double *x = s_fir + tid + nd - 1 - dc, *tp = s_t + lane16;
+      double t[2][NS], xv[2][NS][XB];
+      auto read = [&](int s, int d) {
+#pragma unroll
+        for (int q = 0; q < NS; q++) {
+          t[s][q] = tp[(d * NS + q) * 16];
+#pragma unroll
+          for (int b = 0; b < XB; b++) xv[s][q][b] = x[q * row_len + b * kDT - d];
+        }
+      };
+      auto sums = [&](int s) {
+#pragma unroll
+        for (int q = 0; q < NS; q++)
+#pragma unroll
+          for (int b = 0; b < XB; b++) row_fma<R>(F[b], t[s][q], xv[s][q][b]);
+      };
+      read(0, 0);
+      for (int d = 0; d < nc; d += 2) {
+        read(1, min(d + 1, nc - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        sums(0);
+        read(0, min(d + 2, nc - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        if (d + 1 < nc) sums(1);
+      }
     }
+    if (kAhead && lo > hi && k + 1 < n_mu) fetch(k + 1);  // a bin without cells: nothing was staged
   }
-  long j = j0 + threadIdx.x;
-  if (j < a.n) a.I[(long)p * a.n + j] = acc;
+#pragma unroll
+  for (int b = 0; b < XB; b++) {
+    const long j = j0 + tid + b * kDT;
+    if (j >= n) continue;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (g * R + r < a.n_phase) a.I[(long)(g * R + r) * n + j] = F[b][r];
+  }
 }
 
 // F_p = conv(I_p) (zero outside wid < i < n-1-wid); residual partials of the
@@ -787,93 +903,194 @@ __global__ __launch_bounds__(kDT) void k_diff_convT(DiffArgs a, ConvArgs c, cons
   }
 }
 
-// lag correlations C[k][d][set][p] = sum_j G_I[p][j] X_k[j - dmin - d], in two
-// passes.  Pass 1: block = (chunk of kCorrT pixels, bin k, group of kCorrPG
-// phases); the bin's two seed-row segments are staged once for the group.  Each
-// thread owns kCorrPer consecutive pixels (G_I of the phase in registers) and,
-// per group of kCorrL lags, reads one register window of the staged row and
-// forms kCorrL partial sums; the block adds them up through LDS ([lag][thread]
-// then 32-lane shuffles) into the chunk's partial.  Pass 2 sums the chunk
-// partials in chunk order (deterministic, no atomics).
-constexpr int kCorrPer = 9;  // odd: a thread stride of kCorrPer doubles is free of LDS bank conflicts
-constexpr int kCorrT = kDT * kCorrPer;
-constexpr int kCorrL = 8;
-constexpr int kCorrPG = 10;
-// One pass covers nsp <= 2 seed cubes (x0, x1), written to sets soff, soff + 1 of
-// the ns-set tables; the facula set, when present, is a second pass (three staged
-// rows would not fit the LDS budget).
-__global__ __launch_bounds__(kDT) void k_diff_corr(DiffArgs a, const double *GI, double *Cpart, const double *x0,
-                                                   const double *x1, int nsp, int soff) {
-  extern __shared__ double lds[];  // row(s) [kCorrT + nd - 1 + kCorrL] each, then [kCorrL][kDT] partials
-  const int k = blockIdx.y, chunk = blockIdx.x, nchunk = gridDim.x;
-  const long j0 = (long)chunk * kCorrT;
-  const int nd = a.nd, rl = kCorrT + nd - 1 + kCorrL, ns = a.ns;
-  double *rq = lds, *rs = rq + rl, *red = rq + nsp * rl;
-  const long src0 = j0 - a.dmin - nd + 1;
-  for (int e = threadIdx.x; e < rl; e += blockDim.x) {
-    long i = src0 + e;
-    bool in = i >= 0 && i < a.n && e < kCorrT + nd - 1;
-    rq[e] = in ? x0[(long)k * a.n + i] : 0.0;
-    if (nsp == 2) rs[e] = in ? x1[(long)k * a.n + i] : 0.0;
+// lag correlations C[k][d][set][p] = sum_j G_I[p][j] X_k[j - dmin - d], in two passes.
+// Pass 1: block = (chunk of kCorrT pixels, group of kCorrRB (bin, set) rows, lag tile of
+// 16 and group of PB phases); the rows' segments are staged once and each of four waves
+// takes a quarter of the pixels.  Lane l of a row of 16 lanes is lag l, the four rows of
+// lanes take 16 pixels each of every 64: a step loads G_I of 64 pixels per phase, and
+// multiply-add n takes G_I of the row's pixel n from lane n (DPP row_newbcast) and the
+// rows' pixel at the lane's lag from LDS, which then serves PB phases.  The lane rows'
+// sums are added by swaps between them and the waves' through LDS.  PB kCorrRB = 50
+// accumulators keep three waves per SIMD.  Lags are those the group's bins use.  Pass 2
+// sums the chunk partials in chunk order (deterministic, no atomics).
+constexpr int kCorrRB = 5;
+constexpr int kCorrT = 1024;
+constexpr int kCorrWin = kCorrT + 16;  // staged pixels of a row
+// F[p] += g[p](lane N of this lane's row) x
+template <int N, int PB>
+__device__ __forceinline__ void lag_fma(double (&F)[PB], const double (&g)[PB], double x) {
+  static_assert(PB == 8 || PB == 10, "phases per wave");
+#define SOAP_LAG(I, J) "v_fmac_f64_dpp %" #I ", %" #J ", %[x] row_newbcast:%c[n] row_mask:0xf bank_mask:0xf\n\t"
+  if constexpr (PB == 8)
+    asm("s_nop 1\n\t" SOAP_LAG(0, 8) SOAP_LAG(1, 9) SOAP_LAG(2, 10) SOAP_LAG(3, 11) SOAP_LAG(4, 12) SOAP_LAG(5, 13)
+            SOAP_LAG(6, 14) SOAP_LAG(7, 15)
+        : SOAP_O8(F)
+        : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "v"(g[4]), "v"(g[5]), "v"(g[6]), "v"(g[7]), [x] "v"(x),
+          [n] "i"(N));
+  else
+    asm("s_nop 1\n\t" SOAP_LAG(0, 10) SOAP_LAG(1, 11) SOAP_LAG(2, 12) SOAP_LAG(3, 13) SOAP_LAG(4, 14) SOAP_LAG(5, 15)
+            SOAP_LAG(6, 16) SOAP_LAG(7, 17) SOAP_LAG(8, 18) SOAP_LAG(9, 19)
+        : SOAP_O10(F)
+        : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "v"(g[4]), "v"(g[5]), "v"(g[6]), "v"(g[7]), "v"(g[8]),
+          "v"(g[9]), [x] "v"(x), [n] "i"(N));
+#undef SOAP_LAG
+}
+// the 16 pixels of each lane row from pixel N on; xc: the rows' values at pixel N.  The
+// next pixel's are read before this one's multiply-adds (left to the compiler each read
+// waits right before its use), after the last those of the next step's first pixel.
+template <int N, int PB, int RB>
+__device__ __forceinline__ void lag_steps(double (&F)[RB][PB], const double (&g)[PB], double (&xc)[RB],
+                                          const double *x) {
+  if constexpr (N < 16) {
+    double xn[RB];
+#pragma unroll
+    for (int r = 0; r < RB; r++) xn[r] = x[r * kCorrWin + (N < 15 ? N + 1 : 64)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < RB; r++) lag_fma<N>(F[r], g, xc[r]);
+    lag_steps<N + 1>(F, g, xn, x);
+#pragma unroll
+    for (int r = 0; r < RB; r++) xc[r] = xn[r];
+  }
+}
+
+// first lag of a row group: the least its bins use
+__device__ __forceinline__ int corr_lag0(const DiffArgs &a, int k0, int k1, int &hi) {
+  int lo = a.nd;
+  hi = -1;
+  for (int k = k0; k <= k1; k++) {
+    lo = min(lo, a.blag[2 * k]);
+    hi = max(hi, a.blag[2 * k + 1]);
+  }
+  return lo;
+}
+
+// a + b with the halves (HALF 32) or the neighbouring rows of 16 lanes (HALF 16) of the
+// wave folded: the lower half or even row of the result holds a's, the other b's
+template <int HALF>
+__device__ __forceinline__ double swap_fold(double a, double b) {
+  const long long va = __double_as_longlong(a), vb = __double_as_longlong(b);
+  const unsigned al = (unsigned)va, ah = (unsigned)(va >> 32), bl = (unsigned)vb, bh = (unsigned)(vb >> 32);
+  unsigned l0, l1, h0, h1;
+  if constexpr (HALF == 32) {
+    const auto l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+    l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+  } else {
+    const auto l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+    l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+  }
+  return __longlong_as_double(((long long)h0 << 32) | l0) + __longlong_as_double(((long long)h1 << 32) | l1);
+}
+
+// Cpart [chunk][row][lag tile][P][16]
+template <int PB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_diff_corr(DiffArgs a, const double *GI,
+                                                                                        double *Cpart, int n_z) {
+  extern __shared__ double s_x[];  // [kCorrRB][kCorrWin], room for the last step's read ahead; then the waves' sums
+  constexpr int RB = kCorrRB, NF = (RB * PB + 3) / 4;  // sums per wave, four in a register
+  const int rows = a.n_mu * a.ns, r0 = blockIdx.y * RB, ns = a.ns;
+  const int chunk = blockIdx.x, z = blockIdx.z % n_z, p0 = blockIdx.z / n_z * PB;
+  int hi;
+  const int lag0 = corr_lag0(a, r0 / ns, min(rows - 1, r0 + RB - 1) / ns, hi) + 16 * z;
+  if (lag0 > hi) return;  // uniform over the block
+  const long j0 = (long)chunk * kCorrT, n = a.n;
+  // lag d = lag0 + l reads X[j - dmin - d]: window index (j - j0) + 15 - l
+  const long src0 = j0 - a.dmin - lag0 - 15;
+#pragma unroll
+  for (int r = 0; r < RB; r++) {
+    const int row = min(r0 + r, rows - 1), set = row % ns;
+    const double *X = (set == 0 ? a.q : set == 1 ? a.s : a.f) + (long)(row / ns) * n;
+    for (int e = threadIdx.x; e < kCorrWin; e += 256) {
+      const long i = src0 + e;
+      const bool in = i >= 0 && i < n;
+      const double v = X[in ? i : 0];
+      s_x[r * kCorrWin + e] = in ? v : 0.0;
+    }
   }
   __syncthreads();
-  const int p1 = min(a.n_phase, (int)(blockIdx.z + 1) * kCorrPG);
-  for (int p = blockIdx.z * kCorrPG; p < p1; p++) {
-    double g[kCorrPer];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l = lane & 15;
+  double F[RB][PB], g[PB], gn[PB], xc[RB];
 #pragma unroll
-    for (int u = 0; u < kCorrPer; u++) {
-      long j = j0 + threadIdx.x * kCorrPer + u;
-      g[u] = j < a.n ? GI[(long)p * a.n + j] : 0.0;
+  for (int r = 0; r < RB; r++)
+#pragma unroll
+    for (int p = 0; p < PB; p++) F[r][p] = 0.0;
+  const int j1 = (int)min((long)kCorrT, n - j0);  // pixels of the chunk
+  auto load = [&](double (&v)[PB], int s) {
+    const bool in = s + lane < j1;
+    const double *G = GI + j0 + (in ? s + lane : j1 - 1);
+#pragma unroll
+    for (int p = 0; p < PB; p++) {
+      const double x = G[(long)min(p0 + p, a.n_phase - 1) * n];
+      v[p] = in ? x : 0.0;
     }
-    double *out = Cpart + (((long)p * a.n_mu + k) * nchunk + chunk) * nd * ns;
-    const int dlo = a.blag[2 * k], dhi = a.blag[2 * k + 1];  // the lags this bin's cells use
-    for (int set = 0; set < nsp; set++) {
-      const double *row = (set ? rs : rq) + threadIdx.x * kCorrPer;
-      for (int d0 = dlo; d0 <= dhi; d0 += kCorrL) {
-        // lag d = d0 + l reads X[j - dmin - d] = row[u + nd - 1 - d]; window base nd - d0 - kCorrL
-        const int wb = nd - d0 - kCorrL;
-        double w[kCorrPer + kCorrL - 1];
+  };
+  const int s0 = w * (kCorrT / 4), s1 = min(j1, s0 + kCorrT / 4);
+  const double *x = s_x + (lane & 48) + 15 - l;
 #pragma unroll
-        for (int e = 0; e < kCorrPer + kCorrL - 1; e++) {
-          int x = wb + e;
-          w[e] = x >= 0 ? row[x] : 0.0;  // x < 0 only for lags d >= nd (discarded)
-        }
-        double acc[kCorrL];
+  for (int r = 0; r < RB; r++) xc[r] = x[r * kCorrWin + s0];
+  if (s0 < s1) load(g, s0);
+  for (int s = s0; s < s1; s += 64) {
+    load(gn, s + 64);
+    lag_steps<0>(F, g, xc, x + s);
 #pragma unroll
-        for (int l = 0; l < kCorrL; l++) {
-          acc[l] = 0.0;
+    for (int p = 0; p < PB; p++) g[p] = gn[p];
+  }
+  __syncthreads();  // the staged rows become the waves' sums
+  const int which = (0x3120 >> (4 * (lane >> 4))) & 15;  // rows 0..3 of a folded register hold sums 0, 2, 1, 3
 #pragma unroll
-          for (int u = 0; u < kCorrPer; u++) acc[l] = fma(g[u], w[u + kCorrL - 1 - l], acc[l]);
-        }
-        __syncthreads();  // red is free
+  for (int f = 0; f < NF; f++) {
+    double v[4];
 #pragma unroll
-        for (int l = 0; l < kCorrL; l++) red[l * kDT + threadIdx.x] = acc[l];
-        __syncthreads();
-        // kDT threads = kCorrL lags x 32 lanes: each lane sums kDT / 32 partials
-        const int l = threadIdx.x >> 5, part = threadIdx.x & 31;
-        double x = 0.0;
-#pragma unroll
-        for (int r = 0; r < kDT / 32; r++) x += red[l * kDT + r * 32 + part];
-        for (int off = 16; off > 0; off >>= 1) x += __shfl_xor(x, off);
-        if (part == 0 && d0 + l < nd) out[(d0 + l) * ns + soff + set] = x;
-      }
+    for (int u = 0; u < 4; u++) {
+      const int i = 4 * f + u;
+      v[u] = i < RB * PB ? F[i / PB][i % PB] : 0.0;
     }
+    s_x[((long)w * NF * 4 + 4 * f + which) * 16 + l] = swap_fold<16>(swap_fold<32>(v[0], v[1]), swap_fold<32>(v[2], v[3]));
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < RB * PB * 16; e += 256) {
+    const int r = e / (PB * 16), p = e / 16 % PB;
+    double t = s_x[e];
+#pragma unroll
+    for (int i = 1; i < 4; i++) t += s_x[i * NF * 64 + e];
+    if (r0 + r < rows && p0 + p < a.n_phase)
+      Cpart[((((long)chunk * rows + r0 + r) * n_z + z) * a.n_phase + p0 + p) * 16 + (e & 15)] = t;
   }
 }
 
-__global__ void k_diff_corr_reduce(DiffArgs a, int n_pk, int nd, int nchunk, const double *Cpart, double *C) {
-  const int ns = a.ns;
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;  // (p, k) x (d, set)
-  if (e >= (long)n_pk * nd * ns) return;
-  long pk = e / (nd * ns), r = e % (nd * ns);
-  const int d = (int)(r / ns), p = (int)(pk / a.n_mu), k = (int)(pk % a.n_mu);
-  double x = 0.0;
-  if (d >= a.blag[2 * k] && d <= a.blag[2 * k + 1])  // k_diff_corr computes only these lags
-    for (int c = 0; c < nchunk; c++) x += Cpart[(pk * nchunk + c) * nd * ns + r];
-  C[((long)k * nd * ns + r) * a.n_phase + p] = x;
+static int corr_pb(int n_phase) { return (n_phase + 9) / 10 * 10 <= (n_phase + 7) / 8 * 8 ? 10 : 8; }
+static int corr_chunks(int64_t n) { return (int)((n + kCorrT - 1) / kCorrT); }
+size_t diff_corr_part(int64_t n, int n_phase, int rows, int nd) {
+  return (size_t)corr_chunks(n) * rows * ((nd + 15) / 16) * n_phase * 16;
 }
 
-int diff_corr_chunks(int64_t n) { return (int)((n + kCorrT - 1) / kCorrT); }
+// one thread per (row, phase, lag of a tile of 16)
+__global__ void k_diff_corr_reduce(DiffArgs a, int nchunk, int n_z, const double *Cpart, double *C) {
+  const int ns = a.ns, rows = a.n_mu * ns, P = a.n_phase;
+  const long per = (long)n_z * P * 16, e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows * per) return;
+  const int row = (int)(e / per), z = (int)(e % per / (P * 16)), p = (int)(e % (P * 16) / 16), l = (int)(e % 16);
+  const int k = row / ns, r0 = row / kCorrRB * kCorrRB;
+  int hi;
+  const int d = corr_lag0(a, r0 / ns, min(rows - 1, r0 + kCorrRB - 1) / ns, hi) + 16 * z + l;
+  if (d < a.blag[2 * k] || d > a.blag[2 * k + 1]) return;  // no cell of the bin uses it
+  constexpr int kU = 16;
+  const double *in = Cpart + e;
+  const long cs = rows * per;
+  double x = 0.0;
+  int c = 0;
+  for (; c + kU <= nchunk; c += kU) {
+    double t[kU];
+#pragma unroll
+    for (int u = 0; u < kU; u++) t[u] = in[(c + u) * cs];
+#pragma unroll
+    for (int u = 0; u < kU; u++) x += t[u];
+  }
+  for (; c < nchunk; c++) x += in[c * cs];
+  C[(((long)k * a.nd + d) * ns + row % ns) * P + p] = x;
+}
 
 // a_X = (1 - t) C[d0] + t C[d0 - 1] of the bin and phase (C [k][d][set][P])
 __device__ __forceinline__ double corr_at(const double *Cd, int ns, int P, int set, double t, double &diff) {
@@ -1029,42 +1246,179 @@ __global__ __launch_bounds__(256) void k_diff_mapgrad(DiffArgs a, const double *
   }
 }
 
-// seed gradients gX_k[i] = sum_p sum_d HX_pk[d] G_I,p[i + dmin + d]; block = (tile, bin)
-template <int NS>
+// seed gradients gX_k[i] = sum_p sum_d HX_pk[d] G_I,p[i + dmin + d]; block = (tile of
+// kDT * XB pixels, group of R (bin, set) rows), kSeedP phases staged at a time with the
+// taps of up to kSeedD of the offsets the group's bins use; the next phases' loads and
+// the next offset's reads are in flight as in k_diff_fir
+constexpr int kSeedP = 4;
+constexpr int kSeedD = 32;
+template <int R, int XB>
 __global__ __launch_bounds__(kDT) void k_diff_seedgrad(DiffArgs a, const double *GI, double *gq, double *gs,
                                                        double *gf) {
-  extern __shared__ double gl[];  // G_I,p over [i0 + dmin, i0 + kDT + dmin + nd - 1)
-  int k = blockIdx.y;
-  long i0 = (long)blockIdx.x * kDT;
-  int nd = a.nd, len = kDT + nd - 1;
-  double ax[NS];
+  extern __shared__ double s_sg[];  // [kSeedP][len], then [kSeedP][kSeedD][16]
+  constexpr int kRow = XB + 1, kTap = kSeedD * 16 / kDT;
+  constexpr bool kAhead = XB == 1;
+  const int g = blockIdx.y, ng = gridDim.y, ns = a.ns, rows = a.n_mu * ns, tid = threadIdx.x, lane16 = tid & 15;
+  const long i0 = (long)blockIdx.x * (kDT * XB), n = a.n;
+  const int nd = a.nd, len = kDT * XB + nd - 1, P = a.n_phase;
+  double *s_t = s_sg + kSeedP * len;
+  double F[XB][R];
 #pragma unroll
-  for (int q = 0; q < NS; q++) ax[q] = 0.0;
-  for (int p = 0; p < a.n_phase; p++) {
-    int lo = a.blag[2 * k], hi = a.blag[2 * k + 1];
-    if (lo > hi) continue;  // uniform
-    __syncthreads();
-    for (int e = threadIdx.x; e < len; e += blockDim.x) {
-      long j = i0 + a.dmin + e;
-      gl[e] = (j >= 0 && j < a.n) ? GI[(long)p * a.n + j] : 0.0;
+  for (int b = 0; b < XB; b++)
+#pragma unroll
+    for (int r = 0; r < R; r++) F[b][r] = 0.0;
+  int lo = nd, hi = -1;
+  for (int k = g * R / ns; k <= min(rows - 1, g * R + R - 1) / ns; k++) {
+    lo = min(lo, a.blag[2 * k]);
+    hi = max(hi, a.blag[2 * k + 1]);
+  }
+  auto gi_at = [&](int p, int e) {
+    const long j = i0 + a.dmin + e;
+    const bool in = j >= 0 && j < n;
+    const double v = GI[(long)min(p, P - 1) * n + (in ? j : 0)];
+    return in ? v : 0.0;
+  };
+  auto taps_at = [&](int p, int d) { return a.taps_r + (((long)min(p, P - 1) * ng + g) * nd + d) * 16; };
+  double rv[kSeedP][kRow], tv[kSeedP][kTap];
+  const int nt = min(kSeedD, hi + 1 - lo) * 16;
+  auto fetch = [&](int p0) {
+#pragma unroll
+    for (int u = 0; u < kSeedP; u++) {
+#pragma unroll
+      for (int w = 0; w < kRow; w++) rv[u][w] = gi_at(p0 + u, min(tid + w * kDT, len - 1));
+      const double *T = taps_at(p0 + u, lo);
+#pragma unroll
+      for (int w = 0; w < kTap; w++) tv[u][w] = T[min(tid + w * kDT, nt - 1)];
     }
-    __syncthreads();
-    const double *T = a.taps + ((long)p * a.n_mu + k) * nd * NS;
-    for (int d = lo; d <= hi; d++) {
-      double g = gl[threadIdx.x + d];
+  };
+  if (kAhead && lo <= hi) fetch(0);
+  for (int p0 = 0; p0 < P && lo <= hi; p0 += kSeedP) {
+    const int np = min(kSeedP, P - p0);
+    if (!kAhead) fetch(p0);
+    for (int dc = lo; dc <= hi; dc += kSeedD) {
+      const int nc = min(kSeedD, hi + 1 - dc);
+      __syncthreads();
 #pragma unroll
-      for (int q = 0; q < NS; q++) ax[q] = fma(T[d * NS + q], g, ax[q]);
+      for (int u = 0; u < kSeedP; u++) {
+        if (dc == lo) {
+#pragma unroll
+          for (int w = 0; w < kRow; w++)
+            if (tid + w * kDT < len) s_sg[u * len + tid + w * kDT] = rv[u][w];
+          for (int e = tid + kRow * kDT; e < len; e += kDT) s_sg[u * len + e] = gi_at(p0 + u, e);  // nd > kDT
+#pragma unroll
+          for (int w = 0; w < kTap; w++)
+            if (tid + w * kDT < nt) s_t[u * kSeedD * 16 + tid + w * kDT] = tv[u][w];
+        } else {
+          const double *T = taps_at(p0 + u, dc);
+          for (int e = tid; e < nc * 16; e += kDT) s_t[u * kSeedD * 16 + e] = T[e];
+        }
+      }
+      __syncthreads();
+      if (kAhead && dc == lo && p0 + kSeedP < P) fetch(p0 + kSeedP);
+      for (int u = 0; u < np; u++) {
+        const double *x = s_sg + u * len + tid + dc, *tp = s_t + u * kSeedD * 16 + lane16;
+        constexpr int D = 2;  // offsets per step
+        double t[2][D], xv[2][D][XB];
+        auto read = [&](int s, int d) {
+#pragma unroll
+          for (int w = 0; w < D; w++) {
+            const int dw = min(d + w, nc - 1);
+            t[s][w] = tp[dw * 16];
+#pragma unroll
+            for (int b = 0; b < XB; b++) xv[s][w][b] = x[b * kDT + dw];
+          }
+        };
+        auto sums = [&](int s, int d) {
+#pragma unroll
+          for (int w = 0; w < D; w++)
+            if (d + w < nc)
+#pragma unroll
+              for (int b = 0; b < XB; b++) row_fma<R>(F[b], t[s][w], xv[s][w][b]);
+        };
+        read(0, 0);
+        for (int d = 0; d < nc; d += 2 * D) {
+          read(1, d + D);
+          __builtin_amdgcn_sched_barrier(0);
+          sums(0, d);
+          read(0, d + 2 * D);
+          __builtin_amdgcn_sched_barrier(0);
+          sums(1, d + D);
+        }
+      }
     }
   }
-  long i = i0 + threadIdx.x;
-  if (i < a.n) {
-    gq[(long)k * a.n + i] = ax[0];
-    gs[(long)k * a.n + i] = ax[1];
-    if (NS == 3) gf[(long)k * a.n + i] = ax[NS - 1];
+#pragma unroll
+  for (int b = 0; b < XB; b++) {
+    const long i = i0 + tid + b * kDT;
+    if (i >= n) continue;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int row = g * R + r, k = row / ns, set = row - k * ns;
+      if (row < rows) (set == 0 ? gq : set == 1 ? gs : gf)[(long)k * n + i] = F[b][r];
+    }
   }
 }
 
 // ------------------------------------------------------------ launchers
+// Two pixels per thread serve a coefficient read twice, where that still leaves two
+// blocks per CU; one otherwise.
+static bool two_pixels(int64_t n, int groups) { return (n + 2 * kDT - 1) / (2 * kDT) * groups >= 512; }
+
+template <int NS, int R>
+static hipError_t launch_fir_r(const DiffArgs &a, hipStream_t s) {
+  const int groups = (a.n_phase + R - 1) / R;
+  const bool two = two_pixels(a.n, groups);
+  const int px = two ? 2 * kDT : kDT;
+  const size_t lds = (size_t)(NS * (px + a.nd - 1) + kFirD * NS * 16) * sizeof(double);  // at most 86 KB
+  dim3 gr((unsigned)((a.n + px - 1) / px), groups);
+  if (two)
+    k_diff_fir<NS, R, 2><<<gr, kDT, lds, s>>>(a);
+  else
+    k_diff_fir<NS, R, 1><<<gr, kDT, lds, s>>>(a);
+  return hipGetLastError();
+}
+
+template <int NS>
+static hipError_t launch_fir_ns(const DiffArgs &a, hipStream_t s) {
+  switch (a.grp_p) {
+    case 4: return launch_fir_r<NS, 4>(a, s);
+    case 8: return launch_fir_r<NS, 8>(a, s);
+    case 10: return launch_fir_r<NS, 10>(a, s);
+    case 12: return launch_fir_r<NS, 12>(a, s);
+    case 16: return launch_fir_r<NS, 16>(a, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int R>
+static hipError_t launch_seed_r(const DiffArgs &a, const double *GI, double *gq, double *gs, double *gf,
+                                hipStream_t s) {
+  const int groups = (a.n_mu * a.ns + R - 1) / R;
+  const bool two = two_pixels(a.n, groups);
+  const int px = two ? 2 * kDT : kDT;
+  const size_t lds = (size_t)kSeedP * (px + a.nd - 1 + kSeedD * 16) * sizeof(double);  // at most 98 KB
+  dim3 gr((unsigned)((a.n + px - 1) / px), groups);
+  if (two)
+    k_diff_seedgrad<R, 2><<<gr, kDT, lds, s>>>(a, GI, gq, gs, gf);
+  else
+    k_diff_seedgrad<R, 1><<<gr, kDT, lds, s>>>(a, GI, gq, gs, gf);
+  return hipGetLastError();
+}
+
+template <int PB>
+static hipError_t launch_corr_p(const DiffArgs &a, const double *GI, double *Cpart, double *C, hipStream_t s) {
+  const int rows = a.n_mu * a.ns, n_tile = (a.n_phase + PB - 1) / PB, n_z = (a.nd + 15) / 16, nch = corr_chunks(a.n);
+  if ((long)n_tile * n_z > 65535) return hipErrorInvalidValue;
+  dim3 gr(nch, (rows + kCorrRB - 1) / kCorrRB, n_tile * n_z);
+  const size_t lds = (size_t)std::max(kCorrRB * kCorrWin + 64, 4 * (kCorrRB * PB + 3) / 4 * 64) * sizeof(double);
+  k_diff_corr<PB><<<gr, 256, lds, s>>>(a, GI, Cpart, n_z);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const long tot = (long)rows * n_z * a.n_phase * 16;
+  k_diff_corr_reduce<<<(unsigned)((tot + kDT - 1) / kDT), kDT, 0, s>>>(a, nch, n_z, Cpart, C);
+  return hipGetLastError();
+}
+
 hipError_t launch_diff_forward_spectra(const DiffArgs &a, const ConvArgs &c, const double *target, int trim,
                                        double *res_part, int *res_blocks, hipStream_t s) {
   hipError_t e;
@@ -1087,14 +1441,9 @@ hipError_t launch_diff_forward_spectra(const DiffArgs &a, const ConvArgs &c, con
     k_diff_taps<2><<<gt, 64 * kTapW, 0, s>>>(a);
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  size_t lds_fir = (size_t)a.ns * (kDT + a.nd - 1) * sizeof(double);
-  if (lds_fir > 65536) return hipErrorInvalidValue;
-  dim3 gf((unsigned)((a.n + kDT - 1) / kDT), a.n_phase);
-  if (a.ns == 3)
-    k_diff_fir<3><<<gf, kDT, lds_fir, s>>>(a);
-  else
-    k_diff_fir<2><<<gf, kDT, lds_fir, s>>>(a);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if ((size_t)a.ns * (kDT + a.nd - 1) * sizeof(double) > 65536) return hipErrorInvalidValue;
+  e = a.ns == 3 ? launch_fir_ns<3>(a, s) : launch_fir_ns<2>(a, s);
+  if (e != hipSuccess) return e;
   size_t lds_conv = (size_t)(4 * kDT + 2 * c.ntp) * sizeof(double);
   if (lds_conv > 65536) return hipErrorInvalidValue;
   int nb = (int)((a.n + 4 * kDT - 1) / (4 * kDT));
@@ -1252,19 +1601,9 @@ hipError_t launch_diff_backward(const DiffArgs &a, const ConvArgs &c, const doub
   dim3 gc((unsigned)((a.n + 4 * kDT - 1) / (4 * kDT)), a.n_phase);
   k_diff_convT<<<gc, kDT, lds_conv, s>>>(a, c, GF, GI);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  size_t lds_corr = (size_t)(2 * (kCorrT + a.nd - 1 + kCorrL) + kCorrL * kDT) * sizeof(double);
-  if (lds_corr > 65536) return hipErrorInvalidValue;
-  const int nchunk = diff_corr_chunks(a.n);
-  dim3 gr((unsigned)nchunk, a.n_mu, (a.n_phase + kCorrPG - 1) / kCorrPG);
-  k_diff_corr<<<gr, kDT, lds_corr, s>>>(a, GI, Cpart, a.q, a.s, 2, 0);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if (a.ns == 3) {
-    k_diff_corr<<<gr, kDT, lds_corr, s>>>(a, GI, Cpart, a.f, nullptr, 1, 2);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  long nc = (long)a.n_phase * a.n_mu * a.nd * a.ns;
-  k_diff_corr_reduce<<<(unsigned)((nc + kDT - 1) / kDT), kDT, 0, s>>>(a, a.n_phase * a.n_mu, a.nd, nchunk, Cpart, C);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (a.nd > 761) return hipErrorInvalidValue;  // the widest shift range the adjoint takes
+  e = corr_pb(a.n_phase) == 10 ? launch_corr_p<10>(a, GI, Cpart, C, s) : launch_corr_p<8>(a, GI, Cpart, C, s);
+  if (e != hipSuccess) return e;
   k_diff_piecegrad<<<diff_piece_blocks(a.n_piece), 256, 0, s>>>(a, C, cell_part);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   const int pw = a.n_phase < 64 ? a.n_phase : 64;
@@ -1275,13 +1614,14 @@ hipError_t launch_diff_backward(const DiffArgs &a, const ConvArgs &c, const doub
   else
     k_diff_mapgrad<2><<<gmg, 256, lds_mg, s>>>(a, C, gmaps, gfmaps);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  size_t lds_seed = (size_t)(kDT + a.nd - 1) * sizeof(double);
-  dim3 gsd((unsigned)((a.n + kDT - 1) / kDT), a.n_mu);
-  if (a.ns == 3)
-    k_diff_seedgrad<3><<<gsd, kDT, lds_seed, s>>>(a, GI, gq, gs, gf);
-  else
-    k_diff_seedgrad<2><<<gsd, kDT, lds_seed, s>>>(a, GI, gq, gs, gf);
-  return hipGetLastError();
+  switch (a.grp_r) {
+    case 4: return launch_seed_r<4>(a, GI, gq, gs, gf, s);
+    case 8: return launch_seed_r<8>(a, GI, gq, gs, gf, s);
+    case 10: return launch_seed_r<10>(a, GI, gq, gs, gf, s);
+    case 12: return launch_seed_r<12>(a, GI, gq, gs, gf, s);
+    case 16: return launch_seed_r<16>(a, GI, gq, gs, gf, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace soap

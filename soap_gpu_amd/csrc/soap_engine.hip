@@ -106,7 +106,7 @@ struct soap_ctx {
     int n_piece = 0, plan_G = 0, plan_M = 0;
     std::vector<double> plan_mu;
     double plan_lb[4] = {0, 0, 0, 0};
-    DevBuf row_m, row_t, drow, blag, mom, wts, taps, I, F, res_part, ccf, par, model, depth, bis, iters, th,
+    DevBuf row_m, row_t, drow, blag, mom, wts, taps_p, taps_r, I, F, res_part, ccf, par, model, depth, bis, iters, th,
         dth, gy, GF, GI, C, Cpart, cell_part;
     DevBuf bisd;  // [P][n_v + kBisHead]: span, loss coefficient, dspan/dtheta, dspan/dy
     DevBuf tg;    // per-call targets [3][P] (RV, FWHM, BIS span), the loss [1], the scalar gradients [5]
@@ -2156,8 +2156,10 @@ static int diff_buffers(soap_ctx *c, int nd, int ns) {
   int rc;
   if ((rc = ensure(c, d.drow, (size_t)nd * 2 * 4)) || (rc = ensure(c, d.blag, (size_t)c->n_mu * 2 * 4)) ||
       (rc = ensure(c, d.mom, (size_t)d.n_piece * diff_moments(ns) * d.P * 8)) ||
-      (rc = ensure(c, d.wts, (size_t)d.n_piece * ns * d.P * 8)) || (rc = ensure(c, d.taps, per * 8)) ||
-      (rc = ensure(c, d.C, per * 8)) || (rc = ensure(c, d.Cpart, per * diff_corr_chunks(c->n) * 8)))
+      (rc = ensure(c, d.wts, (size_t)d.n_piece * ns * d.P * 8)) ||
+      (rc = ensure(c, d.taps_p, (size_t)diff_groups(d.P) * c->n_mu * nd * ns * 16 * 8)) ||
+      (rc = ensure(c, d.taps_r, (size_t)d.P * diff_groups(c->n_mu * ns) * nd * 16 * 8)) ||
+      (rc = ensure(c, d.C, per * 8)) || (rc = ensure(c, d.Cpart, diff_corr_part(c->n, d.P, c->n_mu * ns, nd) * 8)))
     return rc;
   return SOAP_OK;
 }
@@ -2246,7 +2248,10 @@ static DiffArgs diff_args(soap_ctx *c) {
   a.wts = (double *)d.wts.p;
   a.maps = d.maps;
   a.fmaps = d.fmaps;
-  a.taps = (double *)d.taps.p;
+  a.grp_p = diff_group(d.P);
+  a.grp_r = diff_group(c->n_mu * d.ns);
+  a.taps_p = (double *)d.taps_p.p;
+  a.taps_r = (double *)d.taps_r.p;
   a.q = d.q;
   a.s = d.s;
   a.f = d.f;
@@ -3008,7 +3013,7 @@ namespace {
 std::vector<uintptr_t> dbatch_signature(const soap_ctx *c) {
   auto &d = c->diff;
   auto u = [](const void *p) { return (uintptr_t)p; };
-  return {u(d.mom.p),  u(d.wts.p),   u(d.drow.p),   u(d.blag.p),  u(d.row_m.p),  u(d.row_t.p),    u(d.taps.p),  u(d.C.p),     u(d.Cpart.p),  u(d.res_part.p), u(d.ccf.p),
+  return {u(d.mom.p),  u(d.wts.p),   u(d.drow.p),   u(d.blag.p),  u(d.row_m.p),  u(d.row_t.p),    u(d.taps_p.p), u(d.taps_r.p), u(d.C.p),     u(d.Cpart.p),  u(d.res_part.p), u(d.ccf.p),
           u(d.par.p),  u(d.model.p), u(d.depth.p),  u(d.bis.p),   u(d.iters.p),  u(d.th.p),       u(d.dth.p),
           u(d.gy.p),   u(d.GF.p),    u(d.GI.p),     u(d.cell_part.p), u(d.I.p),  u(d.F.p),        u(d.ck.p),
           u(d.cell.p), u(d.map_j.p), u(d.map_f.p),  u(d.piece.p), u(d.psum.p), u(d.brow.p), u(d.pstart.p), (uintptr_t)d.n_piece, u(d.mt_ptr.p), u(d.mt_w.p),

@@ -294,6 +294,21 @@ struct DiffPiece {
 };
 constexpr int kDiffPiece = 32;
 constexpr int diff_moments(int ns) { return ns == 3 ? 9 : 3; }
+// Rows of a contraction's group: of the sizes that the kernels have, the one that pads
+// `rows` least, the larger of equals.
+inline int diff_group(int rows) {
+  const int sizes[] = {16, 12, 10, 8, 4};
+  int best = 16, pad = 1 << 30;
+  for (int g : sizes) {
+    const int all = (rows + g - 1) / g * g;
+    if (all < pad) {
+      pad = all;
+      best = g;
+    }
+  }
+  return best;
+}
+inline int diff_groups(int rows) { return (rows + diff_group(rows) - 1) / diff_group(rows); }
 
 struct DiffArgs {
   int64_t n;
@@ -320,8 +335,11 @@ struct DiffArgs {
   double *mom;                   // [n_piece][diff_moments(ns)][P]: sums of phi, psi times 1, a, a^2 (see k_diff_moments)
   double *wts;                   // [n_piece][ns][P]: the tap weights of the sets
   const double *maps, *fmaps;    // spot / facula filling factors [P][M][M] (fmaps null when ns == 2)
-  double *taps;                  // [P][n_mu][nd][ns]
-  int32_t *krange;               // [P][n_mu][2]
+  // the taps twice, for the two contractions that read them: 16 lanes of a row hold the
+  // taps of a group of grp_p phases (taps_p [group][n_mu][nd][ns][16]) or of grp_r
+  // (bin, set) rows (taps_r [P][group][nd][16])
+  int32_t grp_p, grp_r;
+  double *taps_p, *taps_r;
   const double *q, *s, *f;       // quiet / spot / facula seed rows [n_mu][n] (f null when ns == 2)
   double *I, *F;                 // [P][n]
 };
@@ -557,7 +575,8 @@ constexpr int kMaxVDiff = 1024;
 hipError_t launch_diff_bis(const double *v, int n_v, const double *ccf, const double *theta, int n_ccf, double *bisd,
                            hipStream_t s);
 // chunks of the lag-correlation pass (Cpart holds [P][n_mu][chunks][nd][ns])
-int diff_corr_chunks(int64_t n);
+// doubles of the correlations' chunk partials
+size_t diff_corr_part(int64_t n, int n_phase, int rows, int nd);
 hipError_t launch_ccf_sum(const double *part, int nc, int n_spec, int n_v, double *ccf, hipStream_t s);
 // device-side loss of the differentiable model: per phase the residual partials
 // (res_blocks per phase, in order), the RV / FWHM terms and, when w_bis != 0, the
