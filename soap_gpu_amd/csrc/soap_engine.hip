@@ -1803,7 +1803,7 @@ static int ccf_impl(soap_ctx *c, bool norm) {
   if (!c->mask_built && (rc = build_mask(c))) return rc;
   int n_spec = (c->P + 1) * 3;
   if ((rc = dalloc(c, &c->d_ccf, (size_t)n_spec * c->n_v)) ||
-      (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines) * n_spec * c->n_v * 8)))
+      (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines, n_spec) * n_spec * c->n_v * 8)))
     return rc;
   if (norm) {
     NormCcfArgs a{};
@@ -1834,7 +1834,7 @@ static int ccf_impl(soap_ctx *c, bool norm) {
   }
   {
     StageTimer tm(c, ST_CCF_REDUCE);
-    HIPCHK(c, launch_ccf_reduce((const double *)c->ccf_part.p, ccf_chunks(c->n_lines), n_spec, c->n_v, c->d_appod,
+    HIPCHK(c, launch_ccf_reduce((const double *)c->ccf_part.p, ccf_chunks(c->n_lines, n_spec), n_spec, c->n_v, c->d_appod,
                                 (const double *)c->mm.p, (const double *)c->wsum.p, c->d_ccf, c->stream));
   }
   c->have_ccf = true;
@@ -2154,7 +2154,8 @@ static int diff_buffers(soap_ctx *c, int nd, int ns) {
   auto &d = c->diff;
   const size_t per = (size_t)d.P * c->n_mu * nd * ns;
   int rc;
-  if ((rc = ensure(c, d.drow, (size_t)nd * 2 * 4)) || (rc = ensure(c, d.blag, (size_t)c->n_mu * 2 * 4)) ||
+  if ((rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines, d.P) * d.P * c->n_v * 8)) ||
+      (rc = ensure(c, d.drow, (size_t)nd * 2 * 4)) || (rc = ensure(c, d.blag, (size_t)c->n_mu * 2 * 4)) ||
       (rc = ensure(c, d.mom, (size_t)d.n_piece * diff_moments(ns) * d.P * 8)) ||
       (rc = ensure(c, d.wts, (size_t)d.n_piece * ns * d.P * 8)) ||
       (rc = ensure(c, d.taps_p, (size_t)diff_groups(d.P) * c->n_mu * nd * ns * 16 * 8)) ||
@@ -2186,7 +2187,7 @@ int soap_diff_setup(soap_ctx *c, int32_t grid, int32_t n_phase, int32_t map_res,
       (rc = ensure(c, d.gy, (size_t)n_phase * c->n_v * 8)) ||
       (rc = ensure(c, d.bisd, (size_t)n_phase * (c->n_v + kBisHead) * 8)) ||
       (rc = ensure(c, d.tg, ((size_t)n_phase * 3 + 1 + kDiffScalars) * 8)) ||
-      (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines) * n_phase * c->n_v * 8)))
+      (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines, n_phase) * n_phase * c->n_v * 8)))
     return rc;
   int wid = conv_window(c->wave, sigma_ms);
   if (wid < 1 || 2 * (int64_t)wid + 2 >= c->n) return fail(c, SOAP_ERR_ARG, "diff_setup: window %d vs %lld pixels", wid, (long long)c->n);
@@ -2331,7 +2332,7 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
   {
     StageTimer tm(c, ST_CCF);
     HIPCHK(c, ctx_ccf(c, (const double *)d.F.p, d.P, (double *)c->ccf_part.p, c->stream));
-    HIPCHK(c, launch_ccf_sum((const double *)c->ccf_part.p, ccf_chunks(c->n_lines), d.P, c->n_v, (double *)d.ccf.p,
+    HIPCHK(c, launch_ccf_sum((const double *)c->ccf_part.p, ccf_chunks(c->n_lines, d.P), d.P, c->n_v, (double *)d.ccf.p,
                              c->stream));
   }
   {
@@ -2680,8 +2681,8 @@ int batch_build(soap_batch *b) {
     nm[i] = NormJob{c->n, nbx, (const double *)c->mm.p, c->d_lraw, c->d_lower};
     w[BS_NORM][i] = nbx * n_spec;
     // CCF + fit
-    int nc = ccf_chunks(c->n_lines);
-    cc[i] = CcfJob{c->d_lraw, c->n, c->trim, c->n - 2 * (int64_t)c->trim, n_spec, c->n_lines, c->n_v, nc,
+    int nc = ccf_chunks(c->n_lines, n_spec);
+    cc[i] = CcfJob{c->d_lraw, c->n, c->trim, c->n - 2 * (int64_t)c->trim, n_spec, c->n_lines, c->n_v, nc, ccf_lines(c->n_lines, n_spec),
                    (const int32_t *)c->m_start.p, (const uint32_t *)c->m_alive.p, (const double2 *)c->m_val.p,
                    c->d_w_sorted, (const int2 *)c->fp.p, c->ccf_cap, (double *)c->ccf_part.p};
     lds_ccf = std::max(lds_ccf, ccf_lds_bytes(c->ccf_cap));
@@ -3103,7 +3104,7 @@ hipError_t dbatch_enqueue_one(soap_diffbatch::Item &it, hipStream_t st, bool adj
     hipError_t e = launch_diff_forward_spectra(a, ca, it.target, c->trim, (double *)d.res_part.p, &rb, st);
     if (e == hipSuccess) e = ctx_ccf(c, (const double *)d.F.p, d.P, (double *)c->ccf_part.p, st);
     if (e == hipSuccess)
-      e = launch_ccf_sum((const double *)c->ccf_part.p, ccf_chunks(c->n_lines), d.P, c->n_v, (double *)d.ccf.p,
+      e = launch_ccf_sum((const double *)c->ccf_part.p, ccf_chunks(c->n_lines, d.P), d.P, c->n_v, (double *)d.ccf.p,
                          st);
     if (e == hipSuccess)
       e = launch_fit(c->d_vgrid, c->n_v, (const double *)d.ccf.p, nullptr, d.P, (double *)d.par.p, (double *)d.model.p,

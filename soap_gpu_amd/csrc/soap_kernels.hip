@@ -2374,7 +2374,7 @@ hipError_t launch_mask_overwrite(const int32_t *sorted, int n_lines, int n_v, in
   return hipGetLastError();
 }
 
-// calculate_CCF_2 (CCF_func.py:27-36) on the sparse mask.  Block = (chunk of
+// calculate_CCF_2 (CCF_func.py:27-36) on the sparse mask.  Block = (chunk of up to
 // kCcfLines lines in wavelength order, chunk of kCcfSpec spectra); thread = one
 // velocity, summing its lines in order for all spectra of the chunk (each mask
 // entry is read once per block).  Each line's pixel footprint is staged in LDS
@@ -2390,6 +2390,7 @@ hipError_t launch_mask_overwrite(const int32_t *sorted, int n_lines, int n_v, in
 // The CCF therefore runs on x, and spec_norm does not have to finish before it:
 // the two share one launch (k_norm_ccf).
 constexpr int kCcfLines = 32;
+constexpr int kCcfBlocks = 512;
 constexpr int kCcfSpec = 8;
 constexpr int kCcfLdsCap = 512;  // LDS segment of the footprint form: 8 spectra x 512 pixels = 32 KiB
 
@@ -2426,11 +2427,19 @@ hipError_t launch_mask_footprint(int n_lines, int n_v, int64_t n_t, const int32_
 // n_v) adds its window's pixels from LDS, in pixel order.  A footprint longer
 // than cap pixels goes through in segments of cap (a window that straddles two
 // takes its low pixels from the first, so the order of the terms is kept).
-// lds: kCcfSpec * cap doubles.
+// AHEAD: the next segment's first blockDim.x pixels and, at a line's last segment, the
+// next line's mask entry are loaded while this segment's windows are summed.  A block
+// walks its lines in turn, and where the launch is too small for other blocks to hide
+// them one round trip to memory per line (2.3 us) is its time (200 lines, 78 spectra: 75
+// us per launch, 18 with these loads and two lines per block); where blocks fill the CUs
+// the registers cost more waves than the loads save (series of 303 spectra: 0.90 -> 1.17
+// ms), so the large launches and the batched one keep to the plain form.
+// lines: lines per chunk (ccf_lines); lds: kCcfSpec * cap doubles.
+template <bool AHEAD>
 __device__ __forceinline__ void ccf_lds_body(const double *spec_, int64_t spec_stride, int64_t trim, int n_spec,
                                              int n_lines, int n_v, int64_t n_t, const int32_t *m_start_,
                                              const uint32_t *m_pk_, const double2 *m_wv_, const double *w_sorted_,
-                                             const int2 *fp_, int cap, double *part_, int bx_, int by_,
+                                             const int2 *fp_, int cap, double *part_, int lines, int bx_, int by_,
                                              double *lds) {
   const GLOBAL double *spec = gl(spec_), *w_sorted = gl(w_sorted_);
   const GLOBAL int32_t *m_start = gl(m_start_);
@@ -2441,20 +2450,29 @@ __device__ __forceinline__ void ccf_lds_body(const double *spec_, int64_t spec_s
   const int chunk = bx_;
   const int s0 = by_ * kCcfSpec;
   const int ns = min(kCcfSpec, n_spec - s0);
-  const int q0 = chunk * kCcfLines, q1 = min(n_lines, q0 + kCcfLines);
+  const int q0 = chunk * lines, q1 = min(n_lines, q0 + lines);
+  const int iv = threadIdx.x, nt = blockDim.x;
+  const bool act = iv < n_v;
   const GLOBAL double *S[kCcfSpec];
 #pragma unroll
   for (int k = 0; k < kCcfSpec; k++) S[k] = spec + (long)(s0 + (k < ns ? k : 0)) * spec_stride + trim;
-  const int iv = threadIdx.x;
-  const bool act = iv < n_v;
-  double acc[kCcfSpec];
+  double acc[kCcfSpec], v[kCcfSpec];
 #pragma unroll
   for (int k = 0; k < kCcfSpec; k++) acc[k] = 0.0;
-  for (int q = q0; q < q1; q++) {
-    // this line's mask entry, loaded before the staging so that the two overlap
-    int st = 0;
-    uint32_t pk = 0;
-    double wx = 0.0, wy = 0.0;
+  auto load = [&](long base, int seg, int j) {
+#pragma unroll
+    for (int k = 0; k < kCcfSpec; k++) v[k] = (j < seg && k < ns) ? S[k][base + j] : 0.0;
+  };
+  auto store = [&](int seg, int j) {
+    if (j < seg) {
+#pragma unroll
+      for (int k = 0; k < kCcfSpec; k++) lds[k * cap + j] = v[k];
+    }
+  };
+  int st = 0;
+  uint32_t pk = 0;
+  double wx = 0.0, wy = 0.0;
+  auto entry = [&](int q) {  // the velocity's mask entry of line q
     if (act) {
       const long e = (long)q * n_v + iv;
       st = m_start[e];
@@ -2462,35 +2480,60 @@ __device__ __forceinline__ void ccf_lds_body(const double *spec_, int64_t spec_s
       wx = m_wv[2 * e];
       wy = m_wv[2 * e + 1];
     }
-    const double w = w_sorted[q];
-    const int f_lo = fp[2 * q], f_len = fp[2 * q + 1];
+  };
+  int f_lo = fp[2 * q0], f_len = fp[2 * q0 + 1];
+  if (AHEAD) {
+    entry(q0);
+    load(f_lo, min(cap, f_len), iv);
+  }
+  for (int q = q0; q < q1; q++) {
+    if (!AHEAD) {
+      // this line's mask entry, loaded before the staging so that the two overlap
+      entry(q);
+      f_lo = fp[2 * q];
+      f_len = fp[2 * q + 1];
+    }
+    const int c_st = st;
+    const uint32_t c_pk = pk;
+    const double c_wx = wx, c_wy = wy, w = w_sorted[q];
+    const bool more = AHEAD && q + 1 < q1;
+    const int n_lo = more ? fp[2 * q + 2] : 0, n_len = more ? fp[2 * q + 3] : 0;
+    if (more && f_len == 0) {  // nothing of this line in the spectrum: only the next one's loads
+      entry(q + 1);
+      load(n_lo, min(cap, n_len), iv);
+    }
     for (int g0 = 0; g0 < f_len; g0 += cap) {
       const int seg = min(cap, f_len - g0);
       const long base = (long)f_lo + g0;
       __syncthreads();  // the previous segment's readers are done with the buffer
-      for (int j0 = 0; j0 < seg; j0 += blockDim.x) {
-        const int j = j0 + threadIdx.x;
-        double v[kCcfSpec];
-#pragma unroll
-        for (int k = 0; k < kCcfSpec; k++) v[k] = (j < seg && k < ns) ? S[k][base + j] : 0.0;
-        if (j < seg) {
-#pragma unroll
-          for (int k = 0; k < kCcfSpec; k++) lds[k * cap + j] = v[k];
-        }
+      if (AHEAD) store(seg, iv);
+      for (int j0 = AHEAD ? nt : 0; j0 < seg; j0 += nt) {
+        load(base, seg, j0 + iv);
+        store(seg, j0 + iv);
+      }
+      if (AHEAD && g0 + cap < f_len) {
+        load(base + cap, min(cap, f_len - g0 - cap), iv);
+      } else if (more) {
+        entry(q + 1);
+        load(n_lo, min(cap, n_len), iv);
       }
       __syncthreads();
       if (act) {
-        const int ln = (int)(pk & 0xffu);
-        const uint32_t al = pk >> 8;
+        const int ln = (int)(c_pk & 0xffu);
+        const uint32_t al = c_pk >> 8;
         for (int b = 0; b < ln; b++) {
-          const long pp = st + b;
+          const long pp = c_st + b;
           if (!((al >> b) & 1u) || pp < 0 || pp >= n_t || pp < base || pp >= base + seg) continue;
-          const double val = (b == ln - 1) ? wy : ((b == 0) ? wx : w);
+          const double val = (b == ln - 1) ? c_wy : ((b == 0) ? c_wx : w);
           const double *L = lds + (pp - base);
 #pragma unroll
           for (int k = 0; k < kCcfSpec; k++) acc[k] = fma(L[k * cap], val, acc[k]);
         }
       }
+    }
+    if (AHEAD) {
+      f_lo = n_lo;
+      f_len = n_len;
     }
   }
   if (act) {
@@ -2500,11 +2543,12 @@ __device__ __forceinline__ void ccf_lds_body(const double *spec_, int64_t spec_s
   }
 }
 
+template <bool AHEAD>
 __global__ void k_ccf_lds(const double *spec, int64_t spec_stride, int64_t trim, int n_spec, int n_lines, int n_v,
                           int64_t n_t, const int32_t *m_start, const uint32_t *m_pk, const double2 *m_wv,
-                          const double *w_sorted, const int2 *fp, int cap, double *part) {
+                          const double *w_sorted, const int2 *fp, int cap, double *part, int lines) {
   extern __shared__ double ccf_lds[];
-  ccf_lds_body(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t, m_start, m_pk, m_wv, w_sorted, fp, cap, part,
+  ccf_lds_body<AHEAD>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t, m_start, m_pk, m_wv, w_sorted, fp, cap, part, lines,
                blockIdx.x, blockIdx.y, ccf_lds);
 }
 
@@ -2517,11 +2561,16 @@ hipError_t launch_ccf_lds(const double *spec, int64_t spec_stride, int64_t trim,
                           const double *w_sorted, const int2 *fp, int cap, double *part, hipStream_t s) {
   if (n_spec == 0) return hipSuccess;
   if (n_v > 1024 || cap < 1 || cap > kCcfLdsCap) return hipErrorInvalidValue;
-  int nc = ccf_chunks(n_lines);
+  int nc = ccf_chunks(n_lines, n_spec);
   int threads = ((n_v + 63) / 64) * 64;
   dim3 grid(nc, (n_spec + kCcfSpec - 1) / kCcfSpec);
-  k_ccf_lds<<<grid, threads, ccf_lds_bytes(cap), s>>>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t, m_start,
-                                                       m_pk, m_wv, w_sorted, fp, cap, part);
+  const int lines = ccf_lines(n_lines, n_spec);
+  if (lines < kCcfLines)
+    k_ccf_lds<true><<<grid, threads, ccf_lds_bytes(cap), s>>>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t,
+                                                              m_start, m_pk, m_wv, w_sorted, fp, cap, part, lines);
+  else
+    k_ccf_lds<false><<<grid, threads, ccf_lds_bytes(cap), s>>>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t,
+                                                               m_start, m_pk, m_wv, w_sorted, fp, cap, part, lines);
   return hipGetLastError();
 }
 
@@ -2622,6 +2671,7 @@ hipError_t launch_mask_wsum(int n_lines, int n_v, int64_t n_t, const int32_t *m_
 // place moves with the group and eight CCF blocks in a row meet all eight.  blockDim.x is the
 // CCF's thread count (velocities rounded up to a wave); a norm block covers
 // kNormPer * blockDim.x pixels of one spectrum.
+template <bool AHEAD>
 __device__ __forceinline__ void norm_ccf_body(const NormCcfArgs &a, long b, double *ccf_lds) {
   const long grp = (long)a.ratio + 1;
   const long mixed = (long)a.n_ccf * grp;
@@ -2638,15 +2688,16 @@ __device__ __forceinline__ void norm_ccf_body(const NormCcfArgs &a, long b, doub
     ni = (long)a.n_ccf * a.ratio + (b - mixed);
   }
   if (ci >= 0)
-    ccf_lds_body(a.raw, a.n, a.trim, a.n_spec, a.n_lines, a.n_v, a.n_t, a.m_start, a.m_pk, a.m_wv, a.w_sorted, a.fp,
-                 a.cap, a.part, (int)(ci % a.nc), (int)(ci / a.nc), ccf_lds);
+    ccf_lds_body<AHEAD>(a.raw, a.n, a.trim, a.n_spec, a.n_lines, a.n_v, a.n_t, a.m_start, a.m_pk, a.m_wv, a.w_sorted, a.fp,
+                 a.cap, a.part, a.lines, (int)(ci % a.nc), (int)(ci / a.nc), ccf_lds);
   else if (ni < a.n_norm)
     norm_body(a.n, a.mm, a.raw, a.out, (int)(ni % a.nbx), (int)(ni / a.nbx), blockDim.x);
 }
 
+template <bool AHEAD>
 __global__ void k_norm_ccf(NormCcfArgs a) {
   extern __shared__ double ccf_lds[];
-  norm_ccf_body(a, blockIdx.x, ccf_lds);
+  norm_ccf_body<AHEAD>(a, blockIdx.x, ccf_lds);
 }
 
 hipError_t launch_norm_ccf(NormCcfArgs a, hipStream_t s) {
@@ -2654,18 +2705,33 @@ hipError_t launch_norm_ccf(NormCcfArgs a, hipStream_t s) {
   if (a.n_v > 1024 || (((uintptr_t)a.raw ^ (uintptr_t)a.out) & 15)) return hipErrorInvalidValue;
   if (a.cap < 1 || a.cap > kCcfLdsCap) return hipErrorInvalidValue;
   const int threads = ((a.n_v + 63) / 64) * 64;
-  a.nc = ccf_chunks(a.n_lines);
+  a.nc = ccf_chunks(a.n_lines, a.n_spec);
+  a.lines = ccf_lines(a.n_lines, a.n_spec);
   a.n_ccf = a.nc * ((a.n_spec + kCcfSpec - 1) / kCcfSpec);
   a.nbx = (int)((a.n + (int64_t)threads * kNormPer - 1) / ((int64_t)threads * kNormPer));
   a.n_norm = a.nbx * a.n_spec;
   a.ratio = a.n_ccf > 0 ? a.n_norm / a.n_ccf : 0;
   const long blocks = (long)a.n_ccf + a.n_norm;
   if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-  k_norm_ccf<<<(unsigned)blocks, threads, ccf_lds_bytes(a.cap), s>>>(a);
+  if (a.lines < kCcfLines)
+    k_norm_ccf<true><<<(unsigned)blocks, threads, ccf_lds_bytes(a.cap), s>>>(a);
+  else
+    k_norm_ccf<false><<<(unsigned)blocks, threads, ccf_lds_bytes(a.cap), s>>>(a);
   return hipGetLastError();
 }
 
-int ccf_chunks(int n_lines) { return (n_lines + kCcfLines - 1) / kCcfLines; }
+// Lines per chunk: fewer where 32 would leave CUs without a block (the walk over a
+// block's lines is then the launch's time), down to 2.
+int ccf_lines(int n_lines, int n_spec) {
+  const long groups = (n_spec + kCcfSpec - 1) / kCcfSpec;
+  int l = kCcfLines;
+  while (l > 2 && (n_lines + l - 1) / l * groups < kCcfBlocks) l >>= 1;
+  return l;
+}
+int ccf_chunks(int n_lines, int n_spec) {
+  const int l = ccf_lines(n_lines, n_spec);
+  return (n_lines + l - 1) / l;
+}
 
 hipError_t launch_ccf_reduce(const double *part, int nc, int n_spec, int n_v, const double *appod, const double *mm,
                              const double *wsum, double *ccf, hipStream_t s) {
@@ -3150,8 +3216,8 @@ template <bool P>
 __global__ __launch_bounds__(1024) void kb_ccf(SOAP_BATCH_ARGS(CcfJob)) {
   extern __shared__ double ccf_lds[];
   batch_loop<P>(jobs, prefix, n_inst, total, [&](const CcfJob &j, int local) {
-    ccf_lds_body(j.spec, j.stride, j.trim, j.n_spec, j.n_lines, j.n_v, j.n_t, j.m_start, j.m_pk, j.m_wv, j.w_sorted,
-                 j.fp, j.cap, j.part, local % j.nc, local / j.nc, ccf_lds);
+    ccf_lds_body<false>(j.spec, j.stride, j.trim, j.n_spec, j.n_lines, j.n_v, j.n_t, j.m_start, j.m_pk, j.m_wv, j.w_sorted,
+                 j.fp, j.cap, j.part, j.lines, local % j.nc, local / j.nc, ccf_lds);
   });
 }
 
