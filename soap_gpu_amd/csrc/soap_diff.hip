@@ -1466,7 +1466,7 @@ __global__ __launch_bounds__(kDT) void k_diff_loss(int n_phase, int res_blocks, 
                                                    const double *bis_t, double w_spec, double w_rv, double w_fw,
                                                    double w_bis, double *bisd, int n_v, const double *prm,
                                                    double vsini_max, double n_cells, double lbmax, double *loss,
-                                                   double *dth) {
+                                                   double *dth, double *series) {
   extern __shared__ double term[];  // [n_phase]
   for (int p = threadIdx.x; p < n_phase; p += blockDim.x) {
     // the residual partials in order, kResU loads ahead of their adds
@@ -1495,6 +1495,11 @@ __global__ __launch_bounds__(kDT) void k_diff_loss(int n_phase, int res_blocks, 
     }
     term[p] = t;
     for (int q = 0; q < 4; q++) dth[p * 4 + q] = d4[q];
+    if (series) {  // RV, FWHM and span of every phase in one piece, for the host
+      series[p] = theta[p * 4 + 2];
+      series[n_phase + p] = theta[p * 4 + 3];
+      series[2 * n_phase + p] = bisd[(long)p * (n_v + kBisHead)];
+    }
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1542,12 +1547,13 @@ __global__ __launch_bounds__(kDT) void k_diff_grad(int n_blocks, const double *c
 hipError_t launch_diff_loss(int n_phase, int res_blocks, const double *res_part, const double *theta,
                             const double *rv_t, const double *fw_t, const double *bis_t, double w_spec, double w_rv,
                             double w_fw, double w_bis, double *bisd, int n_v, const double *prm, double vsini_max,
-                            double n_cells, double lbmax, double *loss, double *dth, hipStream_t s) {
+                            double n_cells, double lbmax, double *loss, double *dth, double *series,
+                            hipStream_t s) {
   if (n_phase < 1 || (size_t)n_phase * 8 > 65536) return hipErrorInvalidValue;
-  if (w_bis != 0.0 && (!bisd || !bis_t)) return hipErrorInvalidValue;
+  if ((w_bis != 0.0 && (!bisd || !bis_t)) || (series && !bisd)) return hipErrorInvalidValue;
   k_diff_loss<<<1, kDT, (size_t)n_phase * 8, s>>>(n_phase, res_blocks, res_part, theta, rv_t, fw_t, bis_t, w_spec,
                                                   w_rv, w_fw, w_bis, bisd, n_v, prm, vsini_max, n_cells, lbmax, loss,
-                                                  dth);
+                                                  dth, series);
   return hipGetLastError();
 }
 

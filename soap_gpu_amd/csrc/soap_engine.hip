@@ -11,6 +11,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -109,7 +110,7 @@ struct soap_ctx {
     DevBuf row_m, row_t, drow, blag, mom, wts, taps_p, taps_r, I, F, res_part, ccf, par, model, depth, bis, iters, th,
         dth, gy, GF, GI, C, Cpart, cell_part;
     DevBuf bisd;  // [P][n_v + kBisHead]: span, loss coefficient, dspan/dtheta, dspan/dy
-    DevBuf tg;    // per-call targets [3][P] (RV, FWHM, BIS span), the loss [1], the scalar gradients [5]
+    DevBuf tg;    // per-call targets [3][P] (RV, FWHM, BIS span), the loss [1], the scalar gradients [5], the series [3][P]
     DevBuf mt_ptr, mt_w, mt_col, mt_val;  // the mask in sliced pixel-major form (adjoint of the CCF)
     bool mt_ready = false;
   } diff;
@@ -153,7 +154,9 @@ struct soap_ctx {
   bool have_mask = false, mask_built = false;
   double *d_ccf = nullptr;  // [(P+1)*3][n_v]
   bool have_ccf = false;
-  DevBuf f_par, f_model, f_depth, f_bis, f_iter;
+  DevBuf f_all;  // the fit's outputs in one piece: parameters, models, depths, bisectors, iterations
+  DevBuf f_par, f_model, f_depth, f_bis, f_iter;  // their places in it
+  DevBuf fit_ws;  // host-CCF fits: inputs and outputs in one piece
   bool have_fit = false;
   // timing
   bool timing = false;
@@ -219,6 +222,114 @@ static int ensure(soap_ctx *c, DevBuf &b, size_t bytes) {
 
 static void dfree(void *p) {
   if (p) hipFree(p);
+}
+
+// Pinned staging for the calls that move data between host and device.  A copy to
+// pageable memory costs the runtime a staged copy and a wait of its own (20-25 us each);
+// through a pinned buffer a call's results come in one copy and one wait.  The buffers
+// belong to the process (pinning one takes 0.3 ms): a call takes one and gives it back
+// before it returns, so contexts on any threads share them; at most kPinSlots of at most
+// kPinMax bytes, freed with the last context.  A call that finds none copies directly.
+constexpr size_t kPinMax = (size_t)8 << 20, kPinMin = (size_t)1 << 20;
+constexpr int kPinSlots = 8;
+struct PinPool {
+  struct Slot {
+    char *p;
+    size_t bytes;
+  };
+  std::mutex lock;
+  std::vector<Slot> idle;
+  int slots = 0, contexts = 0;
+  PinPool() { idle.reserve(kPinSlots); }
+  static PinPool &get() {
+    static PinPool *pool = new PinPool();  // never destroyed: contexts may outlive static objects
+    return *pool;
+  }
+  void context(int change) {
+    std::lock_guard<std::mutex> g(lock);
+    contexts += change;
+    if (contexts > 0) return;
+    for (Slot &s : idle) hipHostFree(s.p);
+    slots -= (int)idle.size();
+    idle.clear();
+  }
+  Slot take(size_t bytes) {
+    if (bytes > kPinMax) return {nullptr, 0};
+    std::lock_guard<std::mutex> g(lock);
+    size_t best = idle.size();
+    for (size_t i = 0; i < idle.size(); i++)
+      if (idle[i].bytes >= bytes && (best == idle.size() || idle[i].bytes < idle[best].bytes)) best = i;
+    if (best < idle.size()) {
+      Slot s = idle[best];
+      idle.erase(idle.begin() + best);
+      return s;
+    }
+    if (slots >= kPinSlots) {  // a larger one in the place of an idle one
+      if (idle.empty()) return {nullptr, 0};
+      hipHostFree(idle.back().p);
+      idle.pop_back();
+      slots--;
+    }
+    Slot s{nullptr, kPinMin};
+    while (s.bytes < bytes) s.bytes <<= 1;
+    if (hipHostMalloc((void **)&s.p, s.bytes, hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      return {nullptr, 0};
+    }
+    slots++;
+    return s;
+  }
+  void give(Slot s) {
+    if (!s.p) return;
+    std::lock_guard<std::mutex> g(lock);
+    idle.push_back(s);
+  }
+};
+struct Pinned {
+  PinPool::Slot slot;
+  explicit Pinned(size_t bytes) : slot(PinPool::get().take(bytes)) {}
+  ~Pinned() { PinPool::get().give(slot); }
+  Pinned(const Pinned &) = delete;
+  Pinned &operator=(const Pinned &) = delete;
+  char *p() const { return slot.p; }
+};
+
+// Device ranges to host arrays (null: skipped), after the stream's work; waits for them.
+// Ranges that lie together (gaps included not much more than they hold) come in one copy.
+// have: a staging buffer that the call holds already, large enough for them.
+struct FetchPart {
+  void *host;
+  const void *dev;
+  size_t bytes;
+};
+static hipError_t fetch(soap_ctx *c, std::initializer_list<FetchPart> parts, const Pinned *have = nullptr) {
+  uintptr_t lo = UINTPTR_MAX, hi = 0;
+  size_t sum = 0;
+  for (const FetchPart &p : parts)
+    if (p.host && p.bytes) {
+      lo = std::min(lo, (uintptr_t)p.dev);
+      hi = std::max(hi, (uintptr_t)p.dev + p.bytes);
+      sum += p.bytes;
+    }
+  if (!sum) return hipStreamSynchronize(c->stream);
+  const size_t span = hi - lo;
+  const bool together = span <= sum + 4096;
+  Pinned own(together && !have ? span : kPinMax + 1);
+  char *pin = !together ? nullptr : have ? have->p() : own.p();
+  hipError_t e = hipSuccess;
+  if (pin) {
+    e = hipMemcpyAsync(pin, (const void *)lo, span, hipMemcpyDeviceToHost, c->stream);
+  } else {
+    for (const FetchPart &p : parts)
+      if (p.host && p.bytes && e == hipSuccess)
+        e = hipMemcpyAsync(p.host, p.dev, p.bytes, hipMemcpyDeviceToHost, c->stream);
+  }
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = es;
+  if (pin && e == hipSuccess)
+    for (const FetchPart &p : parts)
+      if (p.host && p.bytes) memcpy(p.host, pin + ((uintptr_t)p.dev - lo), p.bytes);
+  return e;
 }
 
 static void dfree_c(soap_ctx *c, void *p) {
@@ -387,6 +498,7 @@ int soap_ctx_create(int device, soap_ctx **out) {
     delete c;
     return SOAP_ERR_HIP;
   }
+  PinPool::get().context(1);
   *out = c;
   return SOAP_OK;
 }
@@ -401,6 +513,7 @@ void soap_ctx_destroy(soap_ctx *c) {
   // (caller-owned cube pointers are not recorded and are not freed)
   for (auto &kv : c->caps) hipFree(kv.first);
   c->caps.clear();
+  PinPool::get().context(-1);
   if (c->aux) hipStreamDestroy(c->aux);
   if (c->ev_fork) hipEventDestroy(c->ev_fork);
   if (c->ev_join) hipEventDestroy(c->ev_join);
@@ -881,8 +994,7 @@ int soap_get_quiet(soap_ctx *c, int which, double *out) {
   if (!c || !out || which < 0 || which > 1) return fail(c, SOAP_ERR_ARG, "get_quiet: bad arguments");
   if (!c->have_quiet) return fail(c, SOAP_ERR_STATE, "get_quiet: no quiet star");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipMemcpyAsync(out, c->d_quiet + (size_t)which * c->n, c->n * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, fetch(c, {{out, c->d_quiet + (size_t)which * c->n, (size_t)c->n * 8}}));
   return SOAP_OK;
 }
 
@@ -1341,12 +1453,9 @@ int soap_get_raw(soap_ctx *c, int32_t phase, double *flux, double *bconv, double
   if (!c || phase < 0 || phase >= c->P) return fail(c, SOAP_ERR_ARG, "get_raw: bad phase");
   if (!c->have_raw) return fail(c, SOAP_ERR_STATE, "get_raw: run integrate first");
   HIPCHK(c, hipSetDevice(c->device));
-  double *outs[3] = {flux, bconv, tot};
-  for (int t = 0; t < 3; t++)
-    if (outs[t])
-      HIPCHK(c, hipMemcpyAsync(outs[t], c->d_raw + ((size_t)phase * 3 + t) * c->n, c->n * 8, hipMemcpyDeviceToHost,
-                               c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  const double *r = c->d_raw + (size_t)phase * 3 * c->n;
+  const size_t b = (size_t)c->n * 8;
+  HIPCHK(c, fetch(c, {{flux, r, b}, {bconv, r + c->n, b}, {tot, r + 2 * c->n, b}}));
   return SOAP_OK;
 }
 
@@ -1569,8 +1678,7 @@ int soap_get_lower(soap_ctx *c, int32_t phase, int type, double *out) {
   if (!c->have_lower) return fail(c, SOAP_ERR_STATE, "get_lower: run resolution first");
   HIPCHK(c, hipSetDevice(c->device));
   int frame = phase < 0 ? c->P : phase;
-  HIPCHK(c, hipMemcpyAsync(out, c->d_lower + ((size_t)frame * 3 + type) * c->n, c->n * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, fetch(c, {{out, c->d_lower + ((size_t)frame * 3 + type) * c->n, (size_t)c->n * 8}}));
   return SOAP_OK;
 }
 
@@ -1579,8 +1687,7 @@ int soap_get_norm(soap_ctx *c, int32_t phase, int type, double *minmax2) {
   if (!c->have_lower) return fail(c, SOAP_ERR_STATE, "get_norm: run resolution first");
   HIPCHK(c, hipSetDevice(c->device));
   int sp = (phase >= 0 ? phase : c->P) * 3 + type;
-  HIPCHK(c, hipMemcpyAsync(minmax2, (double *)c->mm.p + sp * 2, 16, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, fetch(c, {{minmax2, (double *)c->mm.p + sp * 2, 16}}));
   return SOAP_OK;
 }
 
@@ -1848,17 +1955,20 @@ int soap_get_ccf(soap_ctx *c, double *out) {
   if (!c || !out) return SOAP_ERR_ARG;
   if (!c->have_ccf) return fail(c, SOAP_ERR_STATE, "get_ccf: run ccf first");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipMemcpyAsync(out, c->d_ccf, (size_t)(c->P + 1) * 3 * c->n_v * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, fetch(c, {{out, c->d_ccf, (size_t)(c->P + 1) * 3 * c->n_v * 8}}));
   return SOAP_OK;
 }
 
 static int ensure_fit(soap_ctx *c, int n_ccf, int n_v) {
-  int rc;
-  if ((rc = ensure(c, c->f_par, (size_t)n_ccf * 5 * 8)) || (rc = ensure(c, c->f_model, (size_t)n_ccf * n_v * 8)) ||
-      (rc = ensure(c, c->f_depth, (size_t)n_ccf * 91 * 8)) || (rc = ensure(c, c->f_bis, (size_t)n_ccf * 91 * 8)) ||
-      (rc = ensure(c, c->f_iter, (size_t)n_ccf * 4)))
-    return rc;
+  const size_t n = (size_t)n_ccf;
+  int rc = ensure(c, c->f_all, n * (5 + n_v + 2 * 91) * 8 + n * 4);
+  if (rc) return rc;
+  double *p = (double *)c->f_all.p;
+  c->f_par.p = p;
+  c->f_model.p = p + n * 5;
+  c->f_depth.p = p + n * (5 + n_v);
+  c->f_bis.p = p + n * (5 + n_v + 91);
+  c->f_iter.p = p + n * (5 + n_v + 2 * 91);
   return SOAP_OK;
 }
 
@@ -1883,11 +1993,10 @@ int soap_get_fit(soap_ctx *c, double *par, double *model, double *depth, double 
   if (!c->have_fit) return fail(c, SOAP_ERR_STATE, "get_fit: run fit first");
   HIPCHK(c, hipSetDevice(c->device));
   size_t n_ccf = (size_t)(c->P + 1) * 3;
-  if (par) HIPCHK(c, hipMemcpyAsync(par, c->f_par.p, n_ccf * 5 * 8, hipMemcpyDeviceToHost, c->stream));
-  if (model) HIPCHK(c, hipMemcpyAsync(model, c->f_model.p, n_ccf * c->n_v * 8, hipMemcpyDeviceToHost, c->stream));
-  if (depth) HIPCHK(c, hipMemcpyAsync(depth, c->f_depth.p, n_ccf * 91 * 8, hipMemcpyDeviceToHost, c->stream));
-  if (bis) HIPCHK(c, hipMemcpyAsync(bis, c->f_bis.p, n_ccf * 91 * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, fetch(c, {{par, c->f_par.p, n_ccf * 5 * 8},
+                      {model, c->f_model.p, n_ccf * c->n_v * 8},
+                      {depth, c->f_depth.p, n_ccf * 91 * 8},
+                      {bis, c->f_bis.p, n_ccf * 91 * 8}}));
   return SOAP_OK;
 }
 
@@ -1993,29 +2102,36 @@ int soap_fit_ccf_host_err(soap_ctx *c, const double *v, int32_t n_v, const doubl
       if (!std::isfinite(err[i]) || err[i] == 0.0)
         return fail(c, SOAP_ERR_ARG, "fit_ccf_host: error %zu is %g (must be finite and non-zero)", i, err[i]);
   HIPCHK(c, hipSetDevice(c->device));
-  double *dv = nullptr, *dy = nullptr, *de = nullptr, *dpar = nullptr, *dmod = nullptr, *ddep = nullptr, *dbis = nullptr;
-  int32_t *dst = nullptr;
-  int rc = SOAP_OK;
-  if ((rc = dalloc(c, &dv, n_v)) || (rc = dalloc(c, &dy, (size_t)n_ccf * n_v)) ||
-      (err && (rc = dalloc(c, &de, (size_t)n_ccf * n_v))) || (rc = dalloc(c, &dpar, (size_t)n_ccf * 5)) ||
-      (rc = dalloc(c, &dmod, (size_t)n_ccf * n_v)) || (rc = dalloc(c, &ddep, (size_t)n_ccf * 91)) ||
-      (rc = dalloc(c, &dbis, (size_t)n_ccf * 91)) || (status && (rc = dalloc(c, &dst, (size_t)n_ccf)))) {
-    for (double *p : {dv, dy, de, dpar, dmod, ddep, dbis}) dfree_c(c, p);
-    dfree_c(c, dst);
-    return rc;
+  // one workspace of the context: inputs, then outputs, each moved in one piece
+  const size_t nv = (size_t)n_v, nc = (size_t)n_ccf, o_y = nv, o_e = o_y + nc * nv, o_par = o_e + (err ? nc * nv : 0),
+               o_mod = o_par + nc * 5, o_dep = o_mod + nc * nv, o_bis = o_dep + nc * 91, o_st = o_bis + nc * 91;
+  int rc = ensure(c, c->fit_ws, (o_st + (nc + 1) / 2) * 8);
+  if (rc) return rc;
+  double *ws = (double *)c->fit_ws.p;
+  hipError_t e = hipSuccess;
+  // the staging holds the inputs and, after the wait, the outputs: as large as the larger
+  const Pinned stage(std::max(o_par, o_st + (nc + 1) / 2 - o_par) * 8);
+  if (double *pin = (double *)stage.p()) {
+    memcpy(pin, v, nv * 8);
+    memcpy(pin + o_y, y, nc * nv * 8);
+    if (err) memcpy(pin + o_e, err, nc * nv * 8);
+    e = hipMemcpyAsync(ws, pin, o_par * 8, hipMemcpyHostToDevice, c->stream);
+  } else {
+    e = hipMemcpyAsync(ws, v, nv * 8, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(ws + o_y, y, nc * nv * 8, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess && err) e = hipMemcpyAsync(ws + o_e, err, nc * nv * 8, hipMemcpyHostToDevice, c->stream);
   }
-  hipError_t e = hipMemcpyAsync(dv, v, n_v * 8, hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(dy, y, (size_t)n_ccf * n_v * 8, hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess && err) e = hipMemcpyAsync(de, err, (size_t)n_ccf * n_v * 8, hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess) e = launch_fit(dv, n_v, dy, de, n_ccf, dpar, dmod, ddep, dbis, nullptr, c->stream, dst);
-  if (e == hipSuccess) e = hipMemcpyAsync(par, dpar, (size_t)n_ccf * 5 * 8, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess && status) e = hipMemcpyAsync(status, dst, (size_t)n_ccf * 4, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess && model) e = hipMemcpyAsync(model, dmod, (size_t)n_ccf * n_v * 8, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess && depth) e = hipMemcpyAsync(depth, ddep, (size_t)n_ccf * 91 * 8, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess && bis) e = hipMemcpyAsync(bis, dbis, (size_t)n_ccf * 91 * 8, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  for (double *p : {dv, dy, de, dpar, dmod, ddep, dbis}) dfree_c(c, p);
-  dfree_c(c, dst);
+  if (e == hipSuccess)
+    e = launch_fit(ws, n_v, ws + o_y, err ? ws + o_e : nullptr, n_ccf, ws + o_par, ws + o_mod, ws + o_dep, ws + o_bis,
+                   nullptr, c->stream, status ? (int32_t *)(ws + o_st) : nullptr);
+  if (e == hipSuccess)
+    e = fetch(c, {{par, ws + o_par, nc * 5 * 8},
+                  {model, ws + o_mod, nc * nv * 8},
+                  {depth, ws + o_dep, nc * 91 * 8},
+                  {bis, ws + o_bis, nc * 91 * 8},
+                  {status, ws + o_st, nc * 4}}, &stage);
+  else
+    hipStreamSynchronize(c->stream);  // the inputs may still be on their way
   if (e != hipSuccess) return fail(c, SOAP_ERR_HIP, "fit_ccf_host: %s", hipGetErrorString(e));
   return SOAP_OK;
 }
@@ -2186,7 +2302,7 @@ int soap_diff_setup(soap_ctx *c, int32_t grid, int32_t n_phase, int32_t map_res,
       (rc = ensure(c, d.th, (size_t)n_phase * 4 * 8)) || (rc = ensure(c, d.dth, (size_t)n_phase * 4 * 8)) ||
       (rc = ensure(c, d.gy, (size_t)n_phase * c->n_v * 8)) ||
       (rc = ensure(c, d.bisd, (size_t)n_phase * (c->n_v + kBisHead) * 8)) ||
-      (rc = ensure(c, d.tg, ((size_t)n_phase * 3 + 1 + kDiffScalars) * 8)) ||
+      (rc = ensure(c, d.tg, ((size_t)n_phase * 6 + 1 + kDiffScalars) * 8)) ||
       (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines, n_phase) * n_phase * c->n_v * 8)))
     return rc;
   int wid = conv_window(c->wave, sigma_ms);
@@ -2316,10 +2432,19 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
   d.fmaps = d_fmaps;
   d.target = d_target;
   d.w_spec = w_spec;
-  double *tg = (double *)d.tg.p;  // [rv_t | fw_t | bis_t | loss]
-  HIPCHK(c, hipMemcpyAsync(tg, rv_t, (size_t)d.P * 8, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(tg + d.P, fw_t, (size_t)d.P * 8, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(tg + 2 * d.P, bis_t, (size_t)d.P * 8, hipMemcpyHostToDevice, c->stream));
+  double *tg = (double *)d.tg.p;  // [rv_t | fw_t | bis_t | loss | scalar gradients | rv | fw | bis]
+  const size_t pb = (size_t)d.P * 8;
+  const Pinned stage(3 * pb + (1 + kDiffScalars) * 8);  // the targets, then the results
+  if (char *pin = stage.p()) {
+    memcpy(pin, rv_t, pb);
+    memcpy(pin + pb, fw_t, pb);
+    memcpy(pin + 2 * pb, bis_t, pb);
+    HIPCHK(c, hipMemcpyAsync(tg, pin, 3 * pb, hipMemcpyHostToDevice, c->stream));
+  } else {
+    HIPCHK(c, hipMemcpyAsync(tg, rv_t, pb, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(tg + d.P, fw_t, pb, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(tg + 2 * d.P, bis_t, pb, hipMemcpyHostToDevice, c->stream));
+  }
   DiffArgs a = diff_args(c);
   ConvArgs ca = diff_conv(c);
   {
@@ -2346,18 +2471,10 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
     // the loss and the fit-parameter derivatives for the backward stay on the device
     HIPCHK(c, launch_diff_loss(d.P, d.res_blocks, (const double *)d.res_part.p, (const double *)d.th.p, tg, tg + d.P,
                                tg + 2 * d.P, w_spec, w_rv, w_fw, w_bis, (double *)d.bisd.p, c->n_v, nullptr, 0.0,
-                               0.0, 0.0, tg + 3 * d.P, (double *)d.dth.p, c->stream));
+                               0.0, 0.0, tg + 3 * d.P, (double *)d.dth.p, tg + 3 * d.P + 1 + kDiffScalars, c->stream));
   }
-  std::vector<double> th((size_t)d.P * 4), bd((size_t)d.P * (c->n_v + kBisHead));
-  HIPCHK(c, hipMemcpyAsync(loss, tg + 3 * d.P, 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(th.data(), d.th.p, th.size() * 8, hipMemcpyDeviceToHost, c->stream));
-  if (bis) HIPCHK(c, hipMemcpyAsync(bd.data(), d.bisd.p, bd.size() * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int p = 0; p < d.P; p++) {
-    if (rv) rv[p] = th[p * 4 + 2];
-    if (fw) fw[p] = th[p * 4 + 3];
-    if (bis) bis[p] = bd[(size_t)p * (c->n_v + kBisHead)];
-  }
+  const double *series = tg + 3 * d.P + 1 + kDiffScalars;
+  HIPCHK(c, fetch(c, {{loss, tg + 3 * d.P, 8}, {rv, series, pb}, {fw, series + d.P, pb}, {bis, series + 2 * d.P, pb}}, &stage));
   d.have_fwd = true;
   return SOAP_OK;
 }
@@ -2389,8 +2506,7 @@ int soap_diff_backward(soap_ctx *c, double *grad5, double *d_gq, double *d_gs, d
   // land in the tail of the loss slot buffer
   double *g5 = (double *)d.tg.p + 3 * d.P + 1;
   HIPCHK(c, launch_diff_grad(diff_piece_blocks(d.n_piece), (const double *)d.cell_part.p, g5, c->stream));
-  HIPCHK(c, hipMemcpyAsync(grad5, g5, kDiffScalars * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, fetch(c, {{grad5, g5, kDiffScalars * 8}}));
   return SOAP_OK;
 }
 
@@ -3121,7 +3237,7 @@ hipError_t dbatch_enqueue_one(soap_diffbatch::Item &it, hipStream_t st, bool adj
       e = launch_diff_loss(d.P, rb, (const double *)d.res_part.p, (const double *)d.th.p, it.rv_t, it.fw_t, it.bis_t,
                            it.w_spec, it.w_rv, it.w_fw, it.w_bis, bisd, c->n_v, it.prm, it.vsini_max,
                            (double)d.G * d.G, d.ns == 3 ? lb_factor_bound(d.lb) : 0.0, it.loss, (double *)d.dth.p,
-                           st);
+                           nullptr, st);
     if (!adjoint) return e;
     if (e == hipSuccess)
       e = launch_diff_backward(a, ca, it.target, c->trim, it.w_spec, c->d_vgrid, c->n_v, (const double *)d.ccf.p,

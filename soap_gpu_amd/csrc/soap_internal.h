@@ -588,7 +588,7 @@ hipError_t launch_ccf_sum(const double *part, int nc, int n_spec, int n_v, doubl
 hipError_t launch_diff_loss(int n_phase, int res_blocks, const double *res_part, const double *theta,
                             const double *rv_t, const double *fw_t, const double *bis_t, double w_spec, double w_rv,
                             double w_fw, double w_bis, double *bisd, int n_v, const double *prm, double vsini_max,
-                            double n_cells, double lbmax, double *loss, double *dth, hipStream_t s);
+                            double n_cells, double lbmax, double *loss, double *dth, double *series, hipStream_t s);
 // g[q] = sum over blocks (in order) of cell_part[b][q], q < kDiffScalars
 hipError_t launch_diff_grad(int n_blocks, const double *cell_part, double *g, hipStream_t s);
 // batched instances: stage st over jobs[n_inst] (device), prefix[n_inst + 1]

@@ -132,7 +132,7 @@ class SoapLoss(torch.autograd.Function):
         ctx.params_device = params.device
         ctx.n_params = params.numel()
         ctx.rv, ctx.fw, ctx.bis = rv, fw, bs
-        return torch.tensor(loss, dtype=torch.float64, device=params.device)
+        return torch.full((), loss, dtype=torch.float64, device=params.device)
 
     @staticmethod
     def backward(ctx, gout):
