@@ -58,6 +58,8 @@ struct soap_ctx {
   int64_t n = 0;
   int kind = -1;
   double step = 0, h = 0, expm1_h = 0;
+  bool lin_uniform = false;  // linear grid: every wavelength difference is step to 1e-8
+  bool lin_nodes = false;    // and every wavelength lambda_0 + i step to 4 units of its last place
   std::vector<double> wave;
   double *d_wave = nullptr;
   // mu
@@ -119,7 +121,7 @@ struct soap_ctx {
   int lin_off_lo = 0, lin_span = 0;
   bool lin_solid = false;  // delta constant along each disk column (disk_init maps, omega1 = 0)
   DevBuf qcells, qbin_off, acells, abin_off, alist_off;
-  DevBuf qgroups, qg_n, agroups, ag_n, lcnt, qpart, qcolw, qcolf, qcols;
+  DevBuf qgroups, qg_n, agroups, ag_n, lcnt, qpart, qcolw, qcolf, qcols, qpack;
   // solar mode: Lagrange nodes over the facula temperature range
   int solar_k = 0, t_norm_fac = 0;
   double solar_t[kMaxSolarNodes] = {}, solar_w[kMaxSolarNodes] = {};
@@ -586,6 +588,11 @@ int soap_set_wave(soap_ctx *c, int kind, const double *wave, int64_t n, double s
   c->step = step;
   c->h = h;
   c->expm1_h = expm1(h);
+  c->lin_uniform = kind == SOAP_GRID_LINEAR;
+  for (int64_t j = 1; j < n && c->lin_uniform; j++) c->lin_uniform = fabs((w[j] - w[j - 1]) / step - 1) <= 1e-8;
+  c->lin_nodes = c->lin_uniform;
+  for (int64_t j = 0; j < n && c->lin_nodes; j++)
+    c->lin_nodes = fabs(fma(-(double)j, step, w[j] - w[0])) <= 0x1p-50 * fabs(w[j]);
   c->res_sigma = -1;
   int rc = dalloc(c, &c->d_wave, (size_t)n);
   if (rc) return rc;
@@ -721,6 +728,10 @@ static LinArgs lin_args(soap_ctx *c) {
   a.grid = c->G;
   a.lambda0 = c->wave[0];
   a.step = c->step;
+  a.inv_step = 1 / c->step;
+  a.uniform = c->lin_uniform;
+  a.nodes = c->lin_nodes;
+  a.solid = c->lin_solid;
   a.wave = c->d_wave;
   a.off_lo = c->lin_off_lo;
   a.span = c->lin_span;
@@ -913,7 +924,8 @@ int soap_quiet_star(soap_ctx *c) {
       return rc;
     if (by_cols && ((rc = ensure(c, c->qcolw, (size_t)ncs * c->G * 4 * 8)) ||
                          (rc = ensure(c, c->qcolf, (size_t)ncs * c->G * 4)) ||
-                         (rc = ensure(c, c->qcols, (size_t)c->G * sizeof(LinGroup)))))
+                         (rc = ensure(c, c->qcols, (size_t)c->G * sizeof(LinGroup))) ||
+                         (rc = ensure(c, c->qpack, quiet_column_pack_bytes(c->n_mu, c->G)))))
       return rc;
     if (!by_cols) {
       StageTimer tm(c, ST_TAPS_QUIET);
@@ -926,7 +938,8 @@ int soap_quiet_star(soap_ctx *c) {
       if (by_cols)
         HIPCHK(c, launch_gather_quiet_cols(lin_args(c), c->d_cube[SOAP_CUBE_QUIET], c->d_cube[SOAP_CUBE_QUIET_SED],
                                            c->d_region, (double *)c->qcolw.p, (int32_t *)c->qcolf.p,
-                                           (LinGroup *)c->qcols.p, (double *)c->qpart.p, c->d_quiet, c->stream));
+                                           (LinGroup *)c->qcols.p, c->qpack.p, (double *)c->qpart.p, c->d_quiet,
+                                           c->stream));
       else
         HIPCHK(c, launch_gather_quiet_linear(lin_args(c), c->d_cube[SOAP_CUBE_QUIET], c->d_cube[SOAP_CUBE_QUIET_SED],
                                              (const LinGroup *)c->qgroups.p, (const int32_t *)c->qbin_off.p,

@@ -257,6 +257,10 @@ struct LinArgs {
   const double *wave;         // [n]
   int32_t off_lo, span;       // source indices staged per tile: [j0 + off_lo, j0 + off_lo + span)
   const double *delta, *limb, *lbm;
+  int32_t uniform;     // every wavelength difference is step to 1e-8
+  int32_t solid;       // the shift depends on the disk column only
+  int32_t nodes;       // every wavelength is lambda0 + i step to 4 units of its last place
+  double inv_step;
 };
 
 // A run of cells of one (phase, mu bin) cell list with bitwise-equal shifts and
@@ -536,8 +540,9 @@ int quiet_linear_sets(int n_mu);
 // quiet_column_sets(n_mu) * grid * 4 doubles, colf: quiet_column_sets(n_mu) * grid
 // ints, cols: grid groups, part: quiet_column_sets(n_mu) * 2 * n doubles
 hipError_t launch_gather_quiet_cols(const LinArgs &a, const double *q, const double *qs, const int32_t *region,
-                                    double *colw, int32_t *colf, LinGroup *cols, double *part, double *out,
-                                    hipStream_t s);
+                                    double *colw, int32_t *colf, LinGroup *cols, void *pack, double *part,
+                                    double *out, hipStream_t s);
+size_t quiet_column_pack_bytes(int n_mu, int grid);
 int quiet_column_sets(int n_mu);
 bool quiet_columns_fit(int span);  // the staged rows of a bin set fit the block's LDS
 hipError_t launch_gather_active_linear(const LinArgs &a, const FirArgs &f, const LinGroup *groups,
