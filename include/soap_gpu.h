@@ -303,9 +303,10 @@ int soap_set_fir_shape(soap_ctx *ctx, int32_t phases_per_block, int32_t pixels_p
  *        + w_rv sum (RV_p - rv_target_p)^2 + w_fwhm sum (FWHM_p - fwhm_target_p)^2
  *        + w_bis sum (BIS_p - bis_target_p)^2.
  * The facula population is optional: without facula seeds and maps psi = 0.
- * Maps are filling factors in [0, 1].  The per-cell weights enter fixed-point tap
- * sums: G^2 max|L| max(3, |contrast|, |contrast_fac| max|1 + LB|) must stay below
- * 2^30 (SOAP_ERR_LIMIT from soap_diff_forward, a NaN loss in graph replays).
+ * Maps are filling factors in [0, 1].  The per-cell weights enter tap sums, whose
+ * accepted range is that of the series' fixed-point taps:
+ * G^2 max|L| max(3, |contrast|, |contrast_fac| max|1 + LB|) must stay below 2^30
+ * (SOAP_ERR_LIMIT from soap_diff_forward, a NaN loss in graph replays).
  * Array arguments named d_* are device (HIP) pointers: seeds [n_mu][n], maps
  * [P][M][M], target [P][n]; they must stay valid until soap_diff_backward. */
 typedef struct soap_diff_params {
