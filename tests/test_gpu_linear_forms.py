@@ -33,3 +33,19 @@ def test_linear_forms(engine, lmin, stray, w_ratio, n):
     for p in range(2):
         for got, ref in zip(engine.get_raw(p), o["raw"][p]):
             assert normwise(got, ref) <= 1e-12
+
+
+@pytest.mark.parametrize("speed,n", [(0.1, 2561), (2.0, 2815), (6.0, 3001), (9.0, 3001), (14.0, 3001)])
+def test_linear_quiet_reach(engine, speed, n):
+    """The quiet star by columns from windows of a few pixels to ones too wide for the taps (the
+    rotation sped up), against the oracle.  Bar: both sides' weights may be off by one unit in the
+    last place of a shifted wavelength, so by ulp(lambda) / step of the row's change per pixel."""
+    w = synth.linear_small(seed=21, grid=40, n=n, n_mu=5, n_phase=2)
+    w.star["prot"] /= speed
+    o = run_oracle(w, with_ccf=False)
+    setup_workload(engine, w, with_mask=False)
+    engine.quiet_star()
+    limb = np.abs(o["maps"]["limb"][o["maps"]["limb"] != -999.0]).sum()
+    for i, k in enumerate(("q", "qsed")):
+        change = np.abs(np.diff(w.cubes[k], axis=1)).max() * limb / np.abs(o["quiet"][i]).max()
+        assert normwise(engine.get_quiet(i), o["quiet"][i]) <= 2 * np.spacing(w.wave[-1]) / 0.005 * change
