@@ -98,6 +98,8 @@ struct soap_ctx {
   // differentiable path
   struct {
     bool ready = false, have_fwd = false;
+    int64_t fwd_n = 0;  // sizes of the last forward, which its backward's buffers have
+    int fwd_mu = 0, fwd_lines = 0, fwd_v = 0;
     int G = 0, P = 0, M = 0, dmin = 0, nd = 0, res_blocks = 0;
     double sigma = 0, w_spec = 0;
     soap_diff_params prm{};
@@ -2429,12 +2431,14 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
     return (int)ceil(log1p(fb) / c->h);
   };
   int mlo = mshift(-prm->vsini_kms), mhi = mshift(prm->vsini_kms);
-  d.dmin = mlo - 2;
-  d.nd = mhi - d.dmin + 3;
-  if (d.nd > 2048) return fail(c, SOAP_ERR_LIMIT, "diff_forward: shift range of %d pixels", d.nd);
+  const int dmin = mlo - 2, nd = mhi - dmin + 3;
+  if (nd > 2048) return fail(c, SOAP_ERR_LIMIT, "diff_forward: shift range of %d pixels", nd);
   const int ns = d_f ? 3 : 2;
   int rc;
-  if ((rc = diff_plan(c)) || (rc = diff_buffers(c, d.nd, ns))) return rc;
+  d.have_fwd = false;  // the buffers are this forward's from here on
+  if ((rc = diff_plan(c)) || (rc = diff_buffers(c, nd, ns))) return rc;
+  d.dmin = dmin;
+  d.nd = nd;
   if (!c->mask_built && (rc = build_mask(c))) return rc;
   d.prm = *prm;
   d.ns = ns;
@@ -2489,6 +2493,10 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
   const double *series = tg + 3 * d.P + 1 + kDiffScalars;
   HIPCHK(c, fetch(c, {{loss, tg + 3 * d.P, 8}, {rv, series, pb}, {fw, series + d.P, pb}, {bis, series + 2 * d.P, pb}}, &stage));
   d.have_fwd = true;
+  d.fwd_n = c->n;
+  d.fwd_mu = c->n_mu;
+  d.fwd_lines = c->n_lines;
+  d.fwd_v = c->n_v;
   return SOAP_OK;
 }
 
@@ -2497,6 +2505,9 @@ int soap_diff_backward(soap_ctx *c, double *grad5, double *d_gq, double *d_gs, d
   if (!c || !grad5 || !d_gq || !d_gs || !d_gmaps) return fail(c, SOAP_ERR_ARG, "diff_backward: null argument");
   auto &d = c->diff;
   if (!d.have_fwd) return fail(c, SOAP_ERR_STATE, "diff_backward: run diff_forward first");
+  if (d.fwd_n != c->n || d.fwd_mu != c->n_mu || d.fwd_lines != c->n_lines || d.fwd_v != c->n_v)
+    return fail(c, SOAP_ERR_STATE, "diff_backward: the grid, the number of mu bins or the mask's size changed since the "
+                "forward");
   if (d.ns == 3 && (!d_gf || !d_gfmaps))
     return fail(c, SOAP_ERR_ARG, "diff_backward: the forward had faculae: facula gradients need buffers");
   HIPCHK(c, hipSetDevice(c->device));
@@ -3150,7 +3161,7 @@ std::vector<uintptr_t> dbatch_signature(const soap_ctx *c) {
           u(d.mt_col.p), u(d.mt_val.p), u(c->ccf_part.p), u(c->m_start.p), u(c->m_alive.p), u(c->m_val.p),
           u(c->d_w_sorted), u(c->ctap.p), u(d.bisd.p), u(d.maps), u(d.q), u(d.s), u(d.target), u(d.f), u(d.fmaps),
           (uintptr_t)d.ns, (uintptr_t)d.nd,
-          (uintptr_t)d.dmin, (uintptr_t)d.P, (uintptr_t)d.G, (uintptr_t)d.M, (uintptr_t)c->n, (uintptr_t)c->res_ntp,
+          (uintptr_t)d.dmin, (uintptr_t)d.P, (uintptr_t)d.G, (uintptr_t)d.M, (uintptr_t)c->n, (uintptr_t)c->n_mu, (uintptr_t)c->res_ntp,
           (uintptr_t)c->n_lines, (uintptr_t)c->n_v};
 }
 
@@ -3344,6 +3355,7 @@ int soap_diff_batch_bind(soap_diffbatch *b, int32_t i, double vsini_max, const d
   int nd = mshift(vsini_max) - dmin + 3;
   if (nd > 2048) return dfail(b, SOAP_ERR_LIMIT, "diff_batch_bind: shift range of %d pixels", nd);
   int rc;
+  d.have_fwd = false;  // the per-call forward state no longer matches the buffers
   if ((rc = diff_plan(c)) || (rc = diff_buffers(c, nd, ns)) ||
       (!c->mask_built && (rc = build_mask(c))) || (rc = diff_mask_transpose(c)))
     return dfail(b, rc, "diff_batch_bind: instance %d: %s", i, c->err.c_str());
@@ -3356,7 +3368,6 @@ int soap_diff_batch_bind(soap_diffbatch *b, int32_t i, double vsini_max, const d
   d.maps = d_maps;
   d.fmaps = d_fmaps;
   d.target = d_target;
-  d.have_fwd = false;  // the per-call forward state no longer matches the buffers
   it.vsini_max = vsini_max;
   it.dmin = dmin;
   it.nd = nd;
