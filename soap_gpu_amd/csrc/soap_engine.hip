@@ -3174,6 +3174,17 @@ void dbatch_drop_graph(soap_diffbatch *b) {
   }
 }
 
+// Steps are only enqueued: before anything that they read is laid out anew or freed (an
+// instance's plan and buffers, an executable graph) the last one has to have ended.
+hipError_t dbatch_wait(soap_diffbatch *b) {
+  hipError_t e = hipStreamSynchronize(b->stream);
+  for (int k = 0; k < kDiffLanes; k++) {  // joined into the stream, but for a step that failed
+    const hipError_t el = hipStreamSynchronize(b->lane[k]);
+    if (e == hipSuccess) e = el;
+  }
+  return e;
+}
+
 int dfail(soap_diffbatch *b, int code, const char *fmt, ...) {
   char buf[512];
   va_list ap;
@@ -3355,6 +3366,7 @@ int soap_diff_batch_bind(soap_diffbatch *b, int32_t i, double vsini_max, const d
   int nd = mshift(vsini_max) - dmin + 3;
   if (nd > 2048) return dfail(b, SOAP_ERR_LIMIT, "diff_batch_bind: shift range of %d pixels", nd);
   int rc;
+  if (dbatch_wait(b) != hipSuccess) return dfail(b, SOAP_ERR_HIP, "diff_batch_bind: waiting for the last step failed");
   d.have_fwd = false;  // the per-call forward state no longer matches the buffers
   if ((rc = diff_plan(c)) || (rc = diff_buffers(c, nd, ns)) ||
       (!c->mask_built && (rc = build_mask(c))) || (rc = diff_mask_transpose(c)))
@@ -3406,6 +3418,7 @@ int soap_diff_batch_step(soap_diffbatch *b, int32_t use_graph, int32_t with_adjo
     if (it.bound && dbatch_signature(it.c) != it.sig)
       return dfail(b, SOAP_ERR_STATE, "diff_batch_step: an instance was changed after binding");
     if (it.bound && !diff_plan_current(it.c)) {  // other bins of the same number: the plan is laid out anew
+      if (dbatch_wait(b) != hipSuccess) return dfail(b, SOAP_ERR_HIP, "diff_batch_step: waiting for the last step failed");
       int rc = diff_plan(it.c);
       if (!rc) rc = diff_buffers(it.c, it.nd, it.c->diff.ns);
       if (rc) return dfail(b, rc, "diff_batch_step: %s", it.c->err.c_str());

@@ -1,7 +1,8 @@
 """The differentiable model when the mu bins are set anew between its calls: another
 number of them is refused where buffers of the old number are bound or kept (a graph
 step, a backward), and taken up by the next forward; going back to the bound number is
-accepted again."""
+accepted again.  Other bins of the same number are taken up by the next forward and by the
+next step, whether or not the step before it has been waited for."""
 import numpy as np
 import pytest
 
@@ -86,4 +87,52 @@ def test_backward_refuses_another_number_of_bins():
     for a, b in zip(model.backward(), ref):
         assert np.array_equal(np.asarray(a if isinstance(a, np.ndarray) else a.cpu()),
                               np.asarray(b if isinstance(b, np.ndarray) else b.cpu()))
+    model.eng.close()
+
+
+def _same_as_fresh(bounds, t, loss, grads):
+    """Results against those of a new model on these bounds, bit for bit."""
+    w, fresh, _ = _problem()
+    fresh.eng.set_mu_bounds(bounds)
+    assert _forward(fresh, t) == loss
+    for a, b in zip(grads, fresh.backward()):
+        a, b = (x if isinstance(x, np.ndarray) else x.cpu().numpy() for x in (a, b))
+        np.testing.assert_array_equal(a, b)
+    fresh.eng.close()
+
+
+BOUNDS = [np.array(b) for b in ([0.95, 0.8, 0.2], [0.6, 0.4, 0.3], [0.75, 0.5, 0.25])]
+
+
+def test_forward_takes_up_other_bins():
+    w, model, t = _problem()
+    _forward(model, t)
+    for bounds in BOUNDS:
+        model.eng.set_mu_bounds(bounds)
+        loss = _forward(model, t)
+        _same_as_fresh(bounds, t, loss, model.backward())
+    model.eng.close()
+
+
+@pytest.mark.parametrize("graph", [True, False])
+@pytest.mark.parametrize("wait", [True, False])
+def test_step_takes_up_other_bins(graph, wait):
+    import torch
+    from soap_gpu_amd.diff import DiffBatch
+    w, model, t = _problem()
+    batch = DiffBatch([model])
+    out = _bind(batch, t)
+    torch.cuda.synchronize()
+    batch.step(graph=graph)
+    for bounds in BOUNDS:
+        if wait:
+            batch.sync()
+        model.eng.set_mu_bounds(bounds)
+        batch.step(graph=graph)
+        batch.step(graph=graph)
+    batch.sync()
+    # a step's tap range is its bound vsini's, so its FIRs may add zeros that a forward leaves out
+    got = [out["g5"], out["gq"], out["gs"], out["gm"], out["gf"], out["gfm"]]
+    _same_as_fresh(BOUNDS[-1], t, float(out["loss"][0]), [x.cpu().numpy() for x in got])
+    batch.close()
     model.eng.close()
