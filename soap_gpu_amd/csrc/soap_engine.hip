@@ -289,10 +289,16 @@ struct PinPool {
     idle.push_back(s);
   }
 };
+// busy: a stream that may still be copying from or to the buffer, waited for before the buffer
+// goes back (a call that fails between its copy and its own wait).
 struct Pinned {
   PinPool::Slot slot;
+  mutable hipStream_t busy = nullptr;
   explicit Pinned(size_t bytes) : slot(PinPool::get().take(bytes)) {}
-  ~Pinned() { PinPool::get().give(slot); }
+  ~Pinned() {
+    if (busy) hipStreamSynchronize(busy);
+    PinPool::get().give(slot);
+  }
   Pinned(const Pinned &) = delete;
   Pinned &operator=(const Pinned &) = delete;
   char *p() const { return slot.p; }
@@ -330,6 +336,7 @@ static hipError_t fetch(soap_ctx *c, std::initializer_list<FetchPart> parts, con
   }
   const hipError_t es = hipStreamSynchronize(c->stream);
   if (e == hipSuccess) e = es;
+  if (have) have->busy = nullptr;
   if (pin && e == hipSuccess)
     for (const FetchPart &p : parts)
       if (p.host && p.bytes) memcpy(p.host, pin + ((uintptr_t)p.dev - lo), p.bytes);
@@ -2456,6 +2463,7 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
     memcpy(pin, rv_t, pb);
     memcpy(pin + pb, fw_t, pb);
     memcpy(pin + 2 * pb, bis_t, pb);
+    stage.busy = c->stream;
     HIPCHK(c, hipMemcpyAsync(tg, pin, 3 * pb, hipMemcpyHostToDevice, c->stream));
   } else {
     HIPCHK(c, hipMemcpyAsync(tg, rv_t, pb, hipMemcpyHostToDevice, c->stream));

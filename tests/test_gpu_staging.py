@@ -49,3 +49,31 @@ def test_one_output_of_the_fit(engine):
         args[i] = out.ctypes.data_as(dp)
         assert engine.L.soap_get_fit(engine.ctx, *args) == 0
         assert np.array_equal(out.reshape(whole[k].shape), whole[k])
+
+
+def test_refused_forward_gives_its_staging_back():
+    """A forward of the differentiable model that is refused after its targets are on their
+    way (a resolution window too wide for the LDS), then calls that use the same staging."""
+    import torch
+    from soap_gpu_amd import synth
+    from soap_gpu_amd.diff import DiffModel
+    from soap_gpu_amd.engine import SoapError, select_mask_lines
+    ref = _call(7, 0)[0]
+    n, p = 24000, 3
+    w = synth.small(seed=4, grid=24, n=n, n_mu=4, n_phase=1, n_lines=30, lmin=5000.0, lmax=5000.0 * np.exp((n - 1) * 1e-6))
+    sl, sw = select_mask_lines(w.wave, w.mask_l, w.mask_w, 210)
+    dev = lambda a: torch.tensor(a, dtype=torch.float64, device="cuda")  # noqa: E731
+    q, maps, target = dev(w.cubes["q"]), dev(np.full((p, 8, 8), 0.2)), dev(np.full((p, n), 400.0))
+    eng = Engine(0)
+    wide, narrow = (DiffModel(eng, w.wave, w.mu_bounds, sl, sw, w.vgrid, 24, p, 8, s, 210) for s in (65000.0, w.sigma_inst))
+    args = ([2.0, 0.29, 0.34, 0.3], q, q, maps, target, np.arange(3.0), np.full(p, 9e3), 1e-6, 1e-3, 1e-5)
+    loss = narrow.forward(*args)[0]
+    for _ in range(3):
+        eng._chk(eng.L.soap_diff_setup(eng.ctx, 24, p, 8, 65000.0, None), "diff_setup")
+        with pytest.raises(SoapError, match="too wide"):
+            wide.forward(*args)
+        got = _call(7, 0)[0]
+        assert all(np.array_equal(got[k], ref[k]) for k in ref)
+        eng._chk(eng.L.soap_diff_setup(eng.ctx, 24, p, 8, float(w.sigma_inst), None), "diff_setup")
+        assert narrow.forward(*args)[0] == loss
+    eng.close()
