@@ -153,6 +153,7 @@ struct soap_ctx {
   DevBuf m_start, m_len, m_val, m_alive, sorted, rank, ccf_part;
   DevBuf wsum;  // [n_v] live mask weight per velocity (the CCF of a spectrum of ones)
   DevBuf fp;    // [n_lines] int2 line footprints (first trimmed pixel, length)
+  int fp_max = 0;   // longest line footprint
   int ccf_cap = 0;  // LDS segment length of the CCF (ccf_lds_cap of the longest footprint)
   int mask_scan = 0;
   bool have_mask = false, mask_built = false;
@@ -1812,6 +1813,7 @@ static int build_mask(soap_ctx *c) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
   int fmax = 0;
   for (int q = 0; q < c->n_lines; q++) fmax = std::max(fmax, fp[2 * q + 1]);
+  c->fp_max = fmax;
   c->ccf_cap = ccf_lds_cap(fmax);
   c->mask_built = true;
   c->diff.mt_ready = false;
@@ -1916,7 +1918,7 @@ static int diff_mask_transpose(soap_ctx *c) {
 static hipError_t ctx_ccf(soap_ctx *c, const double *spec, int n_spec, double *part, hipStream_t st) {
   return launch_ccf_lds(spec, c->n, c->trim, n_spec, c->n_lines, c->n_v, c->n - 2 * (int64_t)c->trim,
                         (const int32_t *)c->m_start.p, (const uint32_t *)c->m_alive.p, (const double2 *)c->m_val.p,
-                        c->d_w_sorted, (const int2 *)c->fp.p, c->ccf_cap, part, st);
+                        c->d_w_sorted, (const int2 *)c->fp.p, c->fp_max, part, st);
 }
 
 // The CCF runs on the unnormalised spectra d_lraw (the reduction applies the
@@ -1932,7 +1934,7 @@ static int ccf_impl(soap_ctx *c, bool norm) {
   if (!c->mask_built && (rc = build_mask(c))) return rc;
   int n_spec = (c->P + 1) * 3;
   if ((rc = dalloc(c, &c->d_ccf, (size_t)n_spec * c->n_v)) ||
-      (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines, n_spec) * n_spec * c->n_v * 8)))
+      (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines) * n_spec * c->n_v * 8)))
     return rc;
   if (norm) {
     NormCcfArgs a{};
@@ -1950,7 +1952,7 @@ static int ccf_impl(soap_ctx *c, bool norm) {
     a.m_wv = (const double2 *)c->m_val.p;
     a.w_sorted = c->d_w_sorted;
     a.fp = (const int2 *)c->fp.p;
-    a.cap = c->ccf_cap;
+    a.fmax = c->fp_max;
     a.part = (double *)c->ccf_part.p;
     StageTimer tm(c, ST_CCF);
     HIPCHK(c, launch_norm_ccf(a, c->stream));
@@ -1963,7 +1965,7 @@ static int ccf_impl(soap_ctx *c, bool norm) {
   }
   {
     StageTimer tm(c, ST_CCF_REDUCE);
-    HIPCHK(c, launch_ccf_reduce((const double *)c->ccf_part.p, ccf_chunks(c->n_lines, n_spec), n_spec, c->n_v, c->d_appod,
+    HIPCHK(c, launch_ccf_reduce((const double *)c->ccf_part.p, ccf_chunks(c->n_lines), n_spec, c->n_v, c->d_appod,
                                 (const double *)c->mm.p, (const double *)c->wsum.p, c->d_ccf, c->stream));
   }
   c->have_ccf = true;
@@ -2292,7 +2294,7 @@ static int diff_buffers(soap_ctx *c, int nd, int ns) {
   auto &d = c->diff;
   const size_t per = (size_t)d.P * c->n_mu * nd * ns;
   int rc;
-  if ((rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines, d.P) * d.P * c->n_v * 8)) ||
+  if ((rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines) * d.P * c->n_v * 8)) ||
       (rc = ensure(c, d.drow, (size_t)nd * 2 * 4)) || (rc = ensure(c, d.blag, (size_t)c->n_mu * 2 * 4)) ||
       (rc = ensure(c, d.mom, (size_t)d.n_piece * diff_moments(ns) * d.P * 8)) ||
       (rc = ensure(c, d.wts, (size_t)d.n_piece * ns * d.P * 8)) ||
@@ -2325,7 +2327,7 @@ int soap_diff_setup(soap_ctx *c, int32_t grid, int32_t n_phase, int32_t map_res,
       (rc = ensure(c, d.gy, (size_t)n_phase * c->n_v * 8)) ||
       (rc = ensure(c, d.bisd, (size_t)n_phase * (c->n_v + kBisHead) * 8)) ||
       (rc = ensure(c, d.tg, ((size_t)n_phase * 6 + 1 + kDiffScalars) * 8)) ||
-      (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines, n_phase) * n_phase * c->n_v * 8)))
+      (rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines) * n_phase * c->n_v * 8)))
     return rc;
   int wid = conv_window(c->wave, sigma_ms);
   if (wid < 1 || 2 * (int64_t)wid + 2 >= c->n) return fail(c, SOAP_ERR_ARG, "diff_setup: window %d vs %lld pixels", wid, (long long)c->n);
@@ -2482,7 +2484,7 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
   {
     StageTimer tm(c, ST_CCF);
     HIPCHK(c, ctx_ccf(c, (const double *)d.F.p, d.P, (double *)c->ccf_part.p, c->stream));
-    HIPCHK(c, launch_ccf_sum((const double *)c->ccf_part.p, ccf_chunks(c->n_lines, d.P), d.P, c->n_v, (double *)d.ccf.p,
+    HIPCHK(c, launch_ccf_sum((const double *)c->ccf_part.p, ccf_chunks(c->n_lines), d.P, c->n_v, (double *)d.ccf.p,
                              c->stream));
   }
   {
@@ -2829,8 +2831,8 @@ int batch_build(soap_batch *b) {
     nm[i] = NormJob{c->n, nbx, (const double *)c->mm.p, c->d_lraw, c->d_lower};
     w[BS_NORM][i] = nbx * n_spec;
     // CCF + fit
-    int nc = ccf_chunks(c->n_lines, n_spec);
-    cc[i] = CcfJob{c->d_lraw, c->n, c->trim, c->n - 2 * (int64_t)c->trim, n_spec, c->n_lines, c->n_v, nc, ccf_lines(c->n_lines, n_spec),
+    int nc = ccf_chunks(c->n_lines);
+    cc[i] = CcfJob{c->d_lraw, c->n, c->trim, c->n - 2 * (int64_t)c->trim, n_spec, c->n_lines, c->n_v, nc,
                    (const int32_t *)c->m_start.p, (const uint32_t *)c->m_alive.p, (const double2 *)c->m_val.p,
                    c->d_w_sorted, (const int2 *)c->fp.p, c->ccf_cap, (double *)c->ccf_part.p};
     lds_ccf = std::max(lds_ccf, ccf_lds_bytes(c->ccf_cap));
@@ -3263,7 +3265,7 @@ hipError_t dbatch_enqueue_one(soap_diffbatch::Item &it, hipStream_t st, bool adj
     hipError_t e = launch_diff_forward_spectra(a, ca, it.target, c->trim, (double *)d.res_part.p, &rb, st);
     if (e == hipSuccess) e = ctx_ccf(c, (const double *)d.F.p, d.P, (double *)c->ccf_part.p, st);
     if (e == hipSuccess)
-      e = launch_ccf_sum((const double *)c->ccf_part.p, ccf_chunks(c->n_lines, d.P), d.P, c->n_v, (double *)d.ccf.p,
+      e = launch_ccf_sum((const double *)c->ccf_part.p, ccf_chunks(c->n_lines), d.P, c->n_v, (double *)d.ccf.p,
                          st);
     if (e == hipSuccess)
       e = launch_fit(c->d_vgrid, c->n_v, (const double *)d.ccf.p, nullptr, d.P, (double *)d.par.p, (double *)d.model.p,

@@ -393,7 +393,7 @@ struct NormJob { int64_t n, bx; const double *mm, *in; double *o; };     // work
 struct CcfJob {                                                          // work: nc * ceil(n_spec / ccf_spec_chunk())
   const double *spec;
   int64_t stride, trim, n_t;
-  int32_t n_spec, n_lines, n_v, nc, lines;
+  int32_t n_spec, n_lines, n_v, nc;
   const int32_t *m_start;
   const uint32_t *m_pk;
   const double2 *m_wv;
@@ -481,9 +481,9 @@ struct NormCcfArgs {
   const double2 *m_wv;
   const double *w_sorted;
   const int2 *fp;  // line footprints, staged in LDS by the CCF
-  int32_t cap;     // LDS segment length (ccf_lds_cap)
+  int32_t fmax;    // longest footprint
   double *part;
-  int32_t nc, lines, n_ccf, nbx, n_norm, ratio;
+  int32_t cap, nc, n_ccf, nbx, n_norm, ratio;
 };
 hipError_t launch_norm_ccf(NormCcfArgs a, hipStream_t s);
 // the CCF with line footprints staged in LDS (fp from launch_mask_footprint) in
@@ -495,7 +495,7 @@ int ccf_lds_cap(int fmax);
 size_t ccf_lds_bytes(int cap);
 hipError_t launch_ccf_lds(const double *spec, int64_t spec_stride, int64_t trim, int n_spec, int n_lines, int n_v,
                           int64_t n_t, const int32_t *m_start, const uint32_t *m_pk, const double2 *m_wv,
-                          const double *w_sorted, const int2 *fp, int cap, double *part, hipStream_t s);
+                          const double *w_sorted, const int2 *fp, int fmax, double *part, hipStream_t s);
 hipError_t launch_mask_wsum(int n_lines, int n_v, int64_t n_t, const int32_t *m_start, const uint32_t *m_pk,
                             const double2 *m_wv, const double *w_sorted, double *wsum, hipStream_t s);
 // CCF
@@ -505,10 +505,9 @@ hipError_t launch_mask_build(const double *line_l, const double *line_w, const i
                              double2 *m_wv, hipStream_t s);
 hipError_t launch_mask_overwrite(const int32_t *sorted, int n_lines, int n_v, int scan, const int32_t *m_start,
                                  const int32_t *m_len, uint32_t *m_pk, hipStream_t s);
-int ccf_lines(int n_lines, int n_spec);
-int ccf_chunks(int n_lines, int n_spec);
+int ccf_chunks(int n_lines);
 // CCF of n_spec spectra (spec + sp*spec_stride + trim), normalised and appodised;
-// part: ccf_chunks(n_lines, n_spec) * n_spec * n_v doubles; w_sorted[q] = weight of line sorted[q]
+// part: ccf_chunks(n_lines) * n_spec * n_v doubles; w_sorted[q] = weight of line sorted[q]
 hipError_t launch_ccf_reduce(const double *part, int nc, int n_spec, int n_v, const double *appod, const double *mm,
                              const double *wsum, double *ccf, hipStream_t s);
 // err: per-point errors [n_ccf][n_v] or NULL (unit errors); status (optional): per

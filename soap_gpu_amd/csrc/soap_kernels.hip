@@ -2374,7 +2374,7 @@ hipError_t launch_mask_overwrite(const int32_t *sorted, int n_lines, int n_v, in
   return hipGetLastError();
 }
 
-// calculate_CCF_2 (CCF_func.py:27-36) on the sparse mask.  Block = (chunk of up to
+// calculate_CCF_2 (CCF_func.py:27-36) on the sparse mask.  Block = (chunk of
 // kCcfLines lines in wavelength order, chunk of kCcfSpec spectra); thread = one
 // velocity, summing its lines in order for all spectra of the chunk (each mask
 // entry is read once per block).  Each line's pixel footprint is staged in LDS
@@ -2390,7 +2390,6 @@ hipError_t launch_mask_overwrite(const int32_t *sorted, int n_lines, int n_v, in
 // The CCF therefore runs on x, and spec_norm does not have to finish before it:
 // the two share one launch (k_norm_ccf).
 constexpr int kCcfLines = 32;
-constexpr int kCcfBlocks = 512;
 constexpr int kCcfSpec = 8;
 constexpr int kCcfLdsCap = 512;  // LDS segment of the footprint form: 8 spectra x 512 pixels = 32 KiB
 
@@ -2427,19 +2426,11 @@ hipError_t launch_mask_footprint(int n_lines, int n_v, int64_t n_t, const int32_
 // n_v) adds its window's pixels from LDS, in pixel order.  A footprint longer
 // than cap pixels goes through in segments of cap (a window that straddles two
 // takes its low pixels from the first, so the order of the terms is kept).
-// AHEAD: the next segment's first blockDim.x pixels and, at a line's last segment, the
-// next line's mask entry are loaded while this segment's windows are summed.  A block
-// walks its lines in turn, and where the launch is too small for other blocks to hide
-// them one round trip to memory per line (2.3 us) is its time (200 lines, 78 spectra: 75
-// us per launch, 18 with these loads and two lines per block); where blocks fill the CUs
-// the registers cost more waves than the loads save (series of 303 spectra: 0.90 -> 1.17
-// ms), so the large launches and the batched one keep to the plain form.
-// lines: lines per chunk (ccf_lines); lds: kCcfSpec * cap doubles.
-template <bool AHEAD>
+// lds: kCcfSpec * cap doubles.
 __device__ __forceinline__ void ccf_lds_body(const double *spec_, int64_t spec_stride, int64_t trim, int n_spec,
                                              int n_lines, int n_v, int64_t n_t, const int32_t *m_start_,
                                              const uint32_t *m_pk_, const double2 *m_wv_, const double *w_sorted_,
-                                             const int2 *fp_, int cap, double *part_, int lines, int bx_, int by_,
+                                             const int2 *fp_, int cap, double *part_, int bx_, int by_,
                                              double *lds) {
   const GLOBAL double *spec = gl(spec_), *w_sorted = gl(w_sorted_);
   const GLOBAL int32_t *m_start = gl(m_start_);
@@ -2450,29 +2441,20 @@ __device__ __forceinline__ void ccf_lds_body(const double *spec_, int64_t spec_s
   const int chunk = bx_;
   const int s0 = by_ * kCcfSpec;
   const int ns = min(kCcfSpec, n_spec - s0);
-  const int q0 = chunk * lines, q1 = min(n_lines, q0 + lines);
-  const int iv = threadIdx.x, nt = blockDim.x;
-  const bool act = iv < n_v;
+  const int q0 = chunk * kCcfLines, q1 = min(n_lines, q0 + kCcfLines);
   const GLOBAL double *S[kCcfSpec];
 #pragma unroll
   for (int k = 0; k < kCcfSpec; k++) S[k] = spec + (long)(s0 + (k < ns ? k : 0)) * spec_stride + trim;
-  double acc[kCcfSpec], v[kCcfSpec];
+  const int iv = threadIdx.x;
+  const bool act = iv < n_v;
+  double acc[kCcfSpec];
 #pragma unroll
   for (int k = 0; k < kCcfSpec; k++) acc[k] = 0.0;
-  auto load = [&](long base, int seg, int j) {
-#pragma unroll
-    for (int k = 0; k < kCcfSpec; k++) v[k] = (j < seg && k < ns) ? S[k][base + j] : 0.0;
-  };
-  auto store = [&](int seg, int j) {
-    if (j < seg) {
-#pragma unroll
-      for (int k = 0; k < kCcfSpec; k++) lds[k * cap + j] = v[k];
-    }
-  };
-  int st = 0;
-  uint32_t pk = 0;
-  double wx = 0.0, wy = 0.0;
-  auto entry = [&](int q) {  // the velocity's mask entry of line q
+  for (int q = q0; q < q1; q++) {
+    // this line's mask entry, loaded before the staging so that the two overlap
+    int st = 0;
+    uint32_t pk = 0;
+    double wx = 0.0, wy = 0.0;
     if (act) {
       const long e = (long)q * n_v + iv;
       st = m_start[e];
@@ -2480,60 +2462,35 @@ __device__ __forceinline__ void ccf_lds_body(const double *spec_, int64_t spec_s
       wx = m_wv[2 * e];
       wy = m_wv[2 * e + 1];
     }
-  };
-  int f_lo = fp[2 * q0], f_len = fp[2 * q0 + 1];
-  if (AHEAD) {
-    entry(q0);
-    load(f_lo, min(cap, f_len), iv);
-  }
-  for (int q = q0; q < q1; q++) {
-    if (!AHEAD) {
-      // this line's mask entry, loaded before the staging so that the two overlap
-      entry(q);
-      f_lo = fp[2 * q];
-      f_len = fp[2 * q + 1];
-    }
-    const int c_st = st;
-    const uint32_t c_pk = pk;
-    const double c_wx = wx, c_wy = wy, w = w_sorted[q];
-    const bool more = AHEAD && q + 1 < q1;
-    const int n_lo = more ? fp[2 * q + 2] : 0, n_len = more ? fp[2 * q + 3] : 0;
-    if (more && f_len == 0) {  // nothing of this line in the spectrum: only the next one's loads
-      entry(q + 1);
-      load(n_lo, min(cap, n_len), iv);
-    }
+    const double w = w_sorted[q];
+    const int f_lo = fp[2 * q], f_len = fp[2 * q + 1];
     for (int g0 = 0; g0 < f_len; g0 += cap) {
       const int seg = min(cap, f_len - g0);
       const long base = (long)f_lo + g0;
       __syncthreads();  // the previous segment's readers are done with the buffer
-      if (AHEAD) store(seg, iv);
-      for (int j0 = AHEAD ? nt : 0; j0 < seg; j0 += nt) {
-        load(base, seg, j0 + iv);
-        store(seg, j0 + iv);
-      }
-      if (AHEAD && g0 + cap < f_len) {
-        load(base + cap, min(cap, f_len - g0 - cap), iv);
-      } else if (more) {
-        entry(q + 1);
-        load(n_lo, min(cap, n_len), iv);
+      for (int j0 = 0; j0 < seg; j0 += blockDim.x) {
+        const int j = j0 + threadIdx.x;
+        double v[kCcfSpec];
+#pragma unroll
+        for (int k = 0; k < kCcfSpec; k++) v[k] = (j < seg && k < ns) ? S[k][base + j] : 0.0;
+        if (j < seg) {
+#pragma unroll
+          for (int k = 0; k < kCcfSpec; k++) lds[k * cap + j] = v[k];
+        }
       }
       __syncthreads();
       if (act) {
-        const int ln = (int)(c_pk & 0xffu);
-        const uint32_t al = c_pk >> 8;
+        const int ln = (int)(pk & 0xffu);
+        const uint32_t al = pk >> 8;
         for (int b = 0; b < ln; b++) {
-          const long pp = c_st + b;
+          const long pp = st + b;
           if (!((al >> b) & 1u) || pp < 0 || pp >= n_t || pp < base || pp >= base + seg) continue;
-          const double val = (b == ln - 1) ? c_wy : ((b == 0) ? c_wx : w);
+          const double val = (b == ln - 1) ? wy : ((b == 0) ? wx : w);
           const double *L = lds + (pp - base);
 #pragma unroll
           for (int k = 0; k < kCcfSpec; k++) acc[k] = fma(L[k * cap], val, acc[k]);
         }
       }
-    }
-    if (AHEAD) {
-      f_lo = n_lo;
-      f_len = n_len;
     }
   }
   if (act) {
@@ -2543,34 +2500,354 @@ __device__ __forceinline__ void ccf_lds_body(const double *spec_, int64_t spec_s
   }
 }
 
-template <bool AHEAD>
-__global__ void k_ccf_lds(const double *spec, int64_t spec_stride, int64_t trim, int n_spec, int n_lines, int n_v,
-                          int64_t n_t, const int32_t *m_start, const uint32_t *m_pk, const double2 *m_wv,
-                          const double *w_sorted, const int2 *fp, int cap, double *part, int lines) {
-  extern __shared__ double ccf_lds[];
-  ccf_lds_body<AHEAD>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t, m_start, m_pk, m_wv, w_sorted, fp, cap, part, lines,
-               blockIdx.x, blockIdx.y, ccf_lds);
+// The same sums for launches with few chunks and spectra (ccf_form), where the walk over a
+// chunk's lines is the time: one round trip to memory and one decoding of the windows per
+// line.  Block = (chunk, S spectra).  The footprints of a round of lines (all 32, where the
+// LDS holds them) are staged together, a wave to a row; T neighbouring lanes share a velocity,
+// each decodes the window of one of T lines, then the sums go from lane to lane in the lines'
+// order.  A chunk keeps its 32 lines and a sum the order of its terms, so that a spectrum's
+// CCF has the same bits in a call of any size.  78 spectra of 230 lines: 75 us per launch in
+// the plain form, 28 in this one; 10 spectra: 73 and 10.
+constexpr int kCcfRound = 64 << 10;  // bytes of staged rows
+constexpr int kCcfPad = 24;          // pixels of the longest window
+__host__ __device__ constexpr int ccf_row_cap(int S) { return kCcfRound / 32 / S; }  // 4 lines to a round at least
+__host__ __device__ constexpr int ccf_round(int S, int cap) {                         // lines of a round
+  const int n = kCcfRound / 8 / S / cap & ~3;
+  return n < kCcfLines ? n : kCcfLines;
+}
+struct CcfEntry {  // a lane's window of its line
+  int st;
+  uint32_t pk;
+  double wx, wy;
+};
+template <int T, int S>
+__device__ __forceinline__ void ccf_rounds_body(const double *spec_, int64_t spec_stride, int64_t trim, int n_spec,
+                                                int n_lines, int n_v, const int32_t *m_start_, const uint32_t *m_pk_,
+                                                const double2 *m_wv, const double *w_sorted_, const int2 *fp_, int cap,
+                                                double *part_, int bx_, int by_, double *lds) {
+  constexpr int U = S == 1 ? 8 : 4;  // pixels of a window in registers
+  constexpr int Q = 4;               // rows per wave in flight, of 256 pixels
+  const GLOBAL double *spec = gl(spec_);
+  const GLOBAL int32_t *m_start = gl(m_start_);
+  const GLOBAL uint32_t *m_pk = gl(m_pk_);
+  const CONSTANT int32_t *fp = gc((const int32_t *)fp_);  // {lo, len} pairs
+  GLOBAL double *part = gw(part_);
+  const int q0 = bx_ * kCcfLines, q1 = min(n_lines, q0 + kCcfLines), nl = ccf_round(S, cap);
+  const int s0 = by_ * S, ns = min(S, n_spec - s0);
+  const int tid = threadIdx.x, nt = blockDim.x, iv = tid / T, turn = tid % T, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nt >> 6;
+  auto row_of = [&](int k) { return spec + (long)(s0 + min(k, ns - 1)) * spec_stride + trim; };
+  // the chunk's weights and footprints, then the rows with room for a window before and after
+  double *s_w = lds, *rows = lds + 2 * kCcfLines + kCcfPad;
+  int2 *s_fp = (int2 *)(lds + kCcfLines);
+  if (tid < q1 - q0) {
+    s_w[tid] = gl(w_sorted_)[q0 + tid];
+    s_fp[tid] = make_int2(fp[2 * (q0 + tid)], fp[2 * (q0 + tid) + 1]);
+  }
+  const int ivc = min(iv, n_v - 1);
+  auto entry = [&](int q) {
+    const int qc = min(q, q1 - 1), l = min(turn, q1 - 1 - qc);
+    const long e = (long)qc * n_v;
+    const unsigned o = (unsigned)(l * n_v + ivc);
+    const double2 wv = (m_wv + e)[o];
+    return CcfEntry{(m_start + e)[o], (m_pk + e)[o], wv.x, wv.y};
+  };
+  CcfEntry t = entry(q0);
+  double acc[S], x[U][S], val[U], w;
+#pragma unroll
+  for (int k = 0; k < S; k++) acc[k] = 0.0;
+  int ln, off, hi;
+  uint32_t live;
+  bool plain;
+  // this lane's window in the staged pixels [base, base + seg) of its line
+  auto window = [&](int q, int base, int seg) {
+    w = s_w[min(q + turn, q1 - 1) - q0];
+    ln = (int)(t.pk & 0xffu);
+    off = t.st - base;
+    hi = iv < n_v && q + turn < q1 ? min(ln, seg - off) : 0;  // past the velocities or the chunk: no pixels
+    const int lo = max(0, -off);
+    live = hi > lo ? (t.pk >> 8) & ((1u << hi) - (1u << lo)) : 0u;  // at most 24 pixels
+    if (live == 0) off = hi = 0;
+    plain = !__any(!(fabs(w) < HUGE_VAL) || !(fabs(t.wx) < HUGE_VAL) || !(fabs(t.wy) < HUGE_VAL));
+  };
+  // its pixels b0 .. b0 + U - 1.  One that is not live (it may lie beside the row, in the pad or
+  // in another row) adds zero and leaves the sum's bits, where the weights are numbers.
+  auto decode = [&](const double *row, int b0) {
+    const double *L = row + off + b0;
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int k = 0; k < S; k++) x[u][k] = L[k * cap + u];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool on = (live >> b0) & (1u << u);
+#pragma unroll
+      for (int k = 0; k < S; k++) x[u][k] = on ? x[u][k] : 0.0;
+      val[u] = b0 + u == ln - 1 ? t.wy : b0 + u == 0 ? t.wx : w;
+    }
+    if (!plain)
+#pragma unroll
+      for (int u = 0; u < U; u++) val[u] = (live >> b0) & (1u << u) ? val[u] : 0.0;
+  };
+  auto add = [&](double (&y)[S]) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int k = 0; k < S; k++) y[k] = fma(x[u][k], val[u], y[k]);
+  };
+  auto rest = [&](const double *row, double (&y)[S]) {  // pixels from the U'th on
+    for (int b = U; b < hi; b++)
+      if ((live >> b) & 1u)
+#pragma unroll
+        for (int k = 0; k < S; k++) y[k] = fma(row[k * cap + off + b], b == ln - 1 ? t.wy : w, y[k]);
+  };
+  for (int r0 = q0; r0 < q1; r0 += nl) {
+    const int r1 = min(q1, r0 + nl), nr = (r1 - r0) * S;
+    const bool wide = __any(gl((const int32_t *)fp_)[2 * min(r0 + lane, r1 - 1) + 1] > cap);  // a footprint longer than a row
+    __syncthreads();  // the readers of the round before are done with the rows
+    if (!wide) {
+      for (int i0 = wave; i0 < nr; i0 += Q * nw) {
+        double v[Q][4];
+#pragma unroll
+        for (int a = 0; a < Q; a++) {
+          const int i = min(i0 + a * nw, nr - 1), lo = fp[2 * (r0 + i / S)], last = max(fp[2 * (r0 + i / S) + 1] - 1, 0);
+#pragma unroll
+          for (int u = 0; u < 4; u++) v[a][u] = (row_of(i % S) + lo)[(unsigned)min(lane + 64 * u, last)];
+        }
+#pragma unroll
+        for (int a = 0; a < Q; a++) {
+          const int i = i0 + a * nw;
+          if (i >= nr) break;
+          const int lo = fp[2 * (r0 + i / S)], len = fp[2 * (r0 + i / S) + 1];
+          double *row = rows + i * cap;
+#pragma unroll
+          for (int u = 0; u < 4; u++)
+            if (lane + 64 * u < len) row[lane + 64 * u] = v[a][u];
+          for (int j = lane + 256; j < len; j += 64) row[j] = (row_of(i % S) + lo)[(unsigned)j];
+        }
+      }
+      __syncthreads();
+      for (int q = r0; q < r1; q += T) {
+        const CcfEntry next = entry(q + T);
+        const int at = min(q + turn, r1 - 1);
+        const int2 f = s_fp[at - q0];
+        const double *row = rows + (at - r0) * S * cap;
+        window(q, f.x, f.y);
+        if constexpr (T == 1) {
+          for (int b0 = 0; b0 < hi; b0 += U) {
+            decode(row, b0);
+            add(acc);
+          }
+        } else {
+          decode(row, 0);
+          const bool more = __any(hi > U);
+#pragma unroll
+          for (int l = 0; l < T; l++) {  // lane l of the T takes its turn
+            double y[S];
+#pragma unroll
+            for (int k = 0; k < S; k++) y[k] = acc[k];
+            add(y);
+            if (more) rest(row, y);
+#pragma unroll
+            for (int k = 0; k < S; k++)
+              acc[k] = T == 4 ? (l == 0   ? dpp_f64<0x00>(y[k])
+                                 : l == 1 ? dpp_f64<0x55>(y[k])
+                                 : l == 2 ? dpp_f64<0xaa>(y[k])
+                                          : dpp_f64<0xff>(y[k]))
+                              : (l == 0 ? dpp_f64<0xa0>(y[k]) : dpp_f64<0xf5>(y[k]));
+          }
+        }
+        t = next;
+      }
+    } else {
+      for (int q = r0; q < r1; q++) {
+        const int f_lo = fp[2 * q], f_len = fp[2 * q + 1], l = (q - q0) % T;
+        if (l == 0) t = entry(q);
+        for (int g0 = 0; g0 < f_len; g0 += cap) {
+          const int seg = min(cap, f_len - g0);
+          __syncthreads();
+          for (int j = tid; j < seg; j += nt)
+#pragma unroll
+            for (int k = 0; k < S; k++) rows[k * cap + j] = (row_of(k) + f_lo + g0)[(unsigned)j];
+          __syncthreads();
+          window(q - l, f_lo + g0, seg);
+          double y[S];
+#pragma unroll
+          for (int k = 0; k < S; k++) y[k] = acc[k];
+          decode(rows, 0);
+          add(y);
+          rest(rows, y);
+#pragma unroll
+          for (int k = 0; k < S; k++) acc[k] = __shfl(y[k], lane / T * T + l);
+        }
+      }
+      t = entry(r1);
+    }
+  }
+  if (iv < n_v && turn == 0) {
+#pragma unroll
+    for (int k = 0; k < S; k++)
+      if (k < ns) part[((long)bx_ * n_spec + s0 + k) * n_v + iv] = acc[k];
+  }
 }
 
-// LDS segment length for a longest footprint of fmax pixels
+// The plain form with the next line's pixels and entry loaded, and two pixels of a window read,
+// ahead of the sums: for launches whose blocks are too few to hide them (93 spectra of 650
+// lines: 99 us per launch in the plain form, 79 in this one), where the registers do not cost
+// waves.
+__device__ __forceinline__ void ccf_ahead_body(const double *spec_, int64_t spec_stride, int64_t trim, int n_spec,
+                                               int n_lines, int n_v, const int32_t *m_start_, const uint32_t *m_pk_,
+                                               const double2 *m_wv, const double *w_sorted_, const int2 *fp_, int cap,
+                                               double *part_, int bx_, int by_, double *lds) {
+  constexpr int S = kCcfSpec, U = 2;
+  const GLOBAL double *spec = gl(spec_);
+  const GLOBAL int32_t *m_start = gl(m_start_);
+  const GLOBAL uint32_t *m_pk = gl(m_pk_);
+  const CONSTANT int32_t *fp = gc((const int32_t *)fp_);  // {lo, len} pairs
+  const CONSTANT double *w_sorted = gc(w_sorted_);
+  GLOBAL double *part = gw(part_);
+  const int q0 = bx_ * kCcfLines, q1 = min(n_lines, q0 + kCcfLines), s0 = by_ * S, ns = min(S, n_spec - s0);
+  const int iv = threadIdx.x, nt = blockDim.x;
+  const GLOBAL double *sp[S];
+#pragma unroll
+  for (int k = 0; k < S; k++) sp[k] = spec + (long)(s0 + min(k, ns - 1)) * spec_stride + trim;
+  const unsigned ivc = min(iv, n_v - 1);
+  auto entry = [&](int q) {
+    const long e = (long)min(q, q1 - 1) * n_v;
+    const double2 wv = (m_wv + e)[ivc];
+    return CcfEntry{(m_start + e)[ivc], (m_pk + e)[ivc], wv.x, wv.y};
+  };
+  double acc[S], v[S];
+#pragma unroll
+  for (int k = 0; k < S; k++) acc[k] = 0.0;
+  auto load = [&](int q) {  // the first nt pixels of a line's footprint
+    const int line = min(q, q1 - 1), lo = fp[2 * line], last = max(min(cap, fp[2 * line + 1]) - 1, 0);
+#pragma unroll
+    for (int k = 0; k < S; k++) v[k] = (sp[k] + lo)[(unsigned)min(iv, last)];
+  };
+  load(q0);
+  CcfEntry t = entry(q0);
+  for (int q = q0; q < q1; q++) {
+    const int f_lo = fp[2 * q], f_len = fp[2 * q + 1];
+    const double w = w_sorted[q];
+    const CcfEntry next = entry(q + 1);
+    for (int g0 = 0; g0 < f_len; g0 += cap) {
+      const int seg = min(cap, f_len - g0);
+      __syncthreads();  // the previous segment's readers are done with the buffer
+      if (g0 == 0) {
+        if (iv < seg)
+#pragma unroll
+          for (int k = 0; k < S; k++) lds[k * cap + iv] = v[k];
+      }
+      for (int j = g0 == 0 ? iv + nt : iv; j < seg; j += nt)
+#pragma unroll
+        for (int k = 0; k < S; k++) lds[k * cap + j] = (sp[k] + f_lo + g0)[(unsigned)j];
+      if (g0 + cap >= f_len) load(q + 1);
+      __syncthreads();
+      const int ln = (int)(t.pk & 0xffu), off = t.st - f_lo - g0, lo = max(0, -off);
+      const int hi = iv < n_v ? min(ln, seg - off) : 0;
+      const uint32_t live = hi > lo ? (t.pk >> 8) & ((1u << hi) - (1u << lo)) : 0u;  // at most 24 pixels
+      for (int b0 = lo; b0 < hi; b0 += U) {
+        double x[U][S];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int k = 0; k < S; k++) x[u][k] = lds[k * cap + min(off + b0 + u, seg - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int b = b0 + u;
+          if (!((live >> b) & 1u)) continue;
+          const double val = b == ln - 1 ? t.wy : b == 0 ? t.wx : w;
+#pragma unroll
+          for (int k = 0; k < S; k++) acc[k] = fma(x[u][k], val, acc[k]);
+        }
+      }
+    }
+    if (f_len == 0) load(q + 1);  // nothing of this line in the spectrum
+    t = next;
+  }
+  if (iv < n_v) {
+#pragma unroll
+    for (int k = 0; k < S; k++)
+      if (k < ns) part[((long)bx_ * n_spec + s0 + k) * n_v + iv] = acc[k];
+  }
+}
+
+// T = 0: the plain form, 1 with S = kCcfSpec: the plain form with loads ahead
+template <int T, int S>
+__device__ __forceinline__ void ccf_body(const double *spec, int64_t spec_stride, int64_t trim, int n_spec, int n_lines,
+                                         int n_v, int64_t n_t, const int32_t *m_start, const uint32_t *m_pk,
+                                         const double2 *m_wv, const double *w_sorted, const int2 *fp, int cap,
+                                         double *part, int bx, int by, double *lds) {
+  if constexpr (T == 0)
+    ccf_lds_body(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t, m_start, m_pk, m_wv, w_sorted, fp, cap, part, bx,
+                 by, lds);
+  else if constexpr (S == kCcfSpec)
+    ccf_ahead_body(spec, spec_stride, trim, n_spec, n_lines, n_v, m_start, m_pk, m_wv, w_sorted, fp, cap, part, bx, by,
+                   lds);
+  else
+    ccf_rounds_body<T, S>(spec, spec_stride, trim, n_spec, n_lines, n_v, m_start, m_pk, m_wv, w_sorted, fp, cap, part,
+                          bx, by, lds);
+}
+#define SOAP_CCF_WAVES __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(T && S < kCcfSpec ? 5 : 4)))
+
+template <int T, int S>
+__global__ SOAP_CCF_WAVES void k_ccf_lds(const double *spec, int64_t spec_stride, int64_t trim, int n_spec, int n_lines,
+                                         int n_v, int64_t n_t, const int32_t *m_start, const uint32_t *m_pk,
+                                         const double2 *m_wv, const double *w_sorted, const int2 *fp, int cap,
+                                         double *part) {
+  extern __shared__ double ccf_lds[];
+  ccf_body<T, S>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t, m_start, m_pk, m_wv, w_sorted, fp, cap, part,
+                 blockIdx.x, blockIdx.y, ccf_lds);
+}
+
+// LDS segment length of the plain form for a longest footprint of fmax pixels
 int ccf_lds_cap(int fmax) { return fmax < 1 ? 1 : (fmax < kCcfLdsCap ? fmax : kCcfLdsCap); }
 size_t ccf_lds_bytes(int cap) { return (size_t)kCcfSpec * (cap > 0 ? cap : 1) * 8; }
+int ccf_chunks(int n_lines) { return (n_lines + kCcfLines - 1) / kCcfLines; }
+
+// The form of a launch.  From two blocks per CU on, the plain form: other blocks hide its loads
+// (750 blocks: 120 us, 134 with loads ahead).  Below, blocks of one spectrum as long as they
+// are not more than four per CU: beyond that their decoding, once per spectrum, is the time
+// (660 of them: 38 us, 59 with loads ahead; 1950: 132 and 79).  Long footprints always: the
+// plain form's rows cut them into segments (303 spectra, footprints of 940 pixels: 420 us,
+// 830 with loads ahead).  Lanes per velocity as many as a block of all velocities holds.
+struct CcfForm {
+  int T, spectra;  // lanes per velocity (0: plain), spectra per block
+  int threads, cap;
+  size_t lds;
+};
+static CcfForm ccf_form(int n_lines, int n_v, int n_spec, int fmax) {
+  constexpr int kBlocks = 512;
+  const long nc = ccf_chunks(n_lines);
+  CcfForm f{0, kCcfSpec, 0, ccf_lds_cap(fmax), 0};
+  if (nc * ((n_spec + kCcfSpec - 1L) / kCcfSpec) < kBlocks) {
+    if (nc * n_spec <= 2 * kBlocks || fmax > kCcfLdsCap) {
+      f.T = n_v <= 256 ? 4 : n_v <= 512 ? 2 : 1;
+      f.spectra = 1;
+      f.cap = std::min(std::max(fmax, 1), ccf_row_cap(1));
+    } else {
+      f.T = 1;
+    }
+  }
+  f.threads = (std::max(f.T, 1) * n_v + 63) / 64 * 64;
+  f.lds = f.spectra == 1 ? (size_t)(2 * kCcfLines + 2 * kCcfPad + ccf_round(1, f.cap) * f.cap) * sizeof(double)
+                         : ccf_lds_bytes(f.cap);
+  return f;
+}
+#define SOAP_CCF_KERNEL(K, F)                                                                        \
+  ((F).T == 4 ? K<4, 1> : (F).T == 2 ? K<2, 1> : (F).T == 0 ? K<0, kCcfSpec> : (F).spectra == 1 ? K<1, 1> : K<1, kCcfSpec>)
 
 hipError_t launch_ccf_lds(const double *spec, int64_t spec_stride, int64_t trim, int n_spec, int n_lines, int n_v,
                           int64_t n_t, const int32_t *m_start, const uint32_t *m_pk, const double2 *m_wv,
-                          const double *w_sorted, const int2 *fp, int cap, double *part, hipStream_t s) {
+                          const double *w_sorted, const int2 *fp, int fmax, double *part, hipStream_t s) {
   if (n_spec == 0) return hipSuccess;
-  if (n_v > 1024 || cap < 1 || cap > kCcfLdsCap) return hipErrorInvalidValue;
-  int nc = ccf_chunks(n_lines, n_spec);
-  int threads = ((n_v + 63) / 64) * 64;
-  dim3 grid(nc, (n_spec + kCcfSpec - 1) / kCcfSpec);
-  const int lines = ccf_lines(n_lines, n_spec);
-  if (lines < kCcfLines)
-    k_ccf_lds<true><<<grid, threads, ccf_lds_bytes(cap), s>>>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t,
-                                                              m_start, m_pk, m_wv, w_sorted, fp, cap, part, lines);
-  else
-    k_ccf_lds<false><<<grid, threads, ccf_lds_bytes(cap), s>>>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t,
-                                                               m_start, m_pk, m_wv, w_sorted, fp, cap, part, lines);
+  if (n_v > 1024 || fmax < 0) return hipErrorInvalidValue;
+  const CcfForm f = ccf_form(n_lines, n_v, n_spec, fmax);
+  const dim3 grid(ccf_chunks(n_lines), (n_spec + f.spectra - 1) / f.spectra);
+  auto k = SOAP_CCF_KERNEL(k_ccf_lds, f);
+  k<<<grid, f.threads, f.lds, s>>>(spec, spec_stride, trim, n_spec, n_lines, n_v, n_t, m_start, m_pk, m_wv, w_sorted, fp,
+                                   f.cap, part);
   return hipGetLastError();
 }
 
@@ -2671,7 +2948,7 @@ hipError_t launch_mask_wsum(int n_lines, int n_v, int64_t n_t, const int32_t *m_
 // place moves with the group and eight CCF blocks in a row meet all eight.  blockDim.x is the
 // CCF's thread count (velocities rounded up to a wave); a norm block covers
 // kNormPer * blockDim.x pixels of one spectrum.
-template <bool AHEAD>
+template <int T, int S>
 __device__ __forceinline__ void norm_ccf_body(const NormCcfArgs &a, long b, double *ccf_lds) {
   const long grp = (long)a.ratio + 1;
   const long mixed = (long)a.n_ccf * grp;
@@ -2688,49 +2965,35 @@ __device__ __forceinline__ void norm_ccf_body(const NormCcfArgs &a, long b, doub
     ni = (long)a.n_ccf * a.ratio + (b - mixed);
   }
   if (ci >= 0)
-    ccf_lds_body<AHEAD>(a.raw, a.n, a.trim, a.n_spec, a.n_lines, a.n_v, a.n_t, a.m_start, a.m_pk, a.m_wv, a.w_sorted, a.fp,
-                 a.cap, a.part, a.lines, (int)(ci % a.nc), (int)(ci / a.nc), ccf_lds);
+    ccf_body<T, S>(a.raw, a.n, a.trim, a.n_spec, a.n_lines, a.n_v, a.n_t, a.m_start, a.m_pk, a.m_wv, a.w_sorted, a.fp, a.cap,
+                a.part, (int)(ci % a.nc), (int)(ci / a.nc), ccf_lds);
   else if (ni < a.n_norm)
     norm_body(a.n, a.mm, a.raw, a.out, (int)(ni % a.nbx), (int)(ni / a.nbx), blockDim.x);
 }
 
-template <bool AHEAD>
-__global__ void k_norm_ccf(NormCcfArgs a) {
+template <int T, int S>
+__global__ SOAP_CCF_WAVES void k_norm_ccf(NormCcfArgs a) {
   extern __shared__ double ccf_lds[];
-  norm_ccf_body<AHEAD>(a, blockIdx.x, ccf_lds);
+  norm_ccf_body<T, S>(a, blockIdx.x, ccf_lds);
 }
 
 hipError_t launch_norm_ccf(NormCcfArgs a, hipStream_t s) {
   if (a.n_spec == 0) return hipSuccess;
   if (a.n_v > 1024 || (((uintptr_t)a.raw ^ (uintptr_t)a.out) & 15)) return hipErrorInvalidValue;
-  if (a.cap < 1 || a.cap > kCcfLdsCap) return hipErrorInvalidValue;
-  const int threads = ((a.n_v + 63) / 64) * 64;
-  a.nc = ccf_chunks(a.n_lines, a.n_spec);
-  a.lines = ccf_lines(a.n_lines, a.n_spec);
-  a.n_ccf = a.nc * ((a.n_spec + kCcfSpec - 1) / kCcfSpec);
+  if (a.fmax < 0) return hipErrorInvalidValue;
+  const CcfForm f = ccf_form(a.n_lines, a.n_v, a.n_spec, a.fmax);
+  const int threads = f.threads;
+  a.cap = f.cap;
+  a.nc = ccf_chunks(a.n_lines);
+  a.n_ccf = a.nc * ((a.n_spec + f.spectra - 1) / f.spectra);
   a.nbx = (int)((a.n + (int64_t)threads * kNormPer - 1) / ((int64_t)threads * kNormPer));
   a.n_norm = a.nbx * a.n_spec;
   a.ratio = a.n_ccf > 0 ? a.n_norm / a.n_ccf : 0;
   const long blocks = (long)a.n_ccf + a.n_norm;
   if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-  if (a.lines < kCcfLines)
-    k_norm_ccf<true><<<(unsigned)blocks, threads, ccf_lds_bytes(a.cap), s>>>(a);
-  else
-    k_norm_ccf<false><<<(unsigned)blocks, threads, ccf_lds_bytes(a.cap), s>>>(a);
+  auto k = SOAP_CCF_KERNEL(k_norm_ccf, f);
+  k<<<(unsigned)blocks, threads, f.lds, s>>>(a);
   return hipGetLastError();
-}
-
-// Lines per chunk: fewer where 32 would leave CUs without a block (the walk over a
-// block's lines is then the launch's time), down to 2.
-int ccf_lines(int n_lines, int n_spec) {
-  const long groups = (n_spec + kCcfSpec - 1) / kCcfSpec;
-  int l = kCcfLines;
-  while (l > 2 && (n_lines + l - 1) / l * groups < kCcfBlocks) l >>= 1;
-  return l;
-}
-int ccf_chunks(int n_lines, int n_spec) {
-  const int l = ccf_lines(n_lines, n_spec);
-  return (n_lines + l - 1) / l;
 }
 
 hipError_t launch_ccf_reduce(const double *part, int nc, int n_spec, int n_v, const double *appod, const double *mm,
@@ -3216,8 +3479,8 @@ template <bool P>
 __global__ __launch_bounds__(1024) void kb_ccf(SOAP_BATCH_ARGS(CcfJob)) {
   extern __shared__ double ccf_lds[];
   batch_loop<P>(jobs, prefix, n_inst, total, [&](const CcfJob &j, int local) {
-    ccf_lds_body<false>(j.spec, j.stride, j.trim, j.n_spec, j.n_lines, j.n_v, j.n_t, j.m_start, j.m_pk, j.m_wv, j.w_sorted,
-                 j.fp, j.cap, j.part, j.lines, local % j.nc, local / j.nc, ccf_lds);
+    ccf_lds_body(j.spec, j.stride, j.trim, j.n_spec, j.n_lines, j.n_v, j.n_t, j.m_start, j.m_pk, j.m_wv, j.w_sorted,
+                 j.fp, j.cap, j.part, local % j.nc, local / j.nc, ccf_lds);
   });
 }
 

@@ -73,15 +73,16 @@ def test_series_pipeline_equals_staged_calls(n_phase, n, vsini):
 
 
 # spec_norm and the CCF share one launch in groups of one CCF block and `ratio` norm
-# blocks; the CCF block's place in its group depends on gcd(ratio + 1, 8).  81
-# velocities: 128 threads, 1024 pixels per norm block; 63 spectra and 128 lines, two lines
-# per chunk: 512 CCF blocks.
-@pytest.mark.parametrize("n,group", [(58000, 8), (92000, 12), (124500, 16), (41500, 6), (24000, 3), (6000, 1)])
+# blocks; the CCF block's place in its group depends on gcd(ratio + 1, 8).  101 velocities
+# on 4 lanes each: 448 threads, 3584 pixels per norm block; 63 spectra and 128 lines, one
+# spectrum and 32 lines per block: 252 CCF blocks.
+@pytest.mark.parametrize("n,group", [(99000, 8), (156000, 12), (213000, 16), (70000, 6), (27000, 3), (6000, 1)])
 def test_series_norm_ccf_groups(n, group):
-    n_phase, lines = 20, 128
+    n_phase, lines, per_block = 20, 128, 8 * 448
     w = synth.small(seed=3, grid=32, n=n, n_mu=4, n_phase=n_phase, n_lines=200, lmin=5000.0,
                     lmax=5000.0 * np.exp((n - 1) * 1e-6))
-    n_norm, n_ccf = -(-n // 1024) * 3 * (n_phase + 1), lines // 2 * 8
+    w.vgrid = np.linspace(-20e3, 20e3, 101)
+    n_norm, n_ccf = -(-n // per_block) * 3 * (n_phase + 1), lines // 32 * 3 * (n_phase + 1)
     assert n_norm // n_ccf + 1 == group
     sel = (w.mask_w > 0.1) & (w.mask_l > w.wave[300]) & (w.mask_l < w.wave[-300])
     e = Engine(0)
