@@ -35,7 +35,7 @@ constexpr int kDT = 256;
 //   sum_c L phi = M0 - u1 M1 - u2 M2,  M_q = sum_c a^q phi,
 // likewise for psi and b psi.  The kernels below form those sums once per (piece,
 // phase), lanes over phases and cells in turn (no reduction across lanes and no
-// atomics: every sum has a fixed order), and everything after works on pieces: 12,500 of
+// atomics: every sum has a fixed order), and everything after works on pieces: 7,300 of
 // them instead of 283,000 cells at grid 600 with 10 bins.
 
 // per-cell tables of the plan
@@ -69,7 +69,7 @@ __global__ void k_diff_psum(DiffArgs a, double2 *psum) {
   const DiffPiece pc = a.piece[i];
   double s1 = 0.0, s2 = 0.0;
   for (int c = 0; c < pc.len; c++) {
-    const double ca = a.cell[(long)pc.iy * a.grid + pc.iz0 + c].x;
+    const double ca = a.cell[(long)pc.iy * a.grid + a.col[(long)pc.group * kDiffGroup + c]].x;
     s1 += ca;
     s2 = fma(ca, ca, s2);
   }
@@ -140,8 +140,8 @@ __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Moments of one piece for up to 64 phases: one wave per (piece, 64 phases).  The wave
-// samples its cells' filling factors bilinearly (two phases x 32 cells per step, loads
+// Moments of one piece for up to 64 phases: one wave per (piece, 64 phases).  Group by
+// group the wave samples its cells' filling factors bilinearly (two phases x 32 cells per step, loads
 // of neighbouring cells from neighbouring nodes) into LDS and then sums them with lanes
 // over phases, the cell's own factors read from the lane that holds them.  Blocks are in
 // contiguous runs per XCD: neighbouring pieces read the same map rows.  Outputs: mom rows
@@ -149,7 +149,7 @@ __device__ __forceinline__ void wave_lds_order() {
 // sum L (1 - phi - psi), kappa sum L phi, kappa_f sum L b psi.
 constexpr int kMomW = 4;       // waves (pieces) per block
 constexpr int kMomU = 4;       // sampling steps in flight
-constexpr int kMomStride = kDiffPiece + 1;
+constexpr int kMomStride = kDiffGroup + 1;
 template <int NS>
 __global__ __launch_bounds__(64 * kMomW) void k_diff_moments(DiffArgs a, int blocks_per_xcd) {
   extern __shared__ double s_mom[];  // per wave [phases][kMomStride]
@@ -160,56 +160,59 @@ __global__ __launch_bounds__(64 * kMomW) void k_diff_moments(DiffArgs a, int blo
   if (ip >= a.n_piece) return;  // no barriers below
   double *sp = s_mom + (size_t)w * min(64, P) * kMomStride;
   const CONSTANT int32_t *pi = gc((const int32_t *)(a.piece + ip));
-  const DiffPiece pc = {pi[0], pi[1], pi[2], pi[3]};
+  const int iy = pi[0], group = pi[2], len = pi[3];
   const int M = a.map_res;
   const long MM = (long)M * M;
-  // this lane's cell and its stencil (the same for every phase)
   const int c = lane & 31, ph = lane >> 5;
-  const int cc = min(c, pc.len - 1);
-  const double2 me = a.cell[(long)pc.iy * a.grid + pc.iz0 + cc];
-  const int j0 = a.map_j[pc.iz0 + cc], i0 = gc(a.map_j)[pc.iy];
-  const double fz = a.map_f[pc.iz0 + cc], fy = gc(a.map_f)[pc.iy];
-  const double w00 = (1 - fy) * (1 - fz), w10 = fy * (1 - fz), w01 = (1 - fy) * fz, w11 = fy * fz;
-  const long off = (long)i0 * M + j0;
+  const int i0 = gc(a.map_j)[iy];
+  const double fy = gc(a.map_f)[iy];
   double m[9];
 #pragma unroll
   for (int q = 0; q < 9; q++) m[q] = 0.0;
+  for (int c0 = 0; c0 < len; c0 += kDiffGroup) {
+    // this lane's cell and its stencil (the same for every phase)
+    const int n_cell = min(kDiffGroup, len - c0), iz = a.col[(long)group * kDiffGroup + c0 + c];
+    const double2 me = a.cell[(long)iy * a.grid + iz];
+    const double fz = a.map_f[iz];
+    const double w00 = (1 - fy) * (1 - fz), w10 = fy * (1 - fz), w01 = (1 - fy) * fz, w11 = fy * fz;
+    const long off = (long)i0 * M + a.map_j[iz];
 #pragma unroll
-  for (int set = 0; set < NS - 1; set++) {
-    const double *mp = (set ? a.fmaps : a.maps) + (long)p0 * MM + off;
-    for (int s = 0; s < np; s += 2 * kMomU) {
-      double x[kMomU][4];
+    for (int set = 0; set < NS - 1; set++) {
+      const double *mp = (set ? a.fmaps : a.maps) + (long)p0 * MM + off;
+      for (int s = 0; s < np; s += 2 * kMomU) {
+        double x[kMomU][4];
 #pragma unroll
-      for (int u = 0; u < kMomU; u++) {
-        const double *q = mp + (long)min(s + 2 * u + ph, np - 1) * MM;
-        x[u][0] = q[0];
-        x[u][1] = q[M];
-        x[u][2] = q[1];
-        x[u][3] = q[M + 1];
+        for (int u = 0; u < kMomU; u++) {
+          const double *q = mp + (long)min(s + 2 * u + ph, np - 1) * MM;
+          x[u][0] = q[0];
+          x[u][1] = q[M];
+          x[u][2] = q[1];
+          x[u][3] = q[M + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < kMomU; u++) {
+          const int p = s + 2 * u + ph;
+          if (p < np) sp[p * kMomStride + c] = w00 * x[u][0] + w10 * x[u][1] + w01 * x[u][2] + w11 * x[u][3];
+        }
       }
-#pragma unroll
-      for (int u = 0; u < kMomU; u++) {
-        const int p = s + 2 * u + ph;
-        if (p < np) sp[p * kMomStride + c] = w00 * x[u][0] + w10 * x[u][1] + w01 * x[u][2] + w11 * x[u][3];
-      }
-    }
-    wave_lds_order();
-    const double *mine = sp + min(lane, np - 1) * kMomStride;
+      wave_lds_order();
+      const double *mine = sp + min(lane, np - 1) * kMomStride;
 #pragma unroll 4
-    for (int i = 0; i < pc.len; i++) {
-      const double f = mine[i], ca = lane_f64(me.x, i);
-      const double fa = f * ca;
-      m[3 * set] += f;
-      m[3 * set + 1] += fa;
-      m[3 * set + 2] = fma(fa, ca, m[3 * set + 2]);
-      if (set) {
-        const double g = f * lane_f64(me.y, i), ga = g * ca;
-        m[6] += g;
-        m[7] += ga;
-        m[8] = fma(ga, ca, m[8]);
+      for (int i = 0; i < n_cell; i++) {
+        const double f = mine[i], ca = lane_f64(me.x, i);
+        const double fa = f * ca;
+        m[3 * set] += f;
+        m[3 * set + 1] += fa;
+        m[3 * set + 2] = fma(fa, ca, m[3 * set + 2]);
+        if (set) {
+          const double g = f * lane_f64(me.y, i), ga = g * ca;
+          m[6] += g;
+          m[7] += ga;
+          m[8] = fma(ga, ca, m[8]);
+        }
       }
+      wave_lds_order();
     }
-    wave_lds_order();
   }
   if (lane >= np) return;
   constexpr int NM = diff_moments(NS);
@@ -221,7 +224,7 @@ __global__ __launch_bounds__(64 * kMomW) void k_diff_moments(DiffArgs a, int blo
   const double s1 = gc((const double *)(a.psum + ip))[0], s2 = gc((const double *)(a.psum + ip))[1];
   double *wt = a.wts + (long)ip * NS * P + p0 + lane;
   const double Lphi = m[0] - u1 * m[1] - u2 * m[2];
-  wt[0] = ((double)pc.len - m[0] - m[3]) - u1 * (s1 - m[1] - m[4]) - u2 * (s2 - m[2] - m[5]);
+  wt[0] = ((double)len - m[0] - m[3]) - u1 * (s1 - m[1] - m[4]) - u2 * (s2 - m[2] - m[5]);
   wt[P] = kappa * Lphi;
   if (NS == 3) wt[2L * P] = kappa_f * (m[6] - u1 * m[7] - u2 * m[8]);
 }
@@ -904,7 +907,7 @@ __global__ __launch_bounds__(kDT) void k_diff_convT(DiffArgs a, ConvArgs c, cons
 }
 
 // lag correlations C[k][d][set][p] = sum_j G_I[p][j] X_k[j - dmin - d], in two passes.
-// Pass 1: block = (chunk of kCorrT pixels, group of kCorrRB (bin, set) rows, lag tile of
+// Pass 1: block = (chunk of kCorrT pixels or of kCorrG times that, group of kCorrRB (bin, set) rows, lag tile of
 // 16 and group of PB phases); the rows' segments are staged once and each of four waves
 // takes a quarter of the pixels.  Lane l of a row of 16 lanes is lag l, the four rows of
 // lanes take 16 pixels each of every 64: a step loads G_I of 64 pixels per phase, and
@@ -912,9 +915,12 @@ __global__ __launch_bounds__(kDT) void k_diff_convT(DiffArgs a, ConvArgs c, cons
 // rows' pixel at the lane's lag from LDS, which then serves PB phases.  The lane rows'
 // sums are added by swaps between them and the waves' through LDS.  PB kCorrRB = 50
 // accumulators keep three waves per SIMD.  Lags are those the group's bins use.  Pass 2
-// sums the chunk partials in chunk order (deterministic, no atomics).
+// sums the chunk partials (no atomics).  The order of a sum is the same for every launch:
+// kCorrT pixels, kCorrG of those in turn, the groups in turn.  A block takes a whole group
+// where that leaves blocks for all CUs (corr_whole): a fourth of the partials to hold.
 constexpr int kCorrRB = 5;
 constexpr int kCorrT = 1024;
+constexpr int kCorrG = 4;
 constexpr int kCorrWin = kCorrT + 16;  // staged pixels of a row
 // F[p] += g[p](lane N of this lane's row) x
 template <int N, int PB>
@@ -984,111 +990,145 @@ __device__ __forceinline__ double swap_fold(double a, double b) {
   return __longlong_as_double(((long long)h0 << 32) | l0) + __longlong_as_double(((long long)h1 << 32) | l1);
 }
 
-// Cpart [chunk][row][lag tile][P][16]
+constexpr int corr_sums(int pb) { return (kCorrRB * pb + 3) / 4 * 4 * 16; }  // of a wave
+constexpr int corr_lds(int pb) {  // doubles: the staged rows with room for the last step's read ahead, or the waves' sums
+  return kCorrRB * kCorrWin + 64 > 4 * corr_sums(pb) ? kCorrRB * kCorrWin + 64 : 4 * corr_sums(pb);
+}
+// Cpart [chunk][row][lag tile][P][16]; per: stretches of kCorrT pixels to a chunk
 template <int PB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_diff_corr(DiffArgs a, const double *GI,
-                                                                                        double *Cpart, int n_z) {
-  extern __shared__ double s_x[];  // [kCorrRB][kCorrWin], room for the last step's read ahead; then the waves' sums
-  constexpr int RB = kCorrRB, NF = (RB * PB + 3) / 4;  // sums per wave, four in a register
+                                                                                        double *Cpart, int n_z, int per) {
+  extern __shared__ double s_x[];  // [kCorrRB][kCorrWin], then the waves' sums; behind them the chunk's sums
+  constexpr int RB = kCorrRB, NF = corr_sums(PB) / 64;  // sums per wave, four in a register
+  double *s_run = s_x + corr_lds(PB);
   const int rows = a.n_mu * a.ns, r0 = blockIdx.y * RB, ns = a.ns;
   const int chunk = blockIdx.x, z = blockIdx.z % n_z, p0 = blockIdx.z / n_z * PB;
   int hi;
   const int lag0 = corr_lag0(a, r0 / ns, min(rows - 1, r0 + RB - 1) / ns, hi) + 16 * z;
   if (lag0 > hi) return;  // uniform over the block
-  const long j0 = (long)chunk * kCorrT, n = a.n;
-  // lag d = lag0 + l reads X[j - dmin - d]: window index (j - j0) + 15 - l
-  const long src0 = j0 - a.dmin - lag0 - 15;
-#pragma unroll
-  for (int r = 0; r < RB; r++) {
-    const int row = min(r0 + r, rows - 1), set = row % ns;
-    const double *X = (set == 0 ? a.q : set == 1 ? a.s : a.f) + (long)(row / ns) * n;
-    for (int e = threadIdx.x; e < kCorrWin; e += 256) {
-      const long i = src0 + e;
-      const bool in = i >= 0 && i < n;
-      const double v = X[in ? i : 0];
-      s_x[r * kCorrWin + e] = in ? v : 0.0;
-    }
-  }
-  __syncthreads();
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l = lane & 15;
-  double F[RB][PB], g[PB], gn[PB], xc[RB];
+  const long n = a.n;
+#pragma unroll 1
+  for (int c = 0; c < per; c++) {
+    const long j0 = ((long)chunk * per + c) * kCorrT;
+    if (j0 >= n) break;  // uniform
+    // lag d = lag0 + l reads X[j - dmin - d]: window index (j - j0) + 15 - l
+    const long src0 = j0 - a.dmin - lag0 - 15;
+    if (c) __syncthreads();  // the last stretch's sums have been read
 #pragma unroll
-  for (int r = 0; r < RB; r++)
-#pragma unroll
-    for (int p = 0; p < PB; p++) F[r][p] = 0.0;
-  const int j1 = (int)min((long)kCorrT, n - j0);  // pixels of the chunk
-  auto load = [&](double (&v)[PB], int s) {
-    const bool in = s + lane < j1;
-    const double *G = GI + j0 + (in ? s + lane : j1 - 1);
-#pragma unroll
-    for (int p = 0; p < PB; p++) {
-      const double x = G[(long)min(p0 + p, a.n_phase - 1) * n];
-      v[p] = in ? x : 0.0;
+    for (int r = 0; r < RB; r++) {
+      const int row = min(r0 + r, rows - 1), set = row % ns;
+      const double *X = (set == 0 ? a.q : set == 1 ? a.s : a.f) + (long)(row / ns) * n;
+      for (int e = threadIdx.x; e < kCorrWin; e += 256) {
+        const long i = src0 + e;
+        const bool in = i >= 0 && i < n;
+        const double v = X[in ? i : 0];
+        s_x[r * kCorrWin + e] = in ? v : 0.0;
+      }
     }
-  };
-  const int s0 = w * (kCorrT / 4), s1 = min(j1, s0 + kCorrT / 4);
-  const double *x = s_x + (lane & 48) + 15 - l;
+    __syncthreads();
+    double F[RB][PB], g[PB], gn[PB], xc[RB];
 #pragma unroll
-  for (int r = 0; r < RB; r++) xc[r] = x[r * kCorrWin + s0];
-  if (s0 < s1) load(g, s0);
-  for (int s = s0; s < s1; s += 64) {
-    load(gn, s + 64);
-    lag_steps<0>(F, g, xc, x + s);
+    for (int r = 0; r < RB; r++)
 #pragma unroll
-    for (int p = 0; p < PB; p++) g[p] = gn[p];
-  }
-  __syncthreads();  // the staged rows become the waves' sums
-  const int which = (0x3120 >> (4 * (lane >> 4))) & 15;  // rows 0..3 of a folded register hold sums 0, 2, 1, 3
+      for (int p = 0; p < PB; p++) F[r][p] = 0.0;
+    const int j1 = (int)min((long)kCorrT, n - j0);  // pixels of the stretch
+    auto load = [&](double (&v)[PB], int s) {
+      const bool in = s + lane < j1;
+      const double *G = GI + j0 + (in ? s + lane : j1 - 1);
 #pragma unroll
-  for (int f = 0; f < NF; f++) {
-    double v[4];
+      for (int p = 0; p < PB; p++) {
+        const double xv = G[(long)min(p0 + p, a.n_phase - 1) * n];
+        v[p] = in ? xv : 0.0;
+      }
+    };
+    const int s0 = w * (kCorrT / 4), s1 = min(j1, s0 + kCorrT / 4);
+    const double *x = s_x + (lane & 48) + 15 - l;
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int i = 4 * f + u;
-      v[u] = i < RB * PB ? F[i / PB][i % PB] : 0.0;
+    for (int r = 0; r < RB; r++) xc[r] = x[r * kCorrWin + s0];
+    if (s0 < s1) load(g, s0);
+    for (int s = s0; s < s1; s += 64) {
+      load(gn, s + 64);
+      lag_steps<0>(F, g, xc, x + s);
+#pragma unroll
+      for (int p = 0; p < PB; p++) g[p] = gn[p];
     }
-    s_x[((long)w * NF * 4 + 4 * f + which) * 16 + l] = swap_fold<16>(swap_fold<32>(v[0], v[1]), swap_fold<32>(v[2], v[3]));
+    __syncthreads();  // the staged rows become the waves' sums
+    const int which = (0x3120 >> (4 * (lane >> 4))) & 15;  // rows 0..3 of a folded register hold sums 0, 2, 1, 3
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int i = 4 * f + u;
+        v[u] = i < RB * PB ? F[i / PB][i % PB] : 0.0;
+      }
+      s_x[((long)w * NF * 4 + 4 * f + which) * 16 + l] =
+          swap_fold<16>(swap_fold<32>(v[0], v[1]), swap_fold<32>(v[2], v[3]));
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < RB * PB * 16; e += 256) {  // a thread's own sums: no wait in between
+      double t = s_x[e];
+#pragma unroll
+      for (int i = 1; i < 4; i++) t += s_x[i * NF * 64 + e];
+      s_run[e] = c ? s_run[e] + t : t;
+    }
   }
-  __syncthreads();
   for (int e = threadIdx.x; e < RB * PB * 16; e += 256) {
     const int r = e / (PB * 16), p = e / 16 % PB;
-    double t = s_x[e];
-#pragma unroll
-    for (int i = 1; i < 4; i++) t += s_x[i * NF * 64 + e];
     if (r0 + r < rows && p0 + p < a.n_phase)
-      Cpart[((((long)chunk * rows + r0 + r) * n_z + z) * a.n_phase + p0 + p) * 16 + (e & 15)] = t;
+      Cpart[((((long)chunk * rows + r0 + r) * n_z + z) * a.n_phase + p0 + p) * 16 + (e & 15)] = s_run[e];
   }
 }
 
 static int corr_pb(int n_phase) { return (n_phase + 9) / 10 * 10 <= (n_phase + 7) / 8 * 8 ? 10 : 8; }
-static int corr_chunks(int64_t n) { return (int)((n + kCorrT - 1) / kCorrT); }
+// stretches of kCorrT pixels to a block: a whole group where blocks for three to a CU are left
+static int corr_per(int64_t n, int n_phase, int rows, int nd) {
+  const int64_t groups = (n + (int64_t)kCorrG * kCorrT - 1) / (kCorrG * kCorrT);
+  const int pb = corr_pb(n_phase);
+  return groups * ((rows + kCorrRB - 1) / kCorrRB) * ((n_phase + pb - 1) / pb) * ((nd + 15) / 16) >= 768 ? kCorrG : 1;
+}
+static int corr_chunks(int64_t n, int per) { return (int)((n + (int64_t)per * kCorrT - 1) / (per * kCorrT)); }
 size_t diff_corr_part(int64_t n, int n_phase, int rows, int nd) {
-  return (size_t)corr_chunks(n) * rows * ((nd + 15) / 16) * n_phase * 16;
+  return (size_t)corr_chunks(n, corr_per(n, n_phase, rows, nd)) * rows * ((nd + 15) / 16) * n_phase * 16;
 }
 
 // one thread per (row, phase, lag of a tile of 16)
-__global__ void k_diff_corr_reduce(DiffArgs a, int nchunk, int n_z, const double *Cpart, double *C) {
+__global__ void k_diff_corr_reduce(DiffArgs a, int nchunk, int per, int n_z, const double *Cpart, double *C) {
   const int ns = a.ns, rows = a.n_mu * ns, P = a.n_phase;
-  const long per = (long)n_z * P * 16, e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= rows * per) return;
-  const int row = (int)(e / per), z = (int)(e % per / (P * 16)), p = (int)(e % (P * 16) / 16), l = (int)(e % 16);
+  const long tot = (long)n_z * P * 16, e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows * tot) return;
+  const int row = (int)(e / tot), z = (int)(e % tot / (P * 16)), p = (int)(e % (P * 16) / 16), l = (int)(e % 16);
   const int k = row / ns, r0 = row / kCorrRB * kCorrRB;
   int hi;
   const int d = corr_lag0(a, r0 / ns, min(rows - 1, r0 + kCorrRB - 1) / ns, hi) + 16 * z + l;
   if (d < a.blag[2 * k] || d > a.blag[2 * k + 1]) return;  // no cell of the bin uses it
   constexpr int kU = 16;
+  static_assert(kU % kCorrG == 0, "whole groups");
   const double *in = Cpart + e;
-  const long cs = rows * per;
+  const long cs = rows * tot;
+  const int g = kCorrG / per;  // partials of a group: 1 or kCorrG
   double x = 0.0;
-  int c = 0;
-  for (; c + kU <= nchunk; c += kU) {
+  for (int c = 0; c < nchunk; c += kU) {
     double t[kU];
 #pragma unroll
-    for (int u = 0; u < kU; u++) t[u] = in[(c + u) * cs];
+    for (int u = 0; u < kU; u++) t[u] = in[min(c + u, nchunk - 1) * cs];
 #pragma unroll
-    for (int u = 0; u < kU; u++) x += t[u];
+    for (int u = 0; u < kU; u += kCorrG) {
+      double s = t[u];
+#pragma unroll
+      for (int v = 1; v < kCorrG; v++) {
+        if (c + u + v >= nchunk) break;
+        if (g == 1) {
+          x += s;
+          s = t[u + v];
+        } else {
+          s += t[u + v];
+        }
+      }
+      if (c + u < nchunk) x += s;
+    }
   }
-  for (; c < nchunk; c++) x += in[c * cs];
   C[(((long)k * a.nd + d) * ns + row % ns) * P + p] = x;
 }
 
@@ -1110,7 +1150,7 @@ __global__ __launch_bounds__(256) void k_diff_piecegrad(DiffArgs a, const double
   for (int q = 0; q < 16; q++) v[q] = 0.0;
   if (ip < a.n_piece) {
     const CONSTANT int32_t *pc = gc((const int32_t *)(a.piece + ip));
-    const int iy = pc[0], len = pc[2], k = pc[3];
+    const int iy = pc[0], k = pc[1], len = pc[3];
     const double kappa = a.prm ? a.prm[3] : a.kappa, kappa_f = a.prm ? a.prm[4] : a.kappa_f;
     const double u1 = a.prm ? a.prm[1] : a.u1, u2 = a.prm ? a.prm[2] : a.u2;
     const double t = gc((const double *)(a.row_t + iy))[0], dt = gc((const double *)(a.row_t + iy))[1];
@@ -1407,15 +1447,16 @@ static hipError_t launch_seed_r(const DiffArgs &a, const double *GI, double *gq,
 
 template <int PB>
 static hipError_t launch_corr_p(const DiffArgs &a, const double *GI, double *Cpart, double *C, hipStream_t s) {
-  const int rows = a.n_mu * a.ns, n_tile = (a.n_phase + PB - 1) / PB, n_z = (a.nd + 15) / 16, nch = corr_chunks(a.n);
+  const int rows = a.n_mu * a.ns, n_tile = (a.n_phase + PB - 1) / PB, n_z = (a.nd + 15) / 16;
+  const int per = corr_per(a.n, a.n_phase, rows, a.nd), nch = corr_chunks(a.n, per);
   if ((long)n_tile * n_z > 65535) return hipErrorInvalidValue;
   dim3 gr(nch, (rows + kCorrRB - 1) / kCorrRB, n_tile * n_z);
-  const size_t lds = (size_t)std::max(kCorrRB * kCorrWin + 64, 4 * (kCorrRB * PB + 3) / 4 * 64) * sizeof(double);
-  k_diff_corr<PB><<<gr, 256, lds, s>>>(a, GI, Cpart, n_z);
+  const size_t lds = (size_t)(corr_lds(PB) + kCorrRB * PB * 16) * sizeof(double);
+  k_diff_corr<PB><<<gr, 256, lds, s>>>(a, GI, Cpart, n_z, per);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const long tot = (long)rows * n_z * a.n_phase * 16;
-  k_diff_corr_reduce<<<(unsigned)((tot + kDT - 1) / kDT), kDT, 0, s>>>(a, nch, n_z, Cpart, C);
+  k_diff_corr_reduce<<<(unsigned)((tot + kDT - 1) / kDT), kDT, 0, s>>>(a, nch, per, n_z, Cpart, C);
   return hipGetLastError();
 }
 

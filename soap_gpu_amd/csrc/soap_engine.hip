@@ -107,12 +107,14 @@ struct soap_ctx {
     int ns = 2;                   // tap sets of the last forward: 2, or 3 with the facula population
     const double *q = nullptr, *s = nullptr, *f = nullptr, *maps = nullptr, *fmaps = nullptr, *target = nullptr;
     // the disk's plan and what it was built for (diff_plan)
-    DevBuf ck, cell, map_j, map_f, piece, psum, pstart, brow;
+    DevBuf ck, cell, map_j, map_f, piece, col, psum, pstart, brow;
     int n_piece = 0, plan_G = 0, plan_M = 0;
     std::vector<double> plan_mu;
     double plan_lb[4] = {0, 0, 0, 0};
-    DevBuf row_m, row_t, drow, blag, mom, wts, taps_p, taps_r, I, F, res_part, ccf, par, model, depth, bis, iters, th,
-        dth, gy, GF, GI, C, Cpart, cell_part;
+    // S holds I in the forward and G_I in the backward; W the tap weights, then (in the backward) G_F,
+    // then the correlations' partials: none is read after the next one is written
+    DevBuf row_m, row_t, drow, blag, mom, taps_p, taps_r, S, F, W, res_part, ccf, par, model, depth, bis, iters, th, dth,
+        gy, C, cell_part;
     DevBuf bisd;  // [P][n_v + kBisHead]: span, loss coefficient, dspan/dtheta, dspan/dy
     DevBuf tg;    // per-call targets [3][P] (RV, FWHM, BIS span), the loss [1], the scalar gradients [5], the series [3][P]
     DevBuf mt_ptr, mt_w, mt_col, mt_val;  // the mask in sliced pixel-major form (adjoint of the CCF)
@@ -2209,7 +2211,7 @@ int soap_fit_ccf_host_noalloc(soap_ctx *c, const double *v, int32_t n_v, const d
 }
 
 // The disk's plan: per-cell tables, the map stencil of every grid row or column, and the
-// pieces (runs of cells of one bin along a row) sorted by bin and row.  It depends on the
+// pieces (cells of one bin and row) sorted by bin and row.  It depends on the
 // grid, the bins, the map size and LB only; built by diff_setup, and again by the next
 // forward, bind or step when the bins were set anew.
 static bool diff_plan_current(const soap_ctx *c) {
@@ -2245,47 +2247,67 @@ static int diff_plan(soap_ctx *c) {
     map_j[i] = j;
     map_f[i] = g - j;
   }
-  std::vector<std::vector<DiffPiece>> by(n_mu);
+  std::vector<int32_t> in_bin(n_mu, 0);
+  int64_t groups = 0;
   for (int iy = 0; iy < G; iy++) {
-    for (int k = 0; k < n_mu; k++) pstart[(size_t)k * (G + 1) + iy] = (int32_t)by[k].size();
-    const int32_t *row = ck.data() + (size_t)iy * G;
-    for (int iz = 0; iz < G;) {
-      const int k = row[iz];
-      int e = iz + 1;
-      while (e < G && row[e] == k && (k < 0 || e - iz < kDiffPiece)) e++;
-      if (k >= 0) by[k].push_back({iy, iz, e - iz, k});
-      iz = e;
+    for (int iz = 0; iz < G; iz++)
+      if (const int k = ck[(size_t)iy * G + iz]; k >= 0 && in_bin[k]++ % kDiffGroup == 0) groups++;
+    std::fill(in_bin.begin(), in_bin.end(), 0);
+  }
+  const int most = (groups > kDiffMany ? 2 : 1) * kDiffGroup;  // cells of a piece
+  std::vector<std::vector<DiffPiece>> by(n_mu);  // group: among the bin's groups, shifted below
+  std::vector<std::vector<int32_t>> col_of(n_mu);
+  std::vector<std::vector<int32_t>> of_row(n_mu);  // the row's cells by bin
+  for (int iy = 0; iy < G; iy++) {
+    for (int iz = 0; iz < G; iz++)
+      if (const int k = ck[(size_t)iy * G + iz]; k >= 0) of_row[k].push_back(iz);
+    for (int k = 0; k < n_mu; k++) {
+      pstart[(size_t)k * (G + 1) + iy] = (int32_t)by[k].size();
+      const int n = (int)of_row[k].size();
+      for (int at = 0; at < n; at += most)
+        by[k].push_back({iy, k, (int32_t)(col_of[k].size() / kDiffGroup) + at / kDiffGroup, std::min(n - at, most)});
+      while (of_row[k].size() % kDiffGroup) of_row[k].push_back(of_row[k].back());
+      col_of[k].insert(col_of[k].end(), of_row[k].begin(), of_row[k].end());
+      of_row[k].clear();
     }
   }
   std::vector<DiffPiece> pieces;
-  std::vector<int32_t> brow;
+  std::vector<int32_t> col, brow;
   for (int k = 0; k < n_mu; k++) {
     brow.push_back(by[k].empty() ? 1 : by[k].front().iy);
     brow.push_back(by[k].empty() ? 0 : by[k].back().iy);
-    const int32_t base = (int32_t)pieces.size();
+    const int32_t base = (int32_t)pieces.size(), first = (int32_t)(col.size() / kDiffGroup);
     for (int iy = 0; iy < G; iy++) pstart[(size_t)k * (G + 1) + iy] += base;
-    pieces.insert(pieces.end(), by[k].begin(), by[k].end());
+    for (DiffPiece p : by[k]) {
+      p.group += first;
+      pieces.push_back(p);
+    }
+    col.insert(col.end(), col_of[k].begin(), col_of[k].end());
     pstart[(size_t)k * (G + 1) + G] = (int32_t)pieces.size();
   }
   if (pieces.empty()) return fail(c, SOAP_ERR_ARG, "diff: no cell of a %d grid on the disk", G);
-  if ((rc = ensure(c, d.piece, pieces.size() * sizeof(DiffPiece))) || (rc = ensure(c, d.psum, pieces.size() * 16)) ||
-      (rc = ensure(c, d.cell_part, (size_t)diff_piece_blocks((int)pieces.size()) * kDiffScalars * 8)))
+  const size_t n_piece = pieces.size();
+  if ((rc = ensure(c, d.piece, n_piece * sizeof(DiffPiece))) || (rc = ensure(c, d.col, col.size() * 4)) ||
+      (rc = ensure(c, d.psum, n_piece * 16)) ||
+      (rc = ensure(c, d.cell_part, (size_t)diff_piece_blocks((int)n_piece) * kDiffScalars * 8)))
     return rc;
-  HIPCHK(c, hipMemcpyAsync(d.piece.p, pieces.data(), pieces.size() * sizeof(DiffPiece), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(d.piece.p, pieces.data(), n_piece * sizeof(DiffPiece), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(d.col.p, col.data(), col.size() * 4, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(d.pstart.p, pstart.data(), pstart.size() * 4, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(d.brow.p, brow.data(), brow.size() * 4, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(d.map_j.p, map_j.data(), (size_t)G * 4, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(d.map_f.p, map_f.data(), (size_t)G * 8, hipMemcpyHostToDevice, c->stream));
   a.cell = (const double2 *)d.cell.p;
   a.piece = (const DiffPiece *)d.piece.p;
-  a.n_piece = (int)pieces.size();
+  a.col = (const int32_t *)d.col.p;
+  a.n_piece = (int)n_piece;
   HIPCHK(c, launch_diff_psum(a, (double2 *)d.psum.p, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   d.plan_G = G;
   d.plan_M = M;
   d.plan_mu = c->mu_bounds;
   for (int q = 0; q < 4; q++) d.plan_lb[q] = d.lb[q];
-  d.n_piece = (int)pieces.size();
+  d.n_piece = (int)n_piece;
   return SOAP_OK;
 }
 
@@ -2297,10 +2319,11 @@ static int diff_buffers(soap_ctx *c, int nd, int ns) {
   if ((rc = ensure(c, c->ccf_part, (size_t)ccf_chunks(c->n_lines) * d.P * c->n_v * 8)) ||
       (rc = ensure(c, d.drow, (size_t)nd * 2 * 4)) || (rc = ensure(c, d.blag, (size_t)c->n_mu * 2 * 4)) ||
       (rc = ensure(c, d.mom, (size_t)d.n_piece * diff_moments(ns) * d.P * 8)) ||
-      (rc = ensure(c, d.wts, (size_t)d.n_piece * ns * d.P * 8)) ||
+      (rc = ensure(c, d.W, std::max({(size_t)d.n_piece * ns * d.P, (size_t)d.P * c->n,
+                                     diff_corr_part(c->n, d.P, c->n_mu * ns, nd)}) * 8)) ||
       (rc = ensure(c, d.taps_p, (size_t)diff_groups(d.P) * c->n_mu * nd * ns * 16 * 8)) ||
       (rc = ensure(c, d.taps_r, (size_t)d.P * diff_groups(c->n_mu * ns) * nd * 16 * 8)) ||
-      (rc = ensure(c, d.C, per * 8)) || (rc = ensure(c, d.Cpart, diff_corr_part(c->n, d.P, c->n_mu * ns, nd) * 8)))
+      (rc = ensure(c, d.C, per * 8)))
     return rc;
   return SOAP_OK;
 }
@@ -2317,8 +2340,8 @@ int soap_diff_setup(soap_ctx *c, int32_t grid, int32_t n_phase, int32_t map_res,
   HIPCHK(c, hipSetDevice(c->device));
   auto &d = c->diff;
   int rc;
-  if ((rc = ensure(c, d.I, (size_t)n_phase * c->n * 8)) || (rc = ensure(c, d.F, (size_t)n_phase * c->n * 8)) ||
-      (rc = ensure(c, d.GF, (size_t)n_phase * c->n * 8)) || (rc = ensure(c, d.GI, (size_t)n_phase * c->n * 8)) ||
+  if ((rc = ensure(c, d.S, (size_t)n_phase * c->n * 8)) || (rc = ensure(c, d.F, (size_t)n_phase * c->n * 8)) ||
+      (rc = ensure(c, d.W, (size_t)n_phase * c->n * 8)) ||
       (rc = ensure(c, d.res_part, (size_t)n_phase * diff_conv_blocks(c->n) * 8)) ||
       (rc = ensure(c, d.ccf, (size_t)n_phase * c->n_v * 8)) || (rc = ensure(c, d.par, (size_t)n_phase * 5 * 8)) ||
       (rc = ensure(c, d.model, (size_t)n_phase * c->n_v * 8)) || (rc = ensure(c, d.depth, (size_t)n_phase * 91 * 8)) ||
@@ -2377,6 +2400,7 @@ static DiffArgs diff_args(soap_ctx *c) {
   a.map_j = (const int32_t *)d.map_j.p;
   a.map_f = (const double *)d.map_f.p;
   a.piece = (const DiffPiece *)d.piece.p;
+  a.col = (const int32_t *)d.col.p;
   a.psum = (const double2 *)d.psum.p;
   a.pstart = (const int32_t *)d.pstart.p;
   a.brow = (const int32_t *)d.brow.p;
@@ -2386,7 +2410,7 @@ static DiffArgs diff_args(soap_ctx *c) {
   a.drow = (int32_t *)d.drow.p;
   a.blag = (int32_t *)d.blag.p;
   a.mom = (double *)d.mom.p;
-  a.wts = (double *)d.wts.p;
+  a.wts = (double *)d.W.p;
   a.maps = d.maps;
   a.fmaps = d.fmaps;
   a.grp_p = diff_group(d.P);
@@ -2396,7 +2420,7 @@ static DiffArgs diff_args(soap_ctx *c) {
   a.q = d.q;
   a.s = d.s;
   a.f = d.f;
-  a.I = (double *)d.I.p;
+  a.I = (double *)d.S.p;
   a.F = (double *)d.F.p;
   return a;
 }
@@ -2530,8 +2554,8 @@ int soap_diff_backward(soap_ctx *c, double *grad5, double *d_gq, double *d_gs, d
     hipError_t e = launch_diff_backward(
         a, ca, d.target, c->trim, d.w_spec, c->d_vgrid, c->n_v, (const double *)d.ccf.p, (const double *)d.th.p,
         (const double *)d.dth.p, (double *)d.gy.p, c->n - 2 * (int64_t)c->trim, (const int64_t *)d.mt_ptr.p,
-        (const int32_t *)d.mt_w.p, (const int32_t *)d.mt_col.p, (const double *)d.mt_val.p, (double *)d.GF.p,
-        (double *)d.GI.p, (double *)d.Cpart.p, (double *)d.C.p, d_gmaps, d.ns == 3 ? d_gfmaps : nullptr,
+        (const int32_t *)d.mt_w.p, (const int32_t *)d.mt_col.p, (const double *)d.mt_val.p, (double *)d.W.p,
+        (double *)d.S.p, (double *)d.W.p, (double *)d.C.p, d_gmaps, d.ns == 3 ? d_gfmaps : nullptr,
         (double *)d.cell_part.p, d_gq, d_gs, d.ns == 3 ? d_gf : nullptr, (const double *)d.bisd.p, c->stream);
     if (e == hipErrorInvalidValue) return fail(c, SOAP_ERR_LIMIT, "diff_backward: window or shift range too wide");
     HIPCHK(c, e);
@@ -3164,10 +3188,10 @@ namespace {
 std::vector<uintptr_t> dbatch_signature(const soap_ctx *c) {
   auto &d = c->diff;
   auto u = [](const void *p) { return (uintptr_t)p; };
-  return {u(d.mom.p),  u(d.wts.p),   u(d.drow.p),   u(d.blag.p),  u(d.row_m.p),  u(d.row_t.p),    u(d.taps_p.p), u(d.taps_r.p), u(d.C.p),     u(d.Cpart.p),  u(d.res_part.p), u(d.ccf.p),
+  return {u(d.mom.p),  u(d.drow.p),   u(d.blag.p),  u(d.row_m.p),  u(d.row_t.p),    u(d.taps_p.p), u(d.taps_r.p), u(d.C.p),     u(d.res_part.p), u(d.ccf.p),
           u(d.par.p),  u(d.model.p), u(d.depth.p),  u(d.bis.p),   u(d.iters.p),  u(d.th.p),       u(d.dth.p),
-          u(d.gy.p),   u(d.GF.p),    u(d.GI.p),     u(d.cell_part.p), u(d.I.p),  u(d.F.p),        u(d.ck.p),
-          u(d.cell.p), u(d.map_j.p), u(d.map_f.p),  u(d.piece.p), u(d.psum.p), u(d.brow.p), u(d.pstart.p), (uintptr_t)d.n_piece, u(d.mt_ptr.p), u(d.mt_w.p),
+          u(d.gy.p),   u(d.W.p),     u(d.cell_part.p), u(d.S.p),  u(d.F.p),        u(d.ck.p),
+          u(d.cell.p), u(d.map_j.p), u(d.map_f.p),  u(d.piece.p), u(d.col.p), u(d.psum.p), u(d.brow.p), u(d.pstart.p), (uintptr_t)d.n_piece, u(d.mt_ptr.p), u(d.mt_w.p),
           u(d.mt_col.p), u(d.mt_val.p), u(c->ccf_part.p), u(c->m_start.p), u(c->m_alive.p), u(c->m_val.p),
           u(c->d_w_sorted), u(c->ctap.p), u(d.bisd.p), u(d.maps), u(d.q), u(d.s), u(d.target), u(d.f), u(d.fmaps),
           (uintptr_t)d.ns, (uintptr_t)d.nd,
@@ -3288,7 +3312,7 @@ hipError_t dbatch_enqueue_one(soap_diffbatch::Item &it, hipStream_t st, bool adj
       e = launch_diff_backward(a, ca, it.target, c->trim, it.w_spec, c->d_vgrid, c->n_v, (const double *)d.ccf.p,
                                (const double *)d.th.p, (const double *)d.dth.p, (double *)d.gy.p,
                                c->n - 2 * (int64_t)c->trim, (const int64_t *)d.mt_ptr.p, (const int32_t *)d.mt_w.p, (const int32_t *)d.mt_col.p,
-                               (const double *)d.mt_val.p, (double *)d.GF.p, (double *)d.GI.p, (double *)d.Cpart.p,
+                               (const double *)d.mt_val.p, (double *)d.W.p, (double *)d.S.p, (double *)d.W.p,
                                (double *)d.C.p, it.gmaps, it.gfmaps, (double *)d.cell_part.p, it.gq, it.gs, it.gf,
                                bisd, st);
     if (e == hipSuccess) e = launch_diff_grad(diff_piece_blocks(d.n_piece), (const double *)d.cell_part.p,

@@ -290,13 +290,17 @@ struct LinSolar {
 };
 
 // Differentiable path (soap_diff.hip)
-// A run of at most kDiffPiece neighbouring cells (along a disk row) of one mu bin.
-// Rigid rotation gives a row one shift, so everything a cell needs beside its own limb
-// and filling factors is shared by the run.
+// A piece: one group, or up to two, of 32 cells of one disk row and mu bin, in order.  Rigid
+// rotation gives a row one shift, so everything a cell needs beside its own limb and filling
+// factors is shared by the piece.  Sums are held per piece and phase, so memory goes with the
+// pieces (grid 1000, 20 bins: 32,800 of one group, 21,800 of up to two, 17,500 of up to four);
+// a wave takes a piece, so few large ones leave CUs idle at the end (grid 600, 10 bins, 50
+// phases: forward 545, 551 and 576 us with one, two and four; grid 300, 64 phases: 356, 375
+// and 396).  So two groups where there are more than kDiffMany, one otherwise.
 struct DiffPiece {
-  int32_t iy, iz0, len, k;
+  int32_t iy, k, group, len;  // group: its first group; len: cells
 };
-constexpr int kDiffPiece = 32;
+constexpr int kDiffGroup = 32, kDiffMany = 8192;
 constexpr int diff_moments(int ns) { return ns == 3 ? 9 : 3; }
 // Rows of a contraction's group: of the sizes that the kernels have, the one that pads
 // `rows` least, the larger of equals.
@@ -327,6 +331,7 @@ struct DiffArgs {
   const int32_t *map_j;          // per grid row or column: first map node of its bilinear stencil
   const double *map_f;           // and the weight of the second
   const DiffPiece *piece;        // [n_piece], by bin, then row
+  const int32_t *col;            // [groups][kDiffGroup]: the cells' columns, the last one repeated to the end
   const double2 *psum;           // [n_piece]: sums over the piece of a and a^2, a = 1 - mu
   const int32_t *pstart;         // [n_mu][G + 1]: first piece of a bin at or after a row
   const int32_t *brow;           // [n_mu][2]: first and last row that holds cells of a bin (first > last: none)
