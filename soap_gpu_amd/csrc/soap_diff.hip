@@ -1400,6 +1400,9 @@ __global__ __launch_bounds__(kDT) void k_diff_seedgrad(DiffArgs a, const double 
 }
 
 // ------------------------------------------------------------ launchers
+// The widest shift range that the adjoint accepts (forwards take 2048 offsets).  No kernel here needs it: at this bound the seed gradients hold 57 KB of LDS.
+constexpr int kAdjointLags = 761;
+
 // Two pixels per thread serve a coefficient read twice, where that still leaves two
 // blocks per CU; one otherwise.
 static bool two_pixels(int64_t n, int groups) { return (n + 2 * kDT - 1) / (2 * kDT) * groups >= 512; }
@@ -1409,7 +1412,7 @@ static hipError_t launch_fir_r(const DiffArgs &a, hipStream_t s) {
   const int groups = (a.n_phase + R - 1) / R;
   const bool two = two_pixels(a.n, groups);
   const int px = two ? 2 * kDT : kDT;
-  const size_t lds = (size_t)(NS * (px + a.nd - 1) + kFirD * NS * 16) * sizeof(double);  // at most 86 KB
+  const size_t lds = (size_t)(NS * (px + a.nd - 1) + kFirD * NS * 16) * sizeof(double);  // at most 74 KB (2048 offsets)
   dim3 gr((unsigned)((a.n + px - 1) / px), groups);
   if (two)
     k_diff_fir<NS, R, 2><<<gr, kDT, lds, s>>>(a);
@@ -1436,7 +1439,7 @@ static hipError_t launch_seed_r(const DiffArgs &a, const double *GI, double *gq,
   const int groups = (a.n_mu * a.ns + R - 1) / R;
   const bool two = two_pixels(a.n, groups);
   const int px = two ? 2 * kDT : kDT;
-  const size_t lds = (size_t)kSeedP * (px + a.nd - 1 + kSeedD * 16) * sizeof(double);  // at most 98 KB
+  const size_t lds = (size_t)kSeedP * (px + a.nd - 1 + kSeedD * 16) * sizeof(double);  // at most 57 KB (kAdjointLags)
   dim3 gr((unsigned)((a.n + px - 1) / px), groups);
   if (two)
     k_diff_seedgrad<R, 2><<<gr, kDT, lds, s>>>(a, GI, gq, gs, gf);
@@ -1482,7 +1485,6 @@ hipError_t launch_diff_forward_spectra(const DiffArgs &a, const ConvArgs &c, con
     k_diff_taps<2><<<gt, 64 * kTapW, 0, s>>>(a);
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((size_t)a.ns * (kDT + a.nd - 1) * sizeof(double) > 65536) return hipErrorInvalidValue;
   e = a.ns == 3 ? launch_fir_ns<3>(a, s) : launch_fir_ns<2>(a, s);
   if (e != hipSuccess) return e;
   size_t lds_conv = (size_t)(4 * kDT + 2 * c.ntp) * sizeof(double);
@@ -1499,9 +1501,9 @@ int diff_conv_blocks(int64_t n) { return (int)((n + 4 * kDT - 1) / (4 * kDT)); }
 // loss = sum_p [w_spec r2_p + w_rv (RV_p - rv_t)^2 + w_fw (FWHM_p - fw_t)^2], r2_p the
 // residual partials of phase p summed in order; the same order as the host sum
 // With device parameters (graph replays) the loss is NaN when vsini leaves the
-// bound tap range or when the cell weights could exceed the fixed-point tap
-// capacity: n_cells max|L| max(3, |kappa|, |kappa_f| lbmax) >= 2^30, lbmax =
-// max |1 + LB(mu)| (maps are filling factors in [0, 1]).
+// bound tap range or when the cell weights leave the accepted range, which is that of
+// the series' fixed-point taps: n_cells max|L| max(3, |kappa|, |kappa_f| lbmax) >= 2^30,
+// lbmax = max |1 + LB(mu)| (maps are filling factors in [0, 1]).
 __global__ __launch_bounds__(kDT) void k_diff_loss(int n_phase, int res_blocks, const double *res_part,
                                                    const double *theta, const double *rv_t, const double *fw_t,
                                                    const double *bis_t, double w_spec, double w_rv, double w_fw,
@@ -1648,7 +1650,7 @@ hipError_t launch_diff_backward(const DiffArgs &a, const ConvArgs &c, const doub
   dim3 gc((unsigned)((a.n + 4 * kDT - 1) / (4 * kDT)), a.n_phase);
   k_diff_convT<<<gc, kDT, lds_conv, s>>>(a, c, GF, GI);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if (a.nd > 761) return hipErrorInvalidValue;  // the widest shift range the adjoint takes
+  if (a.nd > kAdjointLags) return hipErrorInvalidValue;
   e = corr_pb(a.n_phase) == 10 ? launch_corr_p<10>(a, GI, Cpart, C, s) : launch_corr_p<8>(a, GI, Cpart, C, s);
   if (e != hipSuccess) return e;
   k_diff_piecegrad<<<diff_piece_blocks(a.n_piece), 256, 0, s>>>(a, C, cell_part);

@@ -2453,8 +2453,8 @@ int soap_diff_forward(soap_ctx *c, const soap_diff_params *prm, const double *d_
     double w = lmax * std::max(3.0, std::max(std::fabs(prm->contrast),
                                              d_f ? std::fabs(prm->contrast_fac) * lb_factor_bound(d.lb) : 0.0));
     if (!fx_capacity_ok((double)d.G * d.G, w))
-      return fail(c, SOAP_ERR_LIMIT, "diff_forward: %d^2 cells with weights up to %g exceed the fixed-point tap "
-                  "capacity (cells x weight < 2^30)", d.G, w);
+      return fail(c, SOAP_ERR_LIMIT, "diff_forward: %d^2 cells with weights up to %g exceed the accepted range of "
+                  "tap sums (cells x weight < 2^30)", d.G, w);
   }
   HIPCHK(c, hipSetDevice(c->device));
   // taps span the shifts of delta in [-vsini, vsini] (m monotone in delta), plus margins

@@ -584,8 +584,7 @@ constexpr int kBisHead = 6;
 constexpr int kMaxVDiff = 1024;
 hipError_t launch_diff_bis(const double *v, int n_v, const double *ccf, const double *theta, int n_ccf, double *bisd,
                            hipStream_t s);
-// chunks of the lag-correlation pass (Cpart holds [P][n_mu][chunks][nd][ns])
-// doubles of the correlations' chunk partials
+// doubles of the correlations' partials, Cpart [chunk][row][lag tile][P][16]
 size_t diff_corr_part(int64_t n, int n_phase, int rows, int nd);
 hipError_t launch_ccf_sum(const double *part, int nc, int n_spec, int n_v, double *ccf, hipStream_t s);
 // device-side loss of the differentiable model: per phase the residual partials
@@ -593,7 +592,7 @@ hipError_t launch_ccf_sum(const double *part, int nc, int n_spec, int n_v, doubl
 // bisector-span term from bisd; writes loss[0], the fit-parameter derivatives
 // dth [P][4] and the span coefficients of bisd; loss = NaN when prm (optional) has
 // vsini outside (0, vsini_max] (the fixed tap range of a graph) or weights beyond
-// the fixed-point tap capacity of n_cells cells (lbmax = max |1 + LB(mu)|)
+// the accepted range for n_cells cells (lbmax = max |1 + LB(mu)|)
 hipError_t launch_diff_loss(int n_phase, int res_blocks, const double *res_part, const double *theta,
                             const double *rv_t, const double *fw_t, const double *bis_t, double w_spec, double w_rv,
                             double w_fw, double w_bis, double *bisd, int n_v, const double *prm, double vsini_max,
