@@ -308,7 +308,11 @@ int soap_set_fir_shape(soap_ctx *ctx, int32_t phases_per_block, int32_t pixels_p
  * G^2 max|L| max(3, |contrast|, |contrast_fac| max|1 + LB|) must stay below 2^30
  * (SOAP_ERR_LIMIT from soap_diff_forward, a NaN loss in graph replays).
  * Array arguments named d_* are device (HIP) pointers: seeds [n_mu][n], maps
- * [P][M][M], target [P][n]; they must stay valid until soap_diff_backward. */
+ * [P][M][M], target [P][n]; they must stay valid until soap_diff_backward.
+ * The tap offsets are 2 vsini over the grid's velocity step and a few more: the
+ * forward takes at most 2048 (SOAP_ERR_LIMIT), soap_diff_backward 761 (SOAP_ERR_HIP).
+ * soap_diff_backward refuses a forward that ran with other sizes of the grid, bins or
+ * mask than the context now has (SOAP_ERR_STATE). */
 typedef struct soap_diff_params {
   double vsini_kms, u1, u2, contrast, contrast_fac;
 } soap_diff_params;

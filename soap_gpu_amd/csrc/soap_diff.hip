@@ -286,14 +286,15 @@ __global__ __launch_bounds__(64 * kTapW) void k_diff_taps(DiffArgs a) {
 
 // ------------------------------------------------------------ contractions
 // The forward FIR, the seed gradients and the lag correlations are dense products in
-// FP64.  The matrix unit's 16x16x4 form sustains 32-47 TFLOP/s here and would pad 50
-// phases to 64, the vector unit 62-66, so they run as outer products on the vector unit:
-// R accumulators per lane and pixel, the R coefficients of a step in one register (lane
+// FP64.  Probes that do nothing else sustain 32-47 TFLOP/s with the matrix unit's 16x16x4
+// form, which would also pad 50 phases to 64, and 62-66 with the vector unit, so they run
+// as outer products on the vector unit: R accumulators per lane and pixel, the R coefficients of a step in one register (lane
 // r of each row of 16 lanes holds coefficient r) and broadcast by the multiply-add itself
 // (DPP row_newbcast), so that a step costs one coefficient read and one pixel read for R
-// multiply-adds.  One coefficient per LDS word and multiply-add before: 311 (FIR), 311
-// (seed gradients) and 324 us (correlations, 492 before their lags were cut to the
-// bins') on the full adjoint, 15 TFLOP/s.
+// multiply-adds.  On the full adjoint (grid 600, 100,000 pixels, 50 phases), 4.0 GFLOP
+// each: FIR 104 us (39 TFLOP/s), seed gradients 144 (28), correlations 147 (27), the rest
+// of the time being staging and waves too few to hide it; 311, 311 and 324 us with one
+// coefficient per LDS word and multiply-add.
 #define SOAP_FMB(I) "v_fmac_f64_dpp %" #I ", %[t], %[x] row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\t"
 #define SOAP_FMB4 SOAP_FMB(0) SOAP_FMB(1) SOAP_FMB(2) SOAP_FMB(3)
 #define SOAP_FMB8 SOAP_FMB4 SOAP_FMB(4) SOAP_FMB(5) SOAP_FMB(6) SOAP_FMB(7)

@@ -1082,8 +1082,9 @@ __global__ __launch_bounds__(kLTPB) void k_gather_active_linear(LinArgs a, FirAr
 // the shifted wavelengths' rounding that the reference's weights carry.  Every wave finds its
 // groups' whole parts with one group per lane; a group whose whole part changes inside the tile,
 // comes within 1e-5 of changing, or that has no shift, is interpolated by itself.
-// 25 phases of the production disk, 100,000 pixels: 1315 -> 529 us (a group at a time, with the
-// reciprocal weights: 1004); two groups' scalar loads at a time, 1 and 4 measured 6 % slower.
+// 25 phases of the production disk, 100,000 pixels: 1315 -> 529 us with one set of regions (a
+// group at a time, with the reciprocal weights: 1004), 2670-2900 -> 1040-1120 us with bench.py's,
+// which hold more groups; two groups' scalar loads at a time, 1 and 4 measured 6 % slower.
 __global__ __launch_bounds__(kLTPB) void k_gather_active_runs(LinArgs a, FirArgs f, const LinGroup *groups,
                                                               const int64_t *list_off, const int32_t *bin_off,
                                                               const int32_t *g_n, int n_phase, int n_tiles) {

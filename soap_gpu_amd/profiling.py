@@ -74,7 +74,8 @@ def _short(name):
               "k_mask_build", "k_mask_overwrite", "k_mask_wsum", "k_mask_footprint", "k_disk_init",
               "k_taps_finalize", "k_fill_u64",
               "k_gather_active_runs", "k_gather_active_linear", "k_fir_quiet_cols", "k_gather_quiet_cols", "k_gather_quiet_linear", "k_quiet_columns_maps",
-              "k_quiet_columns_pack", "k_lin_groups", "k_cells_count", "k_cells_write", "k_conv_linear"):
+              "k_quiet_columns_pack", "k_lin_groups", "k_cells_count", "k_cells_write", "k_conv_linear",
+              "k_diff_fir", "k_diff_seedgrad", "k_diff_corr", "k_diff_moments", "k_diff_mapgrad"):
         if (name.endswith(k) or re.search(r"soap::" + k + r"[(<]", name)
                 or ("4soap" + str(len(k)) + k + "E") in name or ("4soap" + str(len(k)) + k + "I") in name):
             return k
@@ -126,7 +127,7 @@ def sq_summary(out_md, title, passes, kernels):
             data.setdefault(k, {})[c] = sum(v) / len(v)
     names = kernels or sorted(data)
     counters = sorted({c for k in names for c in data.get(k, {})})
-    lines = [f"# rocprofv3 SQ counters per dispatch: {title}", "", "Commands (repository root on the MI355X box), one pass each:", ""]
+    lines = [f"# rocprofv3 SQ counters per dispatch: {title}", "", "Commands (repository root on the MI355X), one pass each:", ""]
     lines += [f"    {cmd}" for cmd, _ in passes]
     lines += ["", "| counter | " + " | ".join(f"`{k}`" for k in names) + " |",
               "|---|" + "---:|" * len(names)]
@@ -158,7 +159,7 @@ def stats(out_md, title, command, db, top=25, match=None):
     if match:
         rows = [r for r in rows if re.search(match, r[0])]
     total = sum(r[5] for r in rows) or 1.0
-    lines = [f"# rocprofv3 kernel statistics: {title}", "", "Command (repository root on the MI355X box):", "",
+    lines = [f"# rocprofv3 kernel statistics: {title}", "", "Command (repository root on the MI355X):", "",
              f"    {command}", "",
              "| kernel | calls | average us | min us | max us | total % |", "|---|---:|---:|---:|---:|---:|"]
     for name, n, avg, mn, mx, tot in rows[:top]:
